@@ -319,6 +319,7 @@ struct fkpm_handle {
   int nbD = 0, nnzbD = 0;
   bool d_set = false, d_sym = false, d_fused = false, d_valid = false;
   DevBuf drp, dci, tpos, dacc, dout;
+  DevBuf dout_f;  // D rounded to float for single-precision engines
   std::vector<int> hd_rp, hd_ci;
 
   // --- two-current moments (moments2) ---
@@ -341,7 +342,7 @@ struct fkpm_handle {
     DevBuf* bufs[] = {&rp,    &ci,    &hv,      &rowblk, &hraw, &rraw,  &rcol,     &rval,
                       &rflag, &R,     &A[0],    &A[1],   &A[2], &Bv[0], &Bv[1],    &Bv[2],
                       &xi,    &partial, &psum,  &tune_dacc, &drp, &dci,  &tpos,     &dacc,
-                      &dout,  &atab,  &tabc};
+                      &dout,  &dout_f, &atab,  &tabc, &rdesc};
     for (DevBuf* d : bufs) d->release();
     DevBuf* m2bufs[] = {&j_rp[0], &j_ci[0], &j_rb[0], &j_raw[0], &j_val[0], &j_rp[1], &j_ci[1],
                         &j_rb[1], &j_raw[1], &j_val[1], &m2_a, &m2_b, &m2_ring, &m2_c, &m2_part};
@@ -1064,21 +1065,21 @@ int moments_t(fkpm_handle* h, int M, double* mu) {
   return 0;
 }
 
-// D to the host in the engine type.
+// D to the host in the engine type.  Single-precision engines round on the
+// device (k_round_D), so half the bytes cross PCIe and no host pass follows.
 int copy_D_out(fkpm_handle* h, void* D_val) {
   const size_t cnt = (size_t)h->nnzbD * h->b * h->b * (h->cx ? 2 : 1);
-  if (!dtype_single(h->dtype)) {
-    HIPCHK(hipMemcpyAsync(D_val, h->dout.p, cnt * sizeof(double), hipMemcpyDeviceToHost,
-                          h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
-  } else {
-    std::vector<double> tmp(cnt);
-    HIPCHK(hipMemcpyAsync(tmp.data(), h->dout.p, cnt * sizeof(double), hipMemcpyDeviceToHost,
-                          h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
-    float* o = static_cast<float*>(D_val);
-    for (size_t k = 0; k < cnt; k++) o[k] = (float)tmp[k];
+  const void* src = h->dout.p;
+  size_t bytes = cnt * sizeof(double);
+  if (dtype_single(h->dtype)) {
+    bytes = cnt * sizeof(float);
+    CHK(h->dout_f.ensure(bytes > 0 ? bytes : 16));
+    CHK(launch(&fkd::k_round_D, dim3(grid_for(cnt)), dim3(256), h->stream,
+               (const double*)h->dout.as<double>(), h->dout_f.as<float>(), cnt));
+    src = h->dout_f.p;
   }
+  HIPCHK(hipMemcpyAsync(D_val, src, bytes, hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(hipStreamSynchronize(h->stream));
   return 0;
 }
 

@@ -1405,6 +1405,16 @@ __global__ __launch_bounds__(WG) void k_copy16_nt(const double2* __restrict__ a,
   }
 }
 
+// n doubles rounded to float (D in the type of a single-precision engine);
+// 12 bytes per value, HBM-bound: about 70 us for the 29 M values of 32^3 sites
+// of 8x8 blocks, where the host loop over twice the copied bytes took 18 ms of
+// a 103 ms step (85 ms now).
+__global__ void k_round_D(const double* __restrict__ src, float* __restrict__ dst, size_t n) {
+  for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < n;
+       k += (size_t)gridDim.x * blockDim.x)
+    dst[k] = (float)src[k];
+}
+
 // Fill n doubles with zero (graph-capturable, unlike hipMemsetAsync).
 __global__ void k_zero(double* __restrict__ p, size_t n) {
   for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < n;
