@@ -28,6 +28,8 @@
 #define FKD_DEFINE_HELPERS
 #include "kpm_kernels.h"
 #include "kpm_dots.h"
+#define FKD_RES_SHARED
+#include "kpm_resident.h"
 
 namespace {
 
@@ -102,6 +104,21 @@ int launch(void (*fp)(P...), dim3 grid, dim3 block, hipStream_t st,
     return 0;
   }
   hipError_t e = hipLaunchKernel((const void*)fp, grid, block, argv, 0, st);
+  if (e != hipSuccess) return fail(FKPM_E_HIP, "kernel launch failed: %s", hipGetErrorString(e));
+  return 0;
+}
+
+// The same with dynamic LDS (never recorded: these kernels run whole loops).
+template <typename... P>
+int launch_lds(void (*fp)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t st,
+               typename TypeId<P>::type... args) {
+  if (lds > 65536) {
+    const hipError_t e = hipFuncSetAttribute((const void*)fp,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return fail(FKPM_E_HIP, "%zu bytes of LDS: %s", lds, hipGetErrorString(e));
+  }
+  void* argv[] = {(void*)&args...};
+  const hipError_t e = hipLaunchKernel((const void*)fp, grid, block, argv, lds, st);
   if (e != hipSuccess) return fail(FKPM_E_HIP, "kernel launch failed: %s", hipGetErrorString(e));
   return 0;
 }
@@ -190,6 +207,29 @@ struct DevBuf {
   template <class T>
   T* as() const {
     return static_cast<T*>(p);
+  }
+};
+
+// Pinned host memory the kernels read and write directly (small operands and
+// results of a call); grows only.
+struct PinBuf {
+  void* p = nullptr;
+  size_t bytes = 0;
+  int ensure(size_t n) {
+    if (n <= bytes && p != nullptr) return 0;
+    release();
+    const hipError_t e = hipHostMalloc(&p, n, hipHostMallocDefault);
+    if (e != hipSuccess) {
+      p = nullptr;
+      return fail(FKPM_E_HIP, "hipHostMalloc(%zu bytes): %s", n, hipGetErrorString(e));
+    }
+    bytes = n;
+    return 0;
+  }
+  void release() {
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    bytes = 0;
   }
 };
 
@@ -315,6 +355,18 @@ struct fkpm_handle {
   DevBuf rdesc;            // {row, first block, end block} per sweep position
   long long table_cap_mb = -1;  // FKPM_OPT_ALPHA_TABLE_MB (-1: the default budget)
 
+  // --- whole-recursion kernels of small lattices (kpm_resident.h) ---
+  struct Resident {
+    bool packed = false;  // hval / hoff hold the current H
+    int rpt = 0, threads = 0, nt = 0;
+    DevBuf hval, hoff, atab, btab, xi, coef, part;
+    PinBuf pin;           // coefficients in, moment sums out
+    fkd::ResSet<double> kd;
+    fkd::ResSet<float> kf;
+    bool state = false;   // the held moments state (alpha_M) is atab's
+    int K = 0;            // atab holds alpha_0 .. alpha_K of the current H and R
+  } res;
+
   // --- D ---
   int nbD = 0, nnzbD = 0;
   bool d_set = false, d_sym = false, d_fused = false, d_valid = false;
@@ -347,6 +399,9 @@ struct fkpm_handle {
     DevBuf* m2bufs[] = {&j_rp[0], &j_ci[0], &j_rb[0], &j_raw[0], &j_val[0], &j_rp[1], &j_ci[1],
                         &j_rb[1], &j_raw[1], &j_val[1], &m2_a, &m2_b, &m2_ring, &m2_c, &m2_part};
     for (DevBuf* d : m2bufs) d->release();
+    DevBuf* rbufs[] = {&res.hval, &res.hoff, &res.atab, &res.btab, &res.xi, &res.coef, &res.part};
+    for (DevBuf* d : rbufs) d->release();
+    res.pin.release();
     gcache.clear();
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
@@ -365,7 +420,18 @@ struct fkpm_handle {
   }
   template <class S>
   const fkd::KSet<S>& ks(int kind) const;
+  template <class S>
+  fkd::ResSet<S>& rset();
 };
+
+template <>
+fkd::ResSet<double>& fkpm_handle::rset<double>() {
+  return res.kd;
+}
+template <>
+fkd::ResSet<float>& fkpm_handle::rset<float>() {
+  return res.kf;
+}
 
 template <>
 const fkd::KSet<double>& fkpm_handle::ks<double>(int kind) const {
@@ -748,6 +814,7 @@ int ensure_ready(fkpm_handle* h) {
   h->r_dirty = false;
   h->alpha_M = 0;
   h->tab_K = 0;
+  h->res.K = 0;
   if (h->autotune_on_use && !h->tuned && h->force_L == 0) CHK(tune(h));
   return 0;
 }
@@ -1000,12 +1067,265 @@ int tune_t(fkpm_handle* h) {
 
 int tune(fkpm_handle* h) { return h->single ? tune_t<float>(h) : tune_t<double>(h); }
 
+// mu from the dots of each step, sums[2m] = |alpha_m|^2 and sums[2m+1] =
+// Re<alpha_{m+1}, alpha_m>.
+void moments_from_sums(const double* ps, int nsteps, double* mu) {
+  mu[0] = ps[0];
+  mu[1] = ps[1];
+  for (int m = 1; m < nsteps; m++) {
+    mu[2 * m] = 2 * ps[2 * m] - mu[0];
+    mu[2 * m + 1] = 2 * ps[2 * m + 1] - mu[1];
+  }
+}
+
+// Weights of the table vectors in stoch_matrix (stoch_table): d_0 .. d_K of v,
+// then e_0 .. e_K of u.
+void stoch_table_weights(int M, const double* c, std::vector<double>& w) {
+  const int K = (M + 1) / 2;
+  auto cm = [&](int m) { return m < M ? c[m] : 0.0; };
+  w.assign(2 * (size_t)(K + 1), 0.0);
+  for (int i = 0; i <= K; i++) {
+    w[i] = (i < K ? cm(i) : 0.0) - (i >= 1 ? cm(2 * K - i) : 0.0);  // d_i
+    w[K + 1 + i] = i < K ? cm(K + i) : 0.0;                         // e_i
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Whole-recursion kernels of small lattices (kpm_resident.h): moments,
+// autodiff_matrix and stoch_matrix as one launch per recursion.
+// ---------------------------------------------------------------------------
+
+// LDS of one workgroup.
+constexpr size_t kLdsBytes = 160 << 10;
+// Bytes of H beyond its registers that a workgroup of the backward recursion may
+// read from the L2 in every step.  A call of M = 128 (us, resident against the
+// step kernels; S columns):
+//                       KiB streamed   moments      autodiff_matrix
+//   32x32 x 2, S 32           267     127 / 386      271 / 640
+//   12^3 x 2, S 16            803     407 / 423      618 / 694
+//   8^3 x 4, S 32             910     481 / 580      670 / 1650
+//   64^2 x 1, S 16            320     227 / 400      633 / 521
+// so up to 1 MiB the two calls together gain; past it (14^3 x 2 and larger) a
+// column no longer fits the LDS twice in FP64.
+constexpr size_t kResStream = 1024 << 10;
+
+bool find_res(fkpm_handle* h, int rpt) {
+  if (h->single)
+    return h->cx ? fkd::find_res_fc(h->b, rpt, &h->res.kf) : fkd::find_res_fr(h->b, rpt, &h->res.kf);
+  return h->cx ? fkd::find_res_dc(h->b, rpt, &h->res.kd) : fkd::find_res_dr(h->b, rpt, &h->res.kd);
+}
+
+// Scalars between the orders of a resident table, and of one order.
+size_t res_count(const fkpm_handle* h) { return (size_t)h->n * h->s * (h->cx ? 2 : 1); }
+size_t res_slot(const fkpm_handle* h) { return (res_count(h) + 63) / 64 * 64; }
+
+// Whether the whole-recursion kernels run for the current H and R: the
+// defaults of every switch that names a step kernel or the table (a forced
+// geometry, sweep, order, graph or table mode asks for the step kernels), and a
+// column that fits the LDS twice with little of H left to stream.
+template <class S>
+bool res_wanted(fkpm_handle* h) {
+  if (h->force_L > 0 || h->max_wg > 0 || h->sweep_force >= 0 || h->slice_force >= 0 ||
+      h->order_force >= 0 || h->graph_mode == 1 || h->store_alpha != 1 || h->table_cap_mb >= 0 ||
+      !h->mfma_on || h->rr_force)
+    return false;
+  const int rmax = fkd::res_max_rpt(h->b);
+  if (h->nb > fkd::RES_T * rmax) return false;
+  int rpt = 1;
+  while (h->nb > fkd::RES_T * rpt) rpt *= 2;
+  if (!find_res(h, rpt)) return false;
+  const fkd::ResSet<S>& rs = h->rset<S>();
+  if (2 * ((size_t)(h->nb + 1) * rs.elem_bytes + 16) > kLdsBytes) return false;
+  const int threads = ((h->nb + rpt - 1) / rpt + 63) / 64 * 64;
+  if (h->max_deg > rs.dreg_bwd[0]) {
+    const int d = h->max_deg - rs.dreg_bwd[1];
+    if ((size_t)d * (rs.block_bytes + 4) * h->nb > kResStream) return false;
+  }
+  if (rpt != h->res.rpt || threads != h->res.threads) h->res.packed = false;
+  h->res.rpt = rpt;
+  h->res.threads = threads;
+  h->res.nt = rpt * threads;
+  return true;
+}
+
+// The tables of forward and backward vectors, within the budget of the step
+// kernels' table (moments_t).
+int res_tables(fkpm_handle* h, size_t abytes, size_t bbytes, bool* ok) {
+  fkpm_handle::Resident& r = h->res;
+  size_t budget = ~(size_t)0;
+  if (abytes > r.atab.bytes || bbytes > r.btab.bytes) {
+    size_t free_b = 0, total_b = 0;
+    HIPCHK(hipMemGetInfo(&free_b, &total_b));
+    budget = std::min(free_b / 2 + r.atab.bytes + r.btab.bytes, total_b / 4);
+  }
+  if (const char* e = getenv("FKPM_ALPHA_TABLE_BYTES")) budget = (size_t)strtoull(e, nullptr, 10);
+  *ok = abytes + bbytes <= budget;
+  if (!*ok) return 0;
+  CHK(r.atab.ensure(abytes));
+  return r.btab.ensure(bbytes);
+}
+
+template <class S>
+fkd::ResH<S> res_H(const fkpm_handle* h) {
+  fkd::ResH<S> H;
+  H.val = h->res.hval.as<const S>();
+  H.off = h->res.hoff.as<const int>();
+  H.nb = h->nb;
+  H.nt = h->res.nt;
+  H.deg = h->max_deg;
+  return H;
+}
+
+template <class S>
+int res_pack(fkpm_handle* h) {
+  if (h->res.packed) return 0;
+  const fkd::ResSet<S>& rs = h->rset<S>();
+  const size_t blocks = (size_t)h->res.nt * h->max_deg;
+  CHK(h->res.hval.ensure(blocks * rs.block_bytes + 16));
+  CHK(h->res.hoff.ensure(blocks * sizeof(int) + 16));
+  if (blocks > 0)
+    CHK(launch(rs.pack, dim3(grid_for(blocks)), dim3(fkd::WG), h->stream, h->rp.as<const int>(),
+               h->ci.as<const int>(), h->hv.as<const S>(), h->nb, h->res.nt, h->max_deg,
+               h->res.hval.as<S>(), h->res.hoff.as<int>()));
+  h->res.packed = true;
+  return 0;
+}
+
+template <class S>
+size_t res_lds(fkpm_handle* h) {
+  return 2 * (((size_t)(h->nb + 1) * h->rset<S>().elem_bytes + 15) / 16 * 16);
+}
+
+// Coefficients to the device: pinned memory, read by a kernel on the stream.
+int res_coef(fkpm_handle* h, const double* c, int M) {
+  CHK(h->res.pin.ensure((size_t)M * sizeof(double)));
+  CHK(h->res.coef.ensure((size_t)M * sizeof(double)));
+  memcpy(h->res.pin.p, c, (size_t)M * sizeof(double));
+  return launch(&fkd::k_res_coef, dim3((M + fkd::WG - 1) / fkd::WG), dim3(fkd::WG), h->stream,
+                (const double*)h->res.pin.p, h->res.coef.as<double>(), M);
+}
+
+// *done = false when the table does not fit (nothing was launched).
+template <class S>
+int res_moments(fkpm_handle* h, int M, double* mu, bool* done) {
+  const int nsteps = M / 2;
+  const fkd::ResSet<S>& rs = h->rset<S>();
+  const size_t slot = res_slot(h), cnt = res_count(h);
+  *done = false;
+  bool ok = false;
+  h->res.K = 0;
+  CHK(res_tables(h, (size_t)(nsteps + 1) * slot * sizeof(S), (size_t)nsteps * slot * sizeof(S), &ok));
+  if (!ok) return 0;
+  CHK(res_pack<S>(h));
+  // about 2048 packets per workgroup of the dots
+  const int ny = (int)std::min<size_t>(16, std::max<size_t>(1, cnt * sizeof(S) / 16 / 2048));
+  CHK(h->partial.ensure((size_t)nsteps * ny * 2 * sizeof(double)));
+  CHK(h->res.pin.ensure((size_t)nsteps * 2 * sizeof(double)));
+  CHK(timing_begin(h));
+  CHK(launch_lds(rs.fwd[h->max_deg > rs.dreg_fwd[0]], dim3(h->s), dim3(h->res.threads), res_lds<S>(h), h->stream,
+                 res_H<S>(h), h->R.as<const S>(), h->sp, h->res.atab.as<S>(), slot, nsteps));
+  CHK(timing_end(h, &h->ms_mom, &h->n_mom, nsteps));
+  CHK(launch(&fkd::k_res_dots<S>, dim3(nsteps, ny), dim3(fkd::WG), h->stream,
+             h->res.atab.as<const S>(), slot, cnt, h->partial.as<double>()));
+  double* ps = static_cast<double*>(h->res.pin.p);
+  CHK(launch(&fkd::k_reduce_partials, dim3(nsteps), dim3(fkd::WG), h->stream,
+             (const double*)h->partial.as<double>(), ny, ps));
+  HIPCHK(hipStreamSynchronize(h->stream));
+  moments_from_sums(ps, nsteps, mu);
+  h->res.K = nsteps;
+  h->res.state = true;
+  h->a_stored = false;
+  h->alpha_M = M;
+  *done = true;
+  return 0;
+}
+
+// dst = the D sum over the terms T (nterm of them) on D's pattern.
+template <class S>
+int res_outer(fkpm_handle* h, const fkd::ResTerms<S>& T, int nterm, double* dst) {
+  const size_t cnt = (size_t)h->nnzbD * h->b * h->b * (h->cx ? 2 : 1);
+  if (cnt == 0) return 0;
+  const int gx = (h->nnzbD + fkd::WG - 1) / fkd::WG;
+  const long long pairs = (long long)nterm * h->s;
+  // about 2048 workgroups, at least 16 products a thread, 64 MiB of partial sums
+  long long ny = std::min<long long>({std::max(1, 2048 / gx), (pairs + 15) / 16,
+                                      std::max<long long>(1, (64ll << 20) / (long long)(cnt * 8))});
+  const int per = (int)((pairs + ny - 1) / ny);
+  ny = (pairs + per - 1) / per;
+  CHK(h->res.part.ensure((size_t)ny * cnt * sizeof(double)));
+  const dim3 grid(gx, (int)ny), block(fkd::WG);
+  auto go = [&](auto fn) {
+    return launch(fn, grid, block, h->stream, h->drp.as<const int>(), h->dci.as<const int>(), h->nb,
+                  h->nnzbD, T, nterm, h->s, per, h->res.part.as<double>());
+  };
+  int rc = FKPM_E_UNSUP;
+  if (h->b == 1) rc = h->cx ? go(&fkd::k_res_outer<S, true, 1>) : go(&fkd::k_res_outer<S, false, 1>);
+  if (h->b == 2) rc = h->cx ? go(&fkd::k_res_outer<S, true, 2>) : go(&fkd::k_res_outer<S, false, 2>);
+  if (h->b == 4) rc = h->cx ? go(&fkd::k_res_outer<S, true, 4>) : go(&fkd::k_res_outer<S, false, 4>);
+  CHK(rc);
+  return launch(&fkd::k_res_outer_sum, dim3(grid_for(cnt)), block, h->stream,
+                (const double*)h->res.part.as<double>(), (int)ny, cnt, dst);
+}
+
+// The backward recursion and D from the resident table, into dacc.
+template <class S>
+int res_autodiff(fkpm_handle* h, int M, const double* c, double diag) {
+  const int M2 = M / 2;
+  const fkd::ResSet<S>& rs = h->rset<S>();
+  const size_t slot = res_slot(h);
+  CHK(timing_begin(h));
+  if (M2 > 1) {
+    CHK(res_coef(h, c, M));
+    CHK(launch_lds(rs.bwd[h->max_deg > rs.dreg_bwd[0]], dim3(h->s), dim3(h->res.threads), res_lds<S>(h), h->stream,
+                   res_H<S>(h), h->res.atab.as<const S>(), h->res.btab.as<S>(), slot, M2,
+                   h->res.coef.as<const double>(), 2 * c[M - 1]));
+  }
+  fkd::ResTerms<S> T{h->res.atab.as<const S>(), h->res.btab.as<const S>(), slot, M2, diag,
+                     2 * c[M - 1]};
+  CHK(res_outer<S>(h, T, M2 > 1 ? M2 + 1 : 1, h->dacc.as<double>()));
+  return timing_end(h, &h->ms_ad, &h->n_ad, M2 - 1);
+}
+
+// xi by the Clenshaw recurrence, or from the resident table, then D into dout.
+template <class S>
+int res_stoch(fkpm_handle* h, int M, const double* c, bool table) {
+  const size_t slot = res_slot(h), vb = slot * sizeof(S);
+  const fkd::ResSet<S>& rs = h->rset<S>();
+  CHK(res_pack<S>(h));
+  CHK(h->res.xi.ensure(3 * vb));
+  S* u = h->res.xi.as<S>();
+  S* v = u + slot;
+  S* xi = v + slot;
+  const int K = (M + 1) / 2;
+  std::vector<double> w;
+  if (table) {
+    stoch_table_weights(M, c, w);
+    CHK(res_coef(h, w.data(), (int)w.size()));
+    CHK(launch(&fkd::k_table_sums<S>, dim3(grid_for(slot)), dim3(fkd::WG), h->stream,
+               h->res.atab.as<const S>(), h->res.atab.as<const S>() + slot, slot, K,
+               h->res.coef.as<const double>(), h->res.coef.as<const double>() + K + 1, u, v, slot));
+  } else {
+    CHK(res_coef(h, c, M));
+  }
+  const S* r0 = table ? h->res.atab.as<const S>() : u;
+  CHK(launch_lds(rs.xi[h->max_deg > rs.dreg_xi[0]], dim3(h->s), dim3(h->res.threads), res_lds<S>(h), h->stream,
+                 res_H<S>(h), h->R.as<const S>(), h->sp, (const S*)(table ? u : nullptr),
+                 (const S*)v, h->res.coef.as<const double>(), table ? K : M, u, xi));
+  return res_outer<S>(h, fkd::ResTerms<S>{r0, xi, slot, 0, 0.0, 0.0}, 2, h->dout.as<double>());
+}
+
 // ---------------------------------------------------------------------------
 // moments (engine_cpu.cpp:63-84; engine_cusparse.cpp:755-791)
 // ---------------------------------------------------------------------------
 template <class S>
 int moments_t(fkpm_handle* h, int M, double* mu) {
   const int nsteps = M / 2;
+  if (res_wanted<S>(h)) {
+    bool done = false;
+    CHK(res_moments<S>(h, M, mu, &done));
+    if (done) return 0;
+  }
+  h->res.state = false;
   CHK(ensure_partials(h, nsteps));
   // keep every alpha_k for autodiff_matrix (no backward recomputation of
   // alpha) when wanted (table_wanted), the table fits half the free device
@@ -1055,12 +1375,7 @@ int moments_t(fkpm_handle* h, int M, double* mu) {
   HIPCHK(hipMemcpyAsync(ps.data(), h->psum.p, ps.size() * sizeof(double), hipMemcpyDeviceToHost,
                         h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
-  mu[0] = ps[0];
-  mu[1] = ps[1];
-  for (int m = 1; m < nsteps; m++) {
-    mu[2 * m] = 2 * ps[2 * m] - mu[0];
-    mu[2 * m + 1] = 2 * ps[2 * m + 1] - mu[1];
-  }
+  moments_from_sums(ps.data(), nsteps, mu);
   h->alpha_M = M;
   return 0;
 }
@@ -1151,13 +1466,8 @@ int stoch_table(fkpm_handle* h, int M, const double* c, const S** xi_out) {
   const auto& ks = h->ks<S>(K_MOM);
   const dim3 grid(kc.nwg), block(fkd::WG);
   const size_t vb = h->vbytes();
-  auto cm = [&](int m) { return m < M ? c[m] : 0.0; };
   std::vector<double>& w = h->tabc_host;
-  w.assign(2 * (size_t)(K + 1), 0.0);
-  for (int i = 0; i <= K; i++) {
-    w[i] = (i < K ? cm(i) : 0.0) - (i >= 1 ? cm(2 * K - i) : 0.0);  // d_i
-    w[K + 1 + i] = i < K ? cm(K + i) : 0.0;                         // e_i
-  }
+  stoch_table_weights(M, c, w);
   CHK(h->tabc.ensure(w.size() * sizeof(double)));
   HIPCHK(hipMemcpyAsync(h->tabc.p, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice,
                         h->stream));
@@ -1202,6 +1512,15 @@ int stoch_t(fkpm_handle* h, int M, const double* c) {
   const size_t dcount = (size_t)h->nnzbD * h->b * h->b * (h->cx ? 2 : 1);
   const KCfg& ko = h->kc[K_OUT];
   const auto& kso = h->ks<S>(K_OUT);
+  if (h->stoch_method != FKPM_STOCH_FORWARD && res_wanted<S>(h)) {
+    const bool table = h->stoch_method == FKPM_STOCH_AUTO && h->res.K >= (M + 1) / 2;
+    h->stoch_used = table ? FKPM_STOCH_TABLE : FKPM_STOCH_CLENSHAW;
+    CHK(timing_begin(h));
+    CHK(res_stoch<S>(h, M, c, table));
+    CHK(timing_end(h, &h->ms_stoch, &h->n_stoch, table ? (M + 1) / 2 + 1 : M - 1));
+    h->alpha_M = 0;
+    return 0;
+  }
   CHK(timing_begin(h));
   const bool table = h->stoch_method == FKPM_STOCH_AUTO && h->tab_K >= (M + 1) / 2;
   h->stoch_used = table ? FKPM_STOCH_TABLE
@@ -1264,6 +1583,23 @@ int stoch_t(fkpm_handle* h, int M, const double* c) {
 // ---------------------------------------------------------------------------
 // autodiff_matrix (engine_cpu.cpp:255-304; engine_cusparse.cpp:955-1039)
 // ---------------------------------------------------------------------------
+// D = (symmetrized dacc) / mag into dout; the end of autodiff_matrix.
+int finish_autodiff(fkpm_handle* h) {
+  const double* dacc = h->dacc.as<const double>();
+  // symmetrize + scale(1/mag)
+  const size_t dcnt = (size_t)h->nnzbD * h->b * h->b;
+  if (h->cx)
+    CHK(launch(&fkd::k_symmetrize_scale<true>, dim3(grid_for(dcnt)), dim3(256), h->stream,
+               (const double*)dacc, h->dout.as<double>(), h->tpos.as<const int>(), h->nnzbD, h->b,
+               1.0 / h->mag));
+  else
+    CHK(launch(&fkd::k_symmetrize_scale<false>, dim3(grid_for(dcnt)), dim3(256), h->stream,
+               (const double*)dacc, h->dout.as<double>(), h->tpos.as<const int>(), h->nnzbD, h->b,
+               1.0 / h->mag));
+  h->alpha_M = 0;  // engine_cpu.cpp:301-303
+  return 0;
+}
+
 template <class S>
 int autodiff_t(fkpm_handle* h, int M, const double* c) {
   const dim3 block(fkd::WG);
@@ -1283,6 +1619,10 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
 
   double diag = c[1];
   for (int m = 1; m < M / 2; m++) diag -= c[2 * m + 1];
+  if (h->res.state) {
+    CHK(res_autodiff<S>(h, M, c, diag));
+    return finish_autodiff(h);
+  }
   CHK(zero_doubles(h, dacc, dcount));
   // D = diag R R^+
   CHK(launch(kso.outer_ss, dim3(ko.nwg), block, h->stream, drp, dci, (const S*)h->vec_a(0),
@@ -1337,18 +1677,7 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
   }
   CHK(rec.run());
   CHK(timing_end(h, &h->ms_ad, &h->n_ad, launches));
-  // symmetrize + scale(1/mag)
-  const size_t dcnt = (size_t)h->nnzbD * h->b * h->b;
-  if (h->cx)
-    CHK(launch(&fkd::k_symmetrize_scale<true>, dim3(grid_for(dcnt)), dim3(256), h->stream,
-               (const double*)dacc, h->dout.as<double>(), h->tpos.as<const int>(), h->nnzbD, h->b,
-               1.0 / h->mag));
-  else
-    CHK(launch(&fkd::k_symmetrize_scale<false>, dim3(grid_for(dcnt)), dim3(256), h->stream,
-               (const double*)dacc, h->dout.as<double>(), h->tpos.as<const int>(), h->nnzbD, h->b,
-               1.0 / h->mag));
-  h->alpha_M = 0;  // engine_cpu.cpp:301-303
-  return 0;
+  return finish_autodiff(h);
 }
 
 // ---------------------------------------------------------------------------
@@ -1992,6 +2321,8 @@ int fkpm_set_H(fkpm_handle* h, int nb, int b, int nnzb, const int* row_ptr, cons
   h->h_set = true;
   h->alpha_M = 0;
   h->tab_K = 0;
+  h->res.K = 0;
+  h->res.packed = false;
   if (geo_change) h->r_dirty = true;
   return 0;
 }
@@ -2011,6 +2342,7 @@ int fkpm_set_R(fkpm_handle* h, int n, int s, const void* R_colmajor) {
   h->r_dirty = true;
   h->alpha_M = 0;
   h->tab_K = 0;
+  h->res.K = 0;
   return 0;
 }
 
