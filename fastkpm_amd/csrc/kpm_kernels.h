@@ -221,6 +221,26 @@ __device__ __forceinline__ void reduce_scatter(T* v, int l) {
   rs_level<1, L, NV>(v, l);
 }
 
+// Most values of a D block that the fused outer product reduces with one
+// reduce-scatter (complex 4x4 blocks: 31 adds and moves a lane where one
+// butterfly per value took 32 x log2 L; backward step at 16^3 sites x 4
+// orbitals, S = 72, FP64: 125 -> 61 us recomputing alpha, 81 -> 50 us reading the
+// table).  Larger blocks take a butterfly per value.
+constexpr int RS_MAX = 32;
+
+// The type the lane sums of NV values are reduced in: the storage type up to
+// 2x2 complex blocks, FP64 for larger ones.
+template <typename A, int NV>
+struct RsTypeOf {
+  typedef A type;
+};
+template <>
+struct RsTypeOf<float, 32> {
+  typedef double type;
+};
+template <typename A, int NV>
+using RsType = typename RsTypeOf<A, NV>::type;
+
 // First index owned by lane l after reduce_scatter<L, NV>.
 template <int L, int NV>
 __device__ __forceinline__ int rs_base(int l) {
@@ -773,7 +793,7 @@ __global__ __launch_bounds__(WG) void k_step_xi(
 }
 
 // The D entries one lane updates in a fused outer-product block p (the
-// layouts of the D updates in the autodiff steps): with NV = B*B*HS <= 16
+// layouts of the D updates in the autodiff steps): with NV = B*B*HS <= RS_MAX
 // scalars per block, the CNT entries at rs_base after the reduce-scatter;
 // otherwise own element o*L + l of the block (o < DOWN), HS scalars each.
 template <int N>
@@ -793,11 +813,11 @@ __device__ __forceinline__ auto load_dpre(const double* __restrict__ dacc, int p
   using GE = Geo<S, CX, B, L, KQ>;
   constexpr int HS = GE::HS;
   constexpr int NV = GE::DE * HS;
-  if constexpr (!FUSED_D || (NV > 16 && GE::DOWN * HS > 8)) {
+  if constexpr (!FUSED_D || (NV > RS_MAX && GE::DOWN * HS > 8)) {
     // large blocks (b = 8 on the vector units): the entries would hold too
     // many registers across the gather; the update reads them itself
     return NoPre{};
-  } else if constexpr (NV <= 16) {
+  } else if constexpr (NV <= RS_MAX) {
     constexpr int CNT = NV >= L ? NV / L : 1;
     DVals<CNT> d{};
     if (NV >= L || l < NV) {
@@ -883,11 +903,11 @@ __device__ __forceinline__ void step_autodiff_dev(
       gather_row_pre<S, A, CX, B, L, KQ, 2, true>(
           ci, hv, X, rs, qo, p0, p1, acc, [&](int p, int, auto& xv, const DPre& dp) {
             constexpr int NV = GE::DE * HS;  // scalars of one D block
-            if constexpr (FUSED_D && NV <= 16) {
+            if constexpr (FUSED_D && NV <= RS_MAX) {
               // D_p(bi, bj) += fD * sum_s alpha_m[B i + bi, s] conj(beta_{m+1}[B j + bj, s]):
               // per-lane partial sums of the whole block, then one reduce-scatter
-              // over the group in the storage precision, added to D in FP64
-              A v[NV];
+              // over the group in RsType, added to D in FP64
+              RsType<A, NV> v[NV];
 #pragma unroll
               for (int bj = 0; bj < B; bj++)
 #pragma unroll
@@ -1062,8 +1082,8 @@ __device__ __forceinline__ void step_autodiff_stored_dev(
         if constexpr (!FUSED_D) {
           (void)p;
           (void)xv;
-        } else if constexpr (NV <= 16) {
-          A v[NV];  // reduced in the storage precision, added to D in FP64
+        } else if constexpr (NV <= RS_MAX) {
+          RsType<A, NV> v[NV];  // (as in step_autodiff_dev)
 #pragma unroll
           for (int bj = 0; bj < B; bj++)
 #pragma unroll
