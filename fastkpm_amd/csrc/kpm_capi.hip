@@ -622,14 +622,32 @@ auto adp_fn(const fkd::KSet<S>& ks, const KCfg& c) {
   return c.mfma ? ks.mfma_ad_plain : ks.ad_plain;
 }
 
+// Last-level cache of the device (MI355X: 256 MB).
+constexpr size_t kLlcBytes = (size_t)256 << 20;
+
 // Default geometry of a kernel kind when nothing is tuned: one pass of width
-// wmax; the single-gather kinds take the widest lane groups (wave-uniform
-// rows), the kinds with block reductions groups of 16 lanes (one DPP row).
+// wmax.  From 64 packets on, whole waves per row (wave-uniform rows, scalar
+// offsets and H); below, two packets per lane, which keeps more loads in
+// flight per wave than twice the lanes.  Forward step (us), 64 x 1 / 16 x 4 /
+// 32 x 2 lanes x packets on 64: 256^2 x 2 FP64 81 / 98 / 110, 20^3 x 2 12.9 /
+// 14.9 / 16.2; 16 x 2 / 32 x 1 on 32: 256^2 x 2 FP32 37 / 47, 128^2 x 2 FP64
+// 14.4 / 18.1; 8 x 2 / 16 x 1 on 16: 31x29x27 real 7.2 / 10.6.  The backward
+// step reading the table takes 16 x 4 on 64 while its vectors stay in the
+// last-level cache (20^3 x 2: 23.4 against 26 us; 256^2 x 2: 171 against 165).
 KCfg default_cfg(fkpm_handle* h, int kind) {
-  static const int pref_gather[] = {64, 32, 16, 8, 4};
-  static const int pref_reduce[] = {16, 8, 32, 4, 64};
-  const int* pref = (kind == K_MOM || kind == K_XI || kind == K_MOMT) ? pref_gather : pref_reduce;
+  static const int wide[] = {64, 32, 16, 8, 4};
+  static const int pairs[] = {16, 8, 32, 4, 64};
+  static const int reduce[] = {16, 8, 32, 4, 64};
+  // vectors a step touches; one that writes a fresh table slot meets the ones
+  // of the steps before it in the cache too
+  const int nvec = kind == K_AD || kind == K_ADS ? 6 : kind == K_XI || kind == K_MOMT ? 5 : 3;
+  const bool cached = (size_t)nvec * h->vbytes() <= kLlcBytes;
+  const int* pref = kind == K_OUT || (kind == K_ADS && cached) ? reduce : h->wmax >= 64 ? wide : pairs;
   KCfg c;
+  if (pref == pairs && h->wmax >= 4 && compiled(h->b, h->wmax / 2, 2)) {
+    c.L = h->wmax / 2;
+    c.KQ = 2;
+  }
   for (int t = 0; t < 5 && c.L == 0; t++) {
     const int L = pref[t];
     if (h->wmax % L == 0 && compiled(h->b, L, h->wmax / L)) {
@@ -648,12 +666,16 @@ KCfg default_cfg(fkpm_handle* h, int kind) {
       }
     }
   }
-  c.maxwg = 4096;
+  c.maxwg = 16384;  // one pass over the rows at most sizes (256^2 x 2 FP64: 81 us, 4096: 87)
   c.nt = 0;
-  // one front in segments of two passes: what the tuner picks on the 2-D and
-  // 3-D lattices measured (C2 FP64: forward step 91 -> 81 us, autodiff 188
-  // -> 166 us against per-XCD regions)
-  c.sweep = 2;
+  // While a step's vectors stay in the last-level cache each XCD sweeps its own
+  // region, whose neighbour rows its L2 then holds (128^2 x 2 FP64 forward step
+  // 13.2 us against 16.6 in one front, 20^3 x 2 12.9 / 17.8, autodiff 25 / 30);
+  // past it one front in segments of two passes keeps far neighbours in the
+  // shared cache (256^2 x 2 FP64: 81 us, per XCD 92).  A sweep of fewer than
+  // 64 workgroups has no regions to speak of.
+  const int gwg = (fkd::WG / fkd::WAVE) * (fkd::WAVE / (c.L > 0 ? c.L : fkd::WAVE));
+  c.sweep = cached && h->nb / gwg >= 64 ? 0 : 2;
   if (mfma_avail(h, kind)) {
     c.mfma = 1;
     // row-resident: the forward step always, the autodiff step in FP64 and in
@@ -703,8 +725,22 @@ int choose_geometry(fkpm_handle* h) {
     if (w >= qp0 && (wmax == 0 || w < wmax)) wmax = w;
   }
   if (wmax == 0) wmax = widest;
-  // matrix-core tiles are 16 complex columns wide
-  if (h->mfma_on && h->cx && h->b == 8) wmax = std::max(wmax, 16 / ne);
+  // Matrix-core tiles are 16 complex columns wide (FP32 takes them in pairs) and
+  // a row may hold any number of them: of the compiled widths that are whole
+  // tiles, the one that pads the row least (144 columns: 144 instead of 192).
+  if (h->mfma_on && h->cx && h->b == 8) {
+    const int tile = qp0 <= 16 / ne ? 16 / ne : 16;
+    int best = 0;
+    for (int k = 0; k < ng; k++) {
+      const int w = gs[k].L * gs[k].KQ;
+      if (w % tile != 0) continue;
+      const int pad = (qp0 + w - 1) / w * w;
+      if (best == 0 || pad < best || (pad == best && w > wmax)) {
+        best = pad;
+        wmax = w;
+      }
+    }
+  }
   if (h->force_L > 0) {
     const int fkq = h->force_KQ > 0 ? h->force_KQ : 1;
     if (!compiled(h->b, h->force_L, fkq))
@@ -1850,6 +1886,12 @@ int moments2_t(fkpm_handle* h, int M, int col_chunk, size_t budget, double* mu) 
   if (!km.mfma && km.L * km.KQ == W) {
     ks = h->ks<S>(K_MOM);
     c = km;
+    if (!h->tuned && h->sweep_force < 0 && !(c.nt & fkd::NT_ORDER)) {
+      // every step writes a fresh column of A or B: one front, as past the
+      // last-level cache (default_cfg)
+      c.sweep = 2;
+      derive_grid(h->nb, c);
+    }
   } else {
     int L = 0, KQ = 0;
     if (!kset_for_width<S>(h, W, &ks, &L, &KQ))

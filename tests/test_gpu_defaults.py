@@ -1,0 +1,81 @@
+"""The untuned choices of the step kernels against the oracle (FP64, 1e-10): the
+per-XCD sweep and two-packet geometries of lattices past the whole-recursion
+kernels, the padded widths of the matrix-core kernels, and the fused 4x4 outer
+product reduced in one reduce-scatter on every compiled lane count."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from helpers import rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(oracle, H, S, M=8, prec="fp64", before=None, real=False):
+    from fastkpm_amd import EnergyScale, HipEngine
+    rng = np.random.default_rng(S)
+    n = H.n_rows * H.b_len
+    R = rng.standard_normal((n, S)) + (0 if real else 1j) * rng.standard_normal((n, S))
+    b = H.b_len
+    absrow = np.zeros((H.n_rows, b))
+    np.add.at(absrow, H.row_idx, np.abs(H.val.reshape(-1, b, b)).sum(axis=1))
+    bound = float(absrow.max())
+    eng = HipEngine("double" if real else "cx_double", prec)
+    if before:
+        before(eng)
+    eng.set_R(R)
+    eng.set_H(H, EnergyScale(-bound, bound))
+    orc = oracle.Engine()
+    orc.set_H(H, -bound, bound)
+    orc.set_R(R)
+    c = 1.0 / (1.0 + np.arange(M))
+    tol = 1e-10 if prec == "fp64" else M * 16 * 2.0 ** -24
+    D = H.like()
+    assert rel_err(eng.moments(M), orc.moments(M)) < tol
+    eng.autodiff_matrix(c, D)
+    assert rel_err(D.val, orc.autodiff_matrix(c, D)) < tol
+    eng.stoch_matrix(c, D)
+    assert rel_err(D.val, orc.stoch_matrix(c, D)) < tol
+    return eng
+
+
+# N past the whole-recursion kernels; S at and beside the compiled widths
+@pytest.mark.parametrize("shape,b,S,real", [((70, 61), 1, 8, False), ((70, 61), 1, 17, True),
+                                            ((17, 16, 16), 1, 33, False), ((48, 45), 2, 16, False),
+                                            ((48, 45), 2, 31, False), ((48, 45), 2, 64, False),
+                                            ((13, 13, 14), 2, 65, False)])
+def test_default_sweep_and_geometry(oracle, shape, b, S, real):
+    from fastkpm_amd import lattice
+    H = lattice.lattice(shape, b=b, W=1.0, J=0.0 if b == 1 else 1.0, seed=3,
+                        dtype=np.float64 if real else np.complex128)
+    eng = _run(oracle, H, S, real=real)
+    c = eng.kernel_config(0)
+    assert c["sweep"] in (0, 2)
+    eng.close()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("S", [1, 16, 17, 33, 48, 80, 144])
+def test_matrix_core_padded_width(oracle, S, prec):
+    """144 columns take 144 (FP64) or 160 (FP32, pairs of tiles), not 192."""
+    from fastkpm_amd import lattice
+    H = lattice.lattice((4, 3, 3), b=8, orbital_blocks=True, seed=S)
+    eng = _run(oracle, H, S, prec=prec)
+    tile = 16 if prec == "fp64" or S <= 16 else 32
+    assert eng.config()["s_padded"] == -(-S // tile) * tile
+    assert eng.kernel_config(0)["mfma"]
+    eng.close()
+
+
+@pytest.mark.parametrize("lanes,kq", [(4, 1), (4, 2), (8, 2), (16, 1), (16, 2), (32, 1), (32, 2),
+                                      (64, 1), (64, 2)])
+@pytest.mark.parametrize("store", [0, 2])
+def test_fused_4x4_outer_product(oracle, lanes, kq, store):
+    from fastkpm_amd import lattice
+    H = lattice.lattice((5, 4), b=4, orbital_blocks=True, seed=2)
+
+    def force(eng):
+        eng.set_geometry(lanes, kq, 0)
+        eng.set_store_alpha(store)
+    _run(oracle, H, 11, before=force).close()
