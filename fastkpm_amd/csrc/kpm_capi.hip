@@ -544,9 +544,10 @@ void derive_grid(int nb, KCfg& c) {
 }
 
 // Matrix-core kernels exist for complex 8x8 blocks (forward/Clenshaw steps,
-// also into the table, and the autodiff step that recomputes alpha).
+// also into the table, and both autodiff steps).
 bool mfma_avail(const fkpm_handle* h, int kind) {
-  return h->mfma_on && h->cx && h->b == 8 && (kind == K_MOM || kind == K_MOMT || kind == K_AD);
+  return h->mfma_on && h->cx && h->b == 8 &&
+         (kind == K_MOM || kind == K_MOMT || kind == K_AD || kind == K_ADS);
 }
 
 // The row-resident variants: rows of at most kRowResidentMax blocks (MF_DM of
@@ -620,6 +621,18 @@ auto adf_fn(const fkpm_handle* h, const fkd::KSet<S>& ks, const KCfg& c) {
 template <class S>
 auto adp_fn(const fkd::KSet<S>& ks, const KCfg& c) {
   return c.mfma ? ks.mfma_ad_plain : ks.ad_plain;
+}
+// The backward steps reading the table, as adf_fn / adp_fn choose.
+template <class S>
+auto ads_fn(const fkpm_handle* h, const fkd::KSet<S>& ks, const KCfg& c) {
+  if (c.mfma == 2 && ks.mfma_ads[fkd::ADS_RR2] != nullptr && h->qp % 16 == 0)
+    return ks.mfma_ads[c.dm == 7 ? fkd::ADS_RR2_7 : fkd::ADS_RR2];
+  if (c.mfma == 2) return ks.mfma_ads[c.dm == 7 ? fkd::ADS_RR7 : fkd::ADS_RR];
+  return c.mfma ? ks.mfma_ads[fkd::ADS_FUSED] : ks.ad_stored;
+}
+template <class S>
+auto adsp_fn(const fkd::KSet<S>& ks, const KCfg& c) {
+  return c.mfma ? ks.mfma_ads[fkd::ADS_PLAIN] : ks.ad_stored_plain;
 }
 
 // Last-level cache of the device (MI355X: 256 MB).
@@ -937,7 +950,7 @@ int tune_t(fkpm_handle* h) {
   const int kinds[] = {K_MOM, K_XI, K_AD, K_MOMT, K_ADS};
   for (int kind : kinds) {
     if (kind == K_MOMT) {
-      if (table_wanted(h) && !h->kc[K_AD].mfma) {
+      if (table_wanted(h)) {
         const size_t want = ((size_t)512 << 20) / vb + 1;
         const int n = (int)std::min<size_t>(64, std::max<size_t>(8, want));
         size_t free_b = 0, total_b = 0;
@@ -955,8 +968,7 @@ int tune_t(fkpm_handle* h) {
       }
       if (ns == 0) {
         CHK(set_kind(h, K_MOMT, h->kc[K_MOM]));
-        // no table while autodiff runs on the matrix cores
-        CHK(set_kind(h, K_ADS, h->kc[K_AD].mfma ? default_cfg(h, K_ADS) : h->kc[K_AD]));
+        CHK(set_kind(h, K_ADS, h->kc[K_AD]));
         break;
       }
     }
@@ -1018,7 +1030,7 @@ int tune_t(fkpm_handle* h) {
             if (kind == K_ADS) {  // backward over slots ns-2 .. 1, beta in the ring
               const int t = tstep++;
               const int m = ns - 2 - t % (ns - 2);
-              return launch(ks.ad_stored, dim3(k.nwg), dim3(fkd::WG), h->stream, rp_for(h, k), ci,
+              return launch(ads_fn(h, ks, k), dim3(k.nwg), dim3(fkd::WG), h->stream, rp_for(h, k), ci,
                             hv, (const S*)slot(m), (const S*)slot(m + 1),
                             (const S*)bring[(t + 1) % 3], (const S*)bring[t % 3],
                             (const S*)slot(m - 1), bring[(t + 2) % 3], h->tune_dacc.as<double>(),
@@ -1364,9 +1376,8 @@ int moments_t(fkpm_handle* h, int M, double* mu) {
   h->res.state = false;
   CHK(ensure_partials(h, nsteps));
   // keep every alpha_k for autodiff_matrix (no backward recomputation of
-  // alpha) when wanted (table_wanted), the table fits half the free device
-  // memory (or the byte count in FKPM_ALPHA_TABLE_BYTES) and the autodiff
-  // step runs on the vector units.
+  // alpha) when wanted (table_wanted) and the table fits half the free device
+  // memory (or the byte count in FKPM_ALPHA_TABLE_BYTES).
   {
     const size_t need = (size_t)nsteps * h->vbytes();
     size_t free_b = 0, total_b = 0;
@@ -1378,7 +1389,7 @@ int moments_t(fkpm_handle* h, int M, double* mu) {
     if (h->table_cap_mb >= 0) budget = (size_t)h->table_cap_mb << 20;
     if (const char* e = getenv("FKPM_ALPHA_TABLE_BYTES")) budget = (size_t)strtoull(e, nullptr, 10);
     h->a_stored = false;
-    if (table_wanted(h) && !h->kc[K_AD].mfma && need <= budget) {
+    if (table_wanted(h) && need <= budget) {
       h->tab_K = 0;  // rewritten below (and lost if the table grows)
       CHK(h->atab.ensure(need));
       h->a_stored = true;
@@ -1670,7 +1681,7 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
   LoopRecorder rec(h);
   if (M > 2) {
     const double sb = 2 * c[M - 1];  // beta_{M/2} = 2 c_{M-1} alpha_{M/2-1}
-    const bool stored = h->a_stored && !ka.mfma;
+    const bool stored = h->a_stored;
     for (int m = M / 2 - 1; m >= 1; m--) {
       // alpha_m, alpha_{m+1} and alpha_{m-1}: from the table, or the ring with
       // alpha_{m-1} recomputed by the step
@@ -1689,7 +1700,7 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
         if (!h->d_fused)  // D += 2 alpha_m beta_{m+1}^+ on D's own pattern
           CHK(launch(kso.outer_ss, dim3(ko.nwg), block, h->stream, drp, dci, am, first ? am : bm1,
                      dacc, h->nb, h->qp, ko.chunk, first ? 2.0 * sb : 2.0));
-        CHK(launch(h->d_fused ? kst.ad_stored : kst.ad_stored_plain, dim3(kt.nwg), block,
+        CHK(launch(h->d_fused ? ads_fn(h, kst, kt) : adsp_fn(kst, kt), dim3(kt.nwg), block,
                    h->stream, rp_for(h, kt), ci, hv, am, am1, bm1, bm2, (const S*)aout, bout, dacc,
                    h->nb, h->qp, kt.chunk, c4, c2, w, sb, sb2, 2.0, kt.nt));
       } else if (h->d_fused) {

@@ -73,8 +73,17 @@ struct KSet {
   void (*mfma_ad_rr2_7)(const int*, const int*, const S*, const S*, const S*, const S*, const S*,
                         S*, S*, double*, int, int, int, double, double, double, double, double,
                         double, int) = nullptr;
+  // the backward steps reading alpha_{m-1} from the forward table (signature of
+  // ad_stored): general (D fused on H's pattern, or not), row-resident for
+  // rows of at most 8 and 7 blocks, FP32 on pairs of column tiles
+  void (*mfma_ads[6])(const int*, const int*, const S*, const S*, const S*, const S*, const S*,
+                      const S*, S*, double*, int, int, int, double, double, double, double, double,
+                      double, int) = {};
   int B = 0, L = 0, KQ = 0;
 };
+
+// Entries of mfma_ads.
+enum MfmaAds { ADS_FUSED = 0, ADS_PLAIN = 1, ADS_RR = 2, ADS_RR7 = 3, ADS_RR2 = 4, ADS_RR2_7 = 5 };
 
 // Geometries compiled for each block size (lanes per group, packets per lane).
 struct GeomChoice {

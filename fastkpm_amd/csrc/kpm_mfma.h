@@ -622,7 +622,7 @@ constexpr int mf_rr_group() {
 // and a vector spans less than 4 GiB): A operands and neighbour offsets once
 // per row, buffer loads in the tile loop.
 // ---------------------------------------------------------------------------
-template <typename S, bool FUSED_D, int DM = MF_DM, int GR = 2>
+template <typename S, bool FUSED_D, bool STORED, int DM = MF_DM, int GR = 2>
 __device__ __forceinline__ void mfma_autodiff_rr_dev(
     WgId wid, const int* __restrict__ rp, const int* __restrict__ ci, const S* __restrict__ hv,
     const S* __restrict__ am, const S* __restrict__ am1, const S* __restrict__ bm1,
@@ -716,8 +716,10 @@ __device__ __forceinline__ void mfma_autodiff_rr_dev(
         for (int v = 0; v < GR; v++) {
           if (u0 + v >= DM) continue;  // DM % GR != 0: the last group is short
           const uint32_t sb_ = sj[u0 + v] + so;
-          xa0[v] = IO::ld(ba, vlo, sb_);
-          xa1[v] = IO::ld(ba, vlo, sb_ + half);
+          if constexpr (!STORED) {
+            xa0[v] = IO::ld(ba, vlo, sb_);
+            xa1[v] = IO::ld(ba, vlo, sb_ + half);
+          }
           xb0[v] = IO::ld(bb, vlo, sb_);
           xb1[v] = IO::ld(bb, vlo, sb_ + half);
           if constexpr (FUSED_D) {
@@ -731,7 +733,7 @@ __device__ __forceinline__ void mfma_autodiff_rr_dev(
           S au[4];
 #pragma unroll
           for (int q = 0; q < 4; q++) au[q] = la[u0 + v][lane][q];
-          accA = mfma_block<S>(au, xa0[v], xa1[v], accA);
+          if constexpr (!STORED) accA = mfma_block<S>(au, xa0[v], xa1[v], accA);
           accB = mfma_block<S>(au, xb0[v], xb1[v], accB);
           if constexpr (FUSED_D) {
             V4 gt = V4{S(0), S(0), S(0), S(0)};
@@ -750,17 +752,26 @@ __device__ __forceinline__ void mfma_autodiff_rr_dev(
       const S a1[4] = {a10.x, a10.y, a11.x, a11.y};
       const S b2[4] = {asb2 * b20.x, asb2 * b20.y, asb2 * b21.x, asb2 * b21.y};
       S an[4], bo[4];
+      if constexpr (STORED) {  // alpha_{m-1} from the table
+        const C2 an0 = IO::ld(bao, vlo, si + so), an1 = IO::ld(bao, vlo, si + so + half);
+        an[0] = an0.x;
+        an[1] = an0.y;
+        an[2] = an1.x;
+        an[3] = an1.y;
+      }
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        an[e] = fma(a2, hx[e], -a1[e]);
+        if constexpr (!STORED) an[e] = fma(a2, hx[e], -a1[e]);
         S v = fma(ab2, hb[e], -b2[e]);
         v = fma(ac4, ai[e], v);
         v = fma(ac2, a1[e], v);
         v = fma(aw, an[e], v);
         bo[e] = v;
       }
-      IO::st(C2{an[0], an[1]}, bao, vlo, si + so);
-      IO::st(C2{an[2], an[3]}, bao, vlo, si + so + half);
+      if constexpr (!STORED) {
+        IO::st(C2{an[0], an[1]}, bao, vlo, si + so);
+        IO::st(C2{an[2], an[3]}, bao, vlo, si + so + half);
+      }
       IO::st(C2{bo[0], bo[1]}, bbo, vlo, si + so);
       IO::st(C2{bo[2], bo[3]}, bbo, vlo, si + so + half);
     }
@@ -787,7 +798,7 @@ __device__ __forceinline__ void mfma_autodiff_rr_dev(
 // 1654 us per step).
 constexpr int MF_RR2_GROUP = 2;
 
-template <int DM, int GR>
+template <bool STORED, int DM, int GR>
 __device__ __forceinline__ void mfma_autodiff_rr2_dev(
     WgId wid, const int* __restrict__ rp, const int* __restrict__ ci,
     const float* __restrict__ hv, const float* __restrict__ am, const float* __restrict__ am1,
@@ -877,8 +888,10 @@ __device__ __forceinline__ void mfma_autodiff_rr2_dev(
         for (int v = 0; v < GR; v++) {
           if (u0 + v >= DM) continue;  // DM % GR != 0: the last group is short
           const uint32_t sb_ = sj[u0 + v] + so;
-          xa0[v] = fkd_raw_ld_f32x4(ba, (int)vlo, (int)sb_, 0);
-          xa1[v] = fkd_raw_ld_f32x4(ba, (int)vlo, (int)(sb_ + half), 0);
+          if constexpr (!STORED) {
+            xa0[v] = fkd_raw_ld_f32x4(ba, (int)vlo, (int)sb_, 0);
+            xa1[v] = fkd_raw_ld_f32x4(ba, (int)vlo, (int)(sb_ + half), 0);
+          }
           xb0[v] = fkd_raw_ld_f32x4(bb, (int)vlo, (int)sb_, 0);
           xb1[v] = fkd_raw_ld_f32x4(bb, (int)vlo, (int)(sb_ + half), 0);
 #pragma unroll
@@ -893,8 +906,10 @@ __device__ __forceinline__ void mfma_autodiff_rr2_dev(
           S au[4];
 #pragma unroll
           for (int q = 0; q < 4; q++) au[q] = la[u0 + v][lane][q];
-          accAe = mfma_block<S>(au, C2{xa0[v].x, xa0[v].y}, C2{xa1[v].x, xa1[v].y}, accAe);
-          accAo = mfma_block<S>(au, C2{xa0[v].z, xa0[v].w}, C2{xa1[v].z, xa1[v].w}, accAo);
+          if constexpr (!STORED) {
+            accAe = mfma_block<S>(au, C2{xa0[v].x, xa0[v].y}, C2{xa1[v].x, xa1[v].y}, accAe);
+            accAo = mfma_block<S>(au, C2{xa0[v].z, xa0[v].w}, C2{xa1[v].z, xa1[v].w}, accAo);
+          }
           accBe = mfma_block<S>(au, C2{xb0[v].x, xb0[v].y}, C2{xb1[v].x, xb1[v].y}, accBe);
           accBo = mfma_block<S>(au, C2{xb0[v].z, xb0[v].w}, C2{xb1[v].z, xb1[v].w}, accBo);
           V4 gt = V4{0.f, 0.f, 0.f, 0.f};
@@ -921,20 +936,34 @@ __device__ __forceinline__ void mfma_autodiff_rr2_dev(
       const S a1[2][4] = {{a10.x, a10.y, a11.x, a11.y}, {a10.z, a10.w, a11.z, a11.w}};
       const S b2[2][4] = {{b20.x, b20.y, b21.x, b21.y}, {b20.z, b20.w, b21.z, b21.w}};
       S an[2][4], bo[2][4];
+      if constexpr (STORED) {  // alpha_{m-1} from the table
+        const bf32x4 n0 = fkd_raw_ld_f32x4(bao, (int)vlo, (int)(si + so), 0);
+        const bf32x4 n1 = fkd_raw_ld_f32x4(bao, (int)vlo, (int)(si + so + half), 0);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          an[h][0] = n0[2 * h];
+          an[h][1] = n0[2 * h + 1];
+          an[h][2] = n1[2 * h];
+          an[h][3] = n1[2 * h + 1];
+        }
+      }
 #pragma unroll
       for (int h = 0; h < 2; h++)
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          an[h][e] = fma(a2, hx[h][e], -a1[h][e]);
+          if constexpr (!STORED) an[h][e] = fma(a2, hx[h][e], -a1[h][e]);
           S v = fma(ab2, hb[h][e], -(asb2 * b2[h][e]));
           v = fma(ac4, ai[h][e], v);
           v = fma(ac2, a1[h][e], v);
           v = fma(aw, an[h][e], v);
           bo[h][e] = v;
         }
-      fkd_raw_st_f32x4(bf32x4{an[0][0], an[0][1], an[1][0], an[1][1]}, bao, (int)vlo, (int)(si + so), 0);
-      fkd_raw_st_f32x4(bf32x4{an[0][2], an[0][3], an[1][2], an[1][3]}, bao, (int)vlo,
-                       (int)(si + so + half), 0);
+      if constexpr (!STORED) {
+        fkd_raw_st_f32x4(bf32x4{an[0][0], an[0][1], an[1][0], an[1][1]}, bao, (int)vlo,
+                         (int)(si + so), 0);
+        fkd_raw_st_f32x4(bf32x4{an[0][2], an[0][3], an[1][2], an[1][3]}, bao, (int)vlo,
+                         (int)(si + so + half), 0);
+      }
       fkd_raw_st_f32x4(bf32x4{bo[0][0], bo[0][1], bo[1][0], bo[1][1]}, bbo, (int)vlo, (int)(si + so), 0);
       fkd_raw_st_f32x4(bf32x4{bo[0][2], bo[0][3], bo[1][2], bo[1][3]}, bbo, (int)vlo,
                        (int)(si + so + half), 0);
@@ -963,7 +992,7 @@ constexpr int MF_DMAX = 8;
 // tiles; between passes the partial products Hs alpha_m, Hs beta_{m+1} are
 // parked in a_out / b_out, which only this wave touches.
 // ---------------------------------------------------------------------------
-template <typename S, bool FUSED_D>
+template <typename S, bool FUSED_D, bool STORED = false>
 __device__ __forceinline__ void mfma_autodiff_dev(
     WgId wid,
     const int* __restrict__ rp, const int* __restrict__ ci, const S* __restrict__ hv,
@@ -1007,9 +1036,11 @@ __device__ __forceinline__ void mfma_autodiff_dev(
         const size_t f0 = o0 + co, f1 = o1 + co;
         V4 accA = V4{S(0), S(0), S(0), S(0)}, accB = accA;
         if (!first) {  // partial products parked by the previous pass
-          const C2 pa0 = ldc<S>(a_out + f0), pa1 = ldc<S>(a_out + f1);
+          if constexpr (!STORED) {
+            const C2 pa0 = ldc<S>(a_out + f0), pa1 = ldc<S>(a_out + f1);
+            accA = V4{pa0.x, pa0.y, pa1.x, pa1.y};
+          }
           const C2 pb0 = ldc<S>(b_out + f0), pb1 = ldc<S>(b_out + f1);
-          accA = V4{pa0.x, pa0.y, pa1.x, pa1.y};
           accB = V4{pb0.x, pb0.y, pb1.x, pb1.y};
         }
         S pv[4];
@@ -1030,8 +1061,10 @@ __device__ __forceinline__ void mfma_autodiff_dev(
               const int j = ci[p];
               mfma_a_of<S>(mfma_hraw<S>(hv + (size_t)p * 128, m), m, S(1), a[v]);
               const size_t r0 = (size_t)(8 * j + m.q) * rs + co, r1 = (size_t)(8 * j + 4 + m.q) * rs + co;
-              xa0[v] = ldc<S>(am + r0);
-              xa1[v] = ldc<S>(am + r1);
+              if constexpr (!STORED) {
+                xa0[v] = ldc<S>(am + r0);
+                xa1[v] = ldc<S>(am + r1);
+              }
               xb0[v] = ldc<S>(xb + r0);
               xb1[v] = ldc<S>(xb + r1);
               if constexpr (FUSED_D) {
@@ -1051,7 +1084,7 @@ __device__ __forceinline__ void mfma_autodiff_dev(
 #pragma unroll
           for (int v = 0; v < 2; v++) {
             if (pc + u0 + v >= pe) continue;
-            accA = mfma_block<S>(a[v], xa0[v], xa1[v], accA);
+            if constexpr (!STORED) accA = mfma_block<S>(a[v], xa0[v], xa1[v], accA);
             accB = mfma_block<S>(a[v], xb0[v], xb1[v], accB);
             if constexpr (FUSED_D) {
               V4 gt = V4{S(0), S(0), S(0), S(0)};
@@ -1062,8 +1095,10 @@ __device__ __forceinline__ void mfma_autodiff_dev(
           }
         }
         if (!last) {
-          stc<S>(a_out + f0, C2{accA.x, accA.y});
-          stc<S>(a_out + f1, C2{accA.z, accA.w});
+          if constexpr (!STORED) {
+            stc<S>(a_out + f0, C2{accA.x, accA.y});
+            stc<S>(a_out + f1, C2{accA.z, accA.w});
+          }
           stc<S>(b_out + f0, C2{accB.x, accB.y});
           stc<S>(b_out + f1, C2{accB.z, accB.w});
           continue;
@@ -1084,17 +1119,26 @@ __device__ __forceinline__ void mfma_autodiff_dev(
         const S a1[4] = {a10.x, a10.y, a11.x, a11.y};
         const S b2[4] = {b20.x, b20.y, b21.x, b21.y};
         S an[4], bo[4];
+        if constexpr (STORED) {  // alpha_{m-1} from the table
+          const C2 an0 = ldc<S>(a_out + f0), an1 = ldc<S>(a_out + f1);
+          an[0] = an0.x;
+          an[1] = an0.y;
+          an[2] = an1.x;
+          an[3] = an1.y;
+        }
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          an[e] = fma(a2, hx[e], -a1[e]);
+          if constexpr (!STORED) an[e] = fma(a2, hx[e], -a1[e]);
           S v = fma(ab2, hb[e], -b2[e]);
           v = fma(ac4, ai[e], v);
           v = fma(ac2, a1[e], v);
           v = fma(aw, an[e], v);
           bo[e] = v;
         }
-        stc<S>(a_out + f0, C2{an[0], an[1]});
-        stc<S>(a_out + f1, C2{an[2], an[3]});
+        if constexpr (!STORED) {
+          stc<S>(a_out + f0, C2{an[0], an[1]});
+          stc<S>(a_out + f1, C2{an[2], an[3]});
+        }
         stc<S>(b_out + f0, C2{bo[0], bo[1]});
         stc<S>(b_out + f1, C2{bo[2], bo[3]});
       }
@@ -1183,7 +1227,7 @@ __global__ __launch_bounds__(WG) void k_mfma_autodiff_rr(
     const S* __restrict__ bm2, S* __restrict__ a_out, S* __restrict__ b_out,
     double* __restrict__ dacc, int nb, int qp, int chunk, double c4, double c2, double w,
     double sb, double sb2, double dscale, int nt) {
-  mfma_autodiff_rr_dev<S, true, DM, mf_rr_group<S, DM>()>(wg_self(), rp, ci, hv, am, am1, bm1, bm2,
+  mfma_autodiff_rr_dev<S, true, false, DM, mf_rr_group<S, DM>()>(wg_self(), rp, ci, hv, am, am1, bm1, bm2,
                                                          a_out, b_out, dacc, nb, qp, chunk, c4, c2,
                                                          w, sb, sb2, dscale, nt);
 }
@@ -1211,8 +1255,49 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(3))) void k_
     double* __restrict__ dacc, int nb, int qp, int chunk, double c4, double c2, double w,
     double sb, double sb2, double dscale, int nt) {
   (void)nt;
-  mfma_autodiff_rr2_dev<DM, GR>(wg_self(), rp, ci, hv, am, am1, bm1, bm2, a_out, b_out, dacc, nb,
+  mfma_autodiff_rr2_dev<false, DM, GR>(wg_self(), rp, ci, hv, am, am1, bm1, bm2, a_out, b_out, dacc, nb,
                                 qp, chunk, c4, c2, w, sb, sb2, dscale);
+}
+
+// The same three steps with the forward vectors kept (k_step_autodiff_stored):
+// alpha_{m-1} is read from the table, so a step gathers beta_{m+1} only and has
+// one block product and the outer product per neighbour instead of two and the
+// outer product (8 matrix-core instructions a tile, not 12).
+template <typename S, bool FUSED_D>
+__global__ __launch_bounds__(WG) void k_mfma_autodiff_stored(
+    const int* __restrict__ rp, const int* __restrict__ ci, const S* __restrict__ hv,
+    const S* __restrict__ am, const S* __restrict__ am1, const S* __restrict__ bm1,
+    const S* __restrict__ bm2, const S* __restrict__ amm, S* __restrict__ b_out,
+    double* __restrict__ dacc, int nb, int qp, int chunk, double c4, double c2, double w,
+    double sb, double sb2, double dscale, int nt) {
+  mfma_autodiff_dev<S, FUSED_D, true>(wg_self(), rp, ci, hv, am, am1, bm1, bm2,
+                                      const_cast<S*>(amm), b_out, dacc, nb, qp, chunk, c4, c2, w,
+                                      sb, sb2, dscale, nt);
+}
+
+template <typename S, int DM>
+__global__ __launch_bounds__(WG) void k_mfma_autodiff_rr_stored(
+    const int* __restrict__ rp, const int* __restrict__ ci, const S* __restrict__ hv,
+    const S* __restrict__ am, const S* __restrict__ am1, const S* __restrict__ bm1,
+    const S* __restrict__ bm2, const S* __restrict__ amm, S* __restrict__ b_out,
+    double* __restrict__ dacc, int nb, int qp, int chunk, double c4, double c2, double w,
+    double sb, double sb2, double dscale, int nt) {
+  mfma_autodiff_rr_dev<S, true, true, DM, mf_rr_group<S, DM>()>(
+      wg_self(), rp, ci, hv, am, am1, bm1, bm2, const_cast<S*>(amm), b_out, dacc, nb, qp, chunk, c4,
+      c2, w, sb, sb2, dscale, nt);
+}
+
+template <int DM, int GR>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(3))) void k_mfma_autodiff_rr2_stored(
+    const int* __restrict__ rp, const int* __restrict__ ci, const float* __restrict__ hv,
+    const float* __restrict__ am, const float* __restrict__ am1, const float* __restrict__ bm1,
+    const float* __restrict__ bm2, const float* __restrict__ amm, float* __restrict__ b_out,
+    double* __restrict__ dacc, int nb, int qp, int chunk, double c4, double c2, double w,
+    double sb, double sb2, double dscale, int nt) {
+  (void)nt;
+  mfma_autodiff_rr2_dev<true, DM, GR>(wg_self(), rp, ci, hv, am, am1, bm1, bm2,
+                                      const_cast<float*>(amm), b_out, dacc, nb, qp, chunk, c4, c2,
+                                      w, sb, sb2, dscale);
 }
 
 }  // namespace fkd

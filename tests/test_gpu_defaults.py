@@ -79,3 +79,47 @@ def test_fused_4x4_outer_product(oracle, lanes, kq, store):
         eng.set_geometry(lanes, kq, 0)
         eng.set_store_alpha(store)
     _run(oracle, H, 11, before=force).close()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("rows", [7, 8, "long"])
+@pytest.mark.parametrize("S", [3, 16, 40, 64])
+def test_matrix_core_backward_step_from_the_table(oracle, rows, S, prec):
+    """8x8 blocks with the forward vectors kept: row-resident steps on 7 and 8
+    block slots and the general step on longer rows, one and two column tiles,
+    D on H's pattern and on the diagonal, stoch_matrix from the table."""
+    from fastkpm_amd import EnergyScale, HipEngine, lattice
+    from helpers import with_partner_bonds
+    from test_gpu_resident import _random_H
+    if rows == "long":
+        H, bound = _random_H(40, 8, 9, False, seed=S)
+        assert np.diff(H.row_ptr).max() > 8
+    else:
+        H = lattice.lattice((4, 3, 3), b=8, orbital_blocks=True, seed=S)
+        if rows == 8:
+            H = with_partner_bonds(H, (4, 3, 3), seed=S)
+        bound = float(np.abs(np.linalg.eigvalsh(H.to_dense())).max()) * 1.01
+        assert np.diff(H.row_ptr).max() == rows
+    rng = np.random.default_rng(S)
+    R = rng.standard_normal((H.n_rows * 8, S)) + 1j * rng.standard_normal((H.n_rows * 8, S))
+    nb = H.n_rows
+    Dd = lattice.coo_to_bsr(nb, 8, np.arange(nb), np.arange(nb), np.zeros((nb, 8, 8)))
+    M = 14
+    c = 1.0 / (1.0 + np.arange(M))
+    eng = HipEngine("cx_double", prec)
+    eng.set_store_alpha(2)
+    eng.set_R(R)
+    eng.set_H(H, EnergyScale(-bound, bound))
+    orc = oracle.Engine()
+    orc.set_H(H, -bound, bound)
+    orc.set_R(R)
+    tol = 1e-10 if prec == "fp64" else M * 16 * 2.0 ** -24
+    for D in (H.like(), Dd):
+        assert rel_err(eng.moments(M), orc.moments(M)) < tol
+        assert eng.alpha_table() and eng.kernel_config(5)["mfma"]
+        eng.autodiff_matrix(c, D)
+        assert rel_err(D.val, orc.autodiff_matrix(c, D)) < tol
+    eng.stoch_matrix(c, D)
+    assert eng.stoch_method() == "table"
+    assert rel_err(D.val, orc.stoch_matrix(c, D)) < tol
+    eng.close()
