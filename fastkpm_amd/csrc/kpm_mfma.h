@@ -616,6 +616,61 @@ constexpr int mf_rr_group() {
   return sizeof(S) == 8 && DM == 7 ? 4 : 2;
 }
 
+// The D operands of a tile.  G = P Q^T contracts over columns, so its operands
+// hold rows (orbital and part) along the lanes and columns along the lane
+// groups: lane (q, r) needs row r of columns 4 NC q .. 4 NC q + 4 NC - 1, the
+// transpose of the layout the block products gather (lane (q, c): orbitals q, q + 4
+// of columns NC c .. NC c + NC - 1).  Loading it from memory put the 16 rows of an
+// instruction on 16 lines (64 cache accesses an instruction, 131 of the 181 us of
+// the FP64 backward step at 18x15x13 x 8, S = 144); instead the gathered
+// registers pass through the wave's own slice of LDS, re and im rows apart, a
+// row padded by 16 bytes so that the 16 rows of a read fall on different banks.
+template <typename S, int NC>
+struct MfmaT {
+  static constexpr int ROW = 16 * NC + 16 / (int)sizeof(S);
+  static constexpr int SIZE = 16 * ROW;  // scalars of one wave's slice
+  typedef S VW __attribute__((ext_vector_type(2)));
+
+  // this lane's columns of orbital q (x0) and q + 4 (x1), (re, im) each
+  static __device__ __forceinline__ void put(S* buf, const MfmaLane& m, const S (&x0)[2 * NC],
+                                             const S (&x1)[2 * NC]) {
+#pragma unroll
+    for (int part = 0; part < 2; part++) {
+      S* r0 = buf + (8 * part + m.q) * ROW + NC * m.c;
+      S* r1 = r0 + 4 * ROW;
+      if constexpr (NC == 2) {
+        *reinterpret_cast<VW*>(r0) = VW{x0[part], x0[2 + part]};
+        *reinterpret_cast<VW*>(r1) = VW{x1[part], x1[2 + part]};
+      } else {
+        r0[0] = x0[part];
+        r1[0] = x1[part];
+      }
+    }
+  }
+
+  static __device__ __forceinline__ void get(const S* buf, const MfmaLane& m, S (&v)[4 * NC]) {
+    constexpr int N = 16 / (int)sizeof(S);
+    typedef typename Vec16<S>::V V;
+    const S* r = buf + m.c * ROW + 4 * NC * m.q;
+#pragma unroll
+    for (int k = 0; k < 4 * NC / N; k++) {
+      const V t = *reinterpret_cast<const V*>(r + k * N);
+#pragma unroll
+      for (int e = 0; e < N; e++) v[k * N + e] = t[e];
+    }
+  }
+
+  // One operand through the wave's slice: the LDS serves a wave's accesses in
+  // order, so the fences only keep the compiler from reordering them.
+  static __device__ __forceinline__ void pass(S* buf, const MfmaLane& m, const S (&x0)[2 * NC],
+                                              const S (&x1)[2 * NC], S (&v)[4 * NC]) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    put(buf, m, x0, x1);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    get(buf, m, v);
+  }
+};
+
 // ---------------------------------------------------------------------------
 // Row-resident autodiff step for rows of at most DM blocks (same contract as
 // mfma_autodiff_dev; the host uses it when every row has at most DM blocks
@@ -652,7 +707,6 @@ __device__ __forceinline__ void mfma_autodiff_rr_dev(
   const S a2 = (S)2, ab2 = (S)(2.0 * hb1), ac4 = (S)c4, ac2 = (S)c2, aw = (S)w;
   const S asb2 = bm2 != nullptr ? S(1) : (S)sb2;  // beta_{m+2} = asb2 * (bm2 or alpha_{m+1})
   const double fD = dscale * hb1;
-  const int dorb = m.c & 7, dpart = m.c >> 3;
   const uint32_t half = 4u * rs * ES;
 
   // This wave's slice of LDS holds the row's A operands across the tile loop
@@ -661,8 +715,10 @@ __device__ __forceinline__ void mfma_autodiff_rr_dev(
   // buffer load's SGPR offset): the registers go to loads in flight instead.
   __shared__ S lds_a[WG / WAVE][DM][WAVE][4];
   const int lane = threadIdx.x & (WAVE - 1);
-  const uint32_t vlo = (m.q * rs + 2u * m.c) * ES;                    // MFMA operand layout
-  const uint32_t vld = (dorb * rs + (uint32_t)dpart + 2u * m.q) * ES;  // D layout
+  const uint32_t vlo = (m.q * rs + 2u * m.c) * ES;
+  using TR = MfmaT<S, 1>;
+  __shared__ __attribute__((aligned(16))) S lds_t[WG / WAVE][TR::SIZE];
+  S* const lt = lds_t[g];
   S (&la)[DM][WAVE][4] = lds_a[g];
 
   for (int base = rr.r0; base < rr.r1; base += rr.stride) {
@@ -703,15 +759,11 @@ __device__ __forceinline__ void mfma_autodiff_rr_dev(
     for (int t = 0; t < ntile; t++) {
       const uint32_t so = (uint32_t)t * 32u * ES;
       V4 accA = V4{S(0), S(0), S(0), S(0)}, accB = accA;
+      const C2 ai0 = IO::ld(ba, vlo, si + so), ai1 = IO::ld(ba, vlo, si + so + half);
       S pv[4];
-      if constexpr (FUSED_D) {
-#pragma unroll
-        for (int k = 0; k < 4; k++) pv[k] = IO::ld1(ba, vld + 8u * k * ES, si + so);
-      }
 #pragma unroll
       for (int u0 = 0; u0 < DM; u0 += GR) {
         C2 xa0[GR], xa1[GR], xb0[GR], xb1[GR];
-        S qv[GR][4];
 #pragma unroll
         for (int v = 0; v < GR; v++) {
           if (u0 + v >= DM) continue;  // DM % GR != 0: the last group is short
@@ -722,14 +774,15 @@ __device__ __forceinline__ void mfma_autodiff_rr_dev(
           }
           xb0[v] = IO::ld(bb, vlo, sb_);
           xb1[v] = IO::ld(bb, vlo, sb_ + half);
-          if constexpr (FUSED_D) {
-#pragma unroll
-            for (int k = 0; k < 4; k++) qv[v][k] = IO::ld1(bb, vld + 8u * k * ES, sb_);
-          }
+        }
+        if constexpr (FUSED_D) {
+          if (u0 == 0) TR::pass(lt, m, {ai0.x, ai0.y}, {ai1.x, ai1.y}, pv);
         }
 #pragma unroll
         for (int v = 0; v < GR; v++) {
           if (u0 + v >= DM) continue;
+          S qv[4];
+          if constexpr (FUSED_D) TR::pass(lt, m, {xb0[v].x, xb0[v].y}, {xb1[v].x, xb1[v].y}, qv);
           S au[4];
 #pragma unroll
           for (int q = 0; q < 4; q++) au[q] = la[u0 + v][lane][q];
@@ -738,12 +791,11 @@ __device__ __forceinline__ void mfma_autodiff_rr_dev(
           if constexpr (FUSED_D) {
             V4 gt = V4{S(0), S(0), S(0), S(0)};
 #pragma unroll
-            for (int k = 0; k < 4; k++) gt = MF::mac(pv[k], qv[v][k], gt);
+            for (int k = 0; k < 4; k++) gt = MF::mac(pv[k], qv[k], gt);
             G[u0 + v] += dv4{(double)gt.x, (double)gt.y, (double)gt.z, (double)gt.w};
           }
         }
       }
-      const C2 ai0 = IO::ld(ba, vlo, si + so), ai1 = IO::ld(ba, vlo, si + so + half);
       const C2 a10 = IO::ld(ba1, vlo, si + so), a11 = IO::ld(ba1, vlo, si + so + half);
       const C2 b20 = IO::ld(bb2, vlo, si + so), b21 = IO::ld(bb2, vlo, si + so + half);
       const S hx[4] = {accA.x, accA.y, accA.z, accA.w};
@@ -809,7 +861,6 @@ __device__ __forceinline__ void mfma_autodiff_rr2_dev(
   using C2 = Mfma<float>::c2;
   using V4 = Mfma<float>::v4;
   using MF = Mfma<float>;
-  using IO = BufC2<float>;
   constexpr int NS = Vec16<S>::N;
   constexpr uint32_t ES = sizeof(S);
   const MfmaLane m = mfma_lane<S>();
@@ -828,14 +879,14 @@ __device__ __forceinline__ void mfma_autodiff_rr2_dev(
   const S a2 = 2.0f, ab2 = (S)(2.0 * hb1), ac4 = (S)c4, ac2 = (S)c2, aw = (S)w;
   const S asb2 = bm2 != nullptr ? 1.0f : (S)sb2;  // beta_{m+2} = asb2 * (bm2 or alpha_{m+1})
   const double fD = dscale * hb1;
-  const int dorb = m.c & 7, dpart = m.c >> 3;
   const uint32_t half = 4u * rs * ES;
 
   __shared__ S lds_a[WG / WAVE][DM][WAVE][4];
   const int lane = threadIdx.x & (WAVE - 1);
   const uint32_t vlo = (m.q * rs + 4u * m.c) * ES;  // columns 2c, 2c + 1 of orbital q
-  // D operand of column 2n + h, n = 4k + q: scalar 4n + 2h + dpart of orbital dorb
-  const uint32_t vld = (dorb * rs + 4u * m.q + (uint32_t)dpart) * ES;
+  using TR = MfmaT<float, 2>;
+  __shared__ __attribute__((aligned(16))) float lds_t[WG / WAVE][TR::SIZE];
+  float* const lt = lds_t[g];
   S (&la)[DM][WAVE][4] = lds_a[g];
 
   for (int base = rr.r0; base < rr.r1; base += rr.stride) {
@@ -875,15 +926,12 @@ __device__ __forceinline__ void mfma_autodiff_rr2_dev(
     for (int t = 0; t < npair; t++) {
       const uint32_t so = (uint32_t)t * 64u * ES;
       V4 accAe = V4{0.f, 0.f, 0.f, 0.f}, accAo = accAe, accBe = accAe, accBo = accAe;
-      S pv[4][2];
-#pragma unroll
-      for (int k = 0; k < 4; k++)
-#pragma unroll
-        for (int h = 0; h < 2; h++) pv[k][h] = IO::ld1(ba, vld + (16u * k + 2u * h) * ES, si + so);
+      const bf32x4 ai0 = fkd_raw_ld_f32x4(ba, (int)vlo, (int)(si + so), 0);
+      const bf32x4 ai1 = fkd_raw_ld_f32x4(ba, (int)vlo, (int)(si + so + half), 0);
+      S pv[8];
 #pragma unroll
       for (int u0 = 0; u0 < DM; u0 += GR) {
         bf32x4 xa0[GR], xa1[GR], xb0[GR], xb1[GR];
-        S qv[GR][4][2];
 #pragma unroll
         for (int v = 0; v < GR; v++) {
           if (u0 + v >= DM) continue;  // DM % GR != 0: the last group is short
@@ -894,15 +942,16 @@ __device__ __forceinline__ void mfma_autodiff_rr2_dev(
           }
           xb0[v] = fkd_raw_ld_f32x4(bb, (int)vlo, (int)sb_, 0);
           xb1[v] = fkd_raw_ld_f32x4(bb, (int)vlo, (int)(sb_ + half), 0);
-#pragma unroll
-          for (int k = 0; k < 4; k++)
-#pragma unroll
-            for (int h = 0; h < 2; h++) qv[v][k][h] = IO::ld1(bb, vld + (16u * k + 2u * h) * ES, sb_);
         }
         __builtin_amdgcn_sched_barrier(0);  // the group's loads all issued before its products
+        if (u0 == 0)
+          TR::pass(lt, m, {ai0.x, ai0.y, ai0.z, ai0.w}, {ai1.x, ai1.y, ai1.z, ai1.w}, pv);
 #pragma unroll
         for (int v = 0; v < GR; v++) {
           if (u0 + v >= DM) continue;
+          S qv[8];
+          TR::pass(lt, m, {xb0[v].x, xb0[v].y, xb0[v].z, xb0[v].w},
+                   {xb1[v].x, xb1[v].y, xb1[v].z, xb1[v].w}, qv);
           S au[4];
 #pragma unroll
           for (int q = 0; q < 4; q++) au[q] = la[u0 + v][lane][q];
@@ -914,17 +963,13 @@ __device__ __forceinline__ void mfma_autodiff_rr2_dev(
           accBo = mfma_block<S>(au, C2{xb0[v].z, xb0[v].w}, C2{xb1[v].z, xb1[v].w}, accBo);
           V4 gt = V4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int k = 0; k < 4; k++)
-#pragma unroll
-            for (int h = 0; h < 2; h++) gt = MF::mac(pv[k][h], qv[v][k][h], gt);
+          for (int k = 0; k < 8; k++) gt = MF::mac(pv[k], qv[k], gt);
           G[u0 + v] += dv4{(double)gt.x, (double)gt.y, (double)gt.z, (double)gt.w};
         }
         // one group's operands live at a time (the scheduler would otherwise
         // hoist every group's loads and leave one wave per SIMD)
         __builtin_amdgcn_sched_barrier(0);
       }
-      const bf32x4 ai0 = fkd_raw_ld_f32x4(ba, (int)vlo, (int)(si + so), 0);
-      const bf32x4 ai1 = fkd_raw_ld_f32x4(ba, (int)vlo, (int)(si + so + half), 0);
       const bf32x4 a10 = fkd_raw_ld_f32x4(ba1, (int)vlo, (int)(si + so), 0);
       const bf32x4 a11 = fkd_raw_ld_f32x4(ba1, (int)vlo, (int)(si + so + half), 0);
       const bf32x4 b20 = fkd_raw_ld_f32x4(bb2, (int)vlo, (int)(si + so), 0);
@@ -1015,16 +1060,15 @@ __device__ __forceinline__ void mfma_autodiff_dev(
   const S* __restrict__ xb = vb1 ? am : bm1;  // gathered beta_{m+1} (or alpha_m, scaled by sb)
   const S a2 = (S)2, ab2 = (S)(2.0 * hb1), ac4 = (S)c4, ac2 = (S)c2, aw = (S)w, asb2 = (S)sb2;
   const double fD = dscale * hb1;
-  // D-operand layout: lane l holds row l % 16 (orbital c & 7, part c >> 3)
-  // of column 4 kappa + q of a tile
-  const int dorb = m.c & 7, dpart = m.c >> 3;
+  using TR = MfmaT<S, 1>;
+  __shared__ __attribute__((aligned(16))) S lds_t[WG / WAVE][FUSED_D ? TR::SIZE : 4];
+  S* const lt = lds_t[g];
 
   for (int base = rr.r0; base < rr.r1; base += rr.stride) {
     const int i = __builtin_amdgcn_readfirstlane(base + g);
     if (i >= rr.r1) continue;
     const int p0 = rp[i], p1 = rp[i + 1];
     const size_t o0 = (size_t)(8 * i + m.q) * rs, o1 = (size_t)(8 * i + 4 + m.q) * rs;
-    const size_t od = (size_t)(8 * i + dorb) * rs + dpart;
     for (int pc = p0; pc < p1 || pc == p0; pc += MF_DMAX) {
       const int pe = min(pc + MF_DMAX, p1);
       const bool first = (pc == p0), last = (pe == p1);
@@ -1044,16 +1088,13 @@ __device__ __forceinline__ void mfma_autodiff_dev(
           accB = V4{pb0.x, pb0.y, pb1.x, pb1.y};
         }
         S pv[4];
-        if constexpr (FUSED_D) {
-#pragma unroll
-          for (int k = 0; k < 4; k++) pv[k] = am[od + 2 * ((size_t)t * 16 + 4 * k + m.q)];
-        }
+        const C2 ai0 = ldc<S>(am + f0), ai1 = ldc<S>(am + f1);
+        if constexpr (FUSED_D) TR::pass(lt, m, {ai0.x, ai0.y}, {ai1.x, ai1.y}, pv);
 #pragma unroll
         for (int u0 = 0; u0 < MF_DMAX; u0 += 2) {
           if (pc + u0 >= pe) break;
           S a[2][4];
           C2 xa0[2], xa1[2], xb0[2], xb1[2];
-          S qv[2][4];
 #pragma unroll
           for (int v = 0; v < 2; v++) {
             const int p = pc + u0 + v;
@@ -1067,17 +1108,9 @@ __device__ __forceinline__ void mfma_autodiff_dev(
               }
               xb0[v] = ldc<S>(xb + r0);
               xb1[v] = ldc<S>(xb + r1);
-              if constexpr (FUSED_D) {
-                const size_t jd = (size_t)(8 * j + dorb) * rs + dpart;
-#pragma unroll
-                for (int k = 0; k < 4; k++) qv[v][k] = xb[jd + 2 * ((size_t)t * 16 + 4 * k + m.q)];
-              }
             } else {
 #pragma unroll
-              for (int k = 0; k < 4; k++) {
-                a[v][k] = S(0);
-                qv[v][k] = S(0);
-              }
+              for (int k = 0; k < 4; k++) a[v][k] = S(0);
               xa0[v] = xa1[v] = xb0[v] = xb1[v] = C2{S(0), S(0)};
             }
           }
@@ -1087,9 +1120,11 @@ __device__ __forceinline__ void mfma_autodiff_dev(
             if constexpr (!STORED) accA = mfma_block<S>(a[v], xa0[v], xa1[v], accA);
             accB = mfma_block<S>(a[v], xb0[v], xb1[v], accB);
             if constexpr (FUSED_D) {
+              S qv[4];
+              TR::pass(lt, m, {xb0[v].x, xb0[v].y}, {xb1[v].x, xb1[v].y}, qv);
               V4 gt = V4{S(0), S(0), S(0), S(0)};
 #pragma unroll
-              for (int k = 0; k < 4; k++) gt = MF::mac(pv[k], qv[v][k], gt);
+              for (int k = 0; k < 4; k++) gt = MF::mac(pv[k], qv[k], gt);
               G[u0 + v] += dv4{(double)gt.x, (double)gt.y, (double)gt.z, (double)gt.w};
             }
           }
@@ -1103,7 +1138,6 @@ __device__ __forceinline__ void mfma_autodiff_dev(
           stc<S>(b_out + f1, C2{accB.z, accB.w});
           continue;
         }
-        const C2 ai0 = ldc<S>(am + f0), ai1 = ldc<S>(am + f1);
         const C2 a10 = ldc<S>(am1 + f0), a11 = ldc<S>(am1 + f1);
         C2 b20, b21;
         if (bm2 != nullptr) {
