@@ -641,26 +641,33 @@ constexpr size_t kLlcBytes = (size_t)256 << 20;
 // Default geometry of a kernel kind when nothing is tuned: one pass of width
 // wmax.  From 64 packets on, whole waves per row (wave-uniform rows, scalar
 // offsets and H); below, two packets per lane, which keeps more loads in
-// flight per wave than twice the lanes.  Forward step (us), 64 x 1 / 16 x 4 /
-// 32 x 2 lanes x packets on 64: 256^2 x 2 FP64 81 / 98 / 110, 20^3 x 2 12.9 /
-// 14.9 / 16.2; 16 x 2 / 32 x 1 on 32: 256^2 x 2 FP32 37 / 47, 128^2 x 2 FP64
-// 14.4 / 18.1; 8 x 2 / 16 x 1 on 16: 31x29x27 real 7.2 / 10.6.  The backward
-// step reading the table takes 16 x 4 on 64 while its vectors stay in the
-// last-level cache (20^3 x 2: 23.4 against 26 us; 256^2 x 2: 171 against 165).
+// flight per wave than twice the lanes, where that leaves a workgroup for each
+// of the 256 CUs.  Forward step (us), 64 x 1 / 16 x 4 / 32 x 2 lanes x packets on 64:
+// 256^2 x 2 FP64 81 / 98 / 110, 20^3 x 2 12.9 / 14.9 / 16.2; 16 x 2 / 32 x 1 on
+// 32: 256^2 x 2 FP32 37 / 47, 128^2 x 2 FP64 14.4 / 18.1; 8 x 2 / 16 x 1 on 16:
+// 31x29x27 real 7.2 / 10.6, but 37x52 x 2 (61 / 121 workgroups) 8.4 / 7.9.  The
+// backward step reading the table takes four packets per lane while its vectors
+// stay in the last-level cache (16 x 4 / 64 x 1: 20^3 x 2 23.4 / 26, past it 256^2 x 2
+// 171 / 165; 8 x 4 / 16 x 2: 128^2 x 2 22.0 / 24.5).
 KCfg default_cfg(fkpm_handle* h, int kind) {
   static const int wide[] = {64, 32, 16, 8, 4};
-  static const int pairs[] = {16, 8, 32, 4, 64};
   static const int reduce[] = {16, 8, 32, 4, 64};
   // vectors a step touches; one that writes a fresh table slot meets the ones
   // of the steps before it in the cache too
   const int nvec = kind == K_AD || kind == K_ADS ? 6 : kind == K_XI || kind == K_MOMT ? 5 : 3;
   const bool cached = (size_t)nvec * h->vbytes() <= kLlcBytes;
-  const int* pref = kind == K_OUT || (kind == K_ADS && cached) ? reduce : h->wmax >= 64 ? wide : pairs;
   KCfg c;
-  if (pref == pairs && h->wmax >= 4 && compiled(h->b, h->wmax / 2, 2)) {
-    c.L = h->wmax / 2;
-    c.KQ = 2;
-  }
+  auto packets = [&](int kq) {
+    const int L = h->wmax / kq;
+    if (c.L > 0 || h->wmax % kq != 0 || !compiled(h->b, L, kq) ||
+        h->nb < 256 * (fkd::WG / fkd::WAVE) * (fkd::WAVE / L))
+      return;
+    c.L = L;
+    c.KQ = kq;
+  };
+  if (kind == K_ADS && cached) packets(4);
+  if (kind != K_OUT && h->wmax < 64) packets(2);
+  const int* pref = kind == K_OUT ? reduce : wide;
   for (int t = 0; t < 5 && c.L == 0; t++) {
     const int L = pref[t];
     if (h->wmax % L == 0 && compiled(h->b, L, h->wmax / L)) {
@@ -679,7 +686,11 @@ KCfg default_cfg(fkpm_handle* h, int kind) {
       }
     }
   }
-  c.maxwg = 16384;  // one pass over the rows at most sizes (256^2 x 2 FP64: 81 us, 4096: 87)
+  // One pass over the rows: with several, a workgroup's next rows lie far off and
+  // an XCD sweeps as many windows at once, each with its share of the L2 (FP64
+  // forward step 256^2 x 2: 81 us, 4096 workgroups 87; 64^3 x 2 in lattice row
+  // order: 687 us, 16384 workgroups 772; its autodiff step 1590 and 1690).
+  c.maxwg = 65536;
   c.nt = 0;
   // While a step's vectors stay in the last-level cache each XCD sweeps its own
   // region, whose neighbour rows its L2 then holds (128^2 x 2 FP64 forward step
@@ -689,6 +700,13 @@ KCfg default_cfg(fkpm_handle* h, int kind) {
   // 64 workgroups has no regions to speak of.
   const int gwg = (fkd::WG / fkd::WAVE) * (fkd::WAVE / (c.L > 0 ? c.L : fkd::WAVE));
   c.sweep = cached && h->nb / gwg >= 64 ? 0 : 2;
+  // The lattice row order where the vectors miss the cache and a tile plane of
+  // 128 sites (512 KB a vector) fills the L2 better than a plane of the lattice
+  // (64^3 x 2, S = 128 FP64: 687 against 762 us); with half the bytes a site the two
+  // sweeps measured the same (FP32: 377 and 366).
+  if (h->has_order && !cached && kind != K_OUT &&
+      h->vbytes() / (size_t)h->nb >= 4096)
+    c.nt |= fkd::NT_ORDER;
   if (mfma_avail(h, kind)) {
     c.mfma = 1;
     // row-resident: the forward step always, the autodiff step in FP64 and in
@@ -696,19 +714,21 @@ KCfg default_cfg(fkpm_handle* h, int kind) {
     if (mfma_rr_avail(h, kind) && (kind == K_MOM || kind == K_MOMT || !h->single ||
                                    h->qp % 16 == 0 || h->rr_force))
       c.mfma = 2;
+    // per XCD while three vectors stay in the last-level cache (forward step at
+    // 18x15x13 x 8 FP64, 65 MB vectors: 52 us, one front 65), else one front of
+    // single passes (32^3 x 8 FP32: 447, segments of two 466, per XCD 555)
+    if (h->nb / gwg >= 64) c.sweep = 3 * h->vbytes() <= kLlcBytes ? 0 : 1;
   }
   return c;
 }
 
-// Whether moments(M) keeps the forward vectors (when they fit): always with
-// FKPM_OPT_STORE_ALPHA 2; with 1 (automatic) when the three-vector ring
-// exceeds the 32 MB of L2: below that the forward steps lose more on the
-// table's write-back than the backward steps gain.  (Measured at C2, FP32:
-// forward step 35 -> 38 us on a table, autodiff 107 -> 91 us; FP64: 81 ->
-// 81 us, 191 -> 167 us.)
-bool table_wanted(const fkpm_handle* h) {
-  return h->store_alpha == 2 || (h->store_alpha == 1 && 3 * h->vbytes() > ((size_t)32 << 20));
-}
+// Whether moments(M) keeps the forward vectors (when they fit).  The backward
+// steps then gather one vector instead of two and stoch_matrix takes half the
+// steps; the forward step pays a write-back to a fresh slot.  M = 128, us per
+// call, ring / table: 60x40 x 2 FP64 set_H + moments + autodiff_matrix 1168 / 1101
+// and moments + autodiff_matrix + stoch_matrix 1827 / 1445; 140x120 x 1 1672 / 1667
+// and 2321 / 1921; 256^2 x 2 FP32 forward step 35 / 38, autodiff 107 / 91.
+bool table_wanted(const fkpm_handle* h) { return h->store_alpha != 0; }
 
 // Process-wide cache of tuned geometries, keyed by the problem shape.
 std::mutex g_tune_mu;
@@ -868,9 +888,16 @@ int ensure_ready(fkpm_handle* h) {
   return 0;
 }
 
+// Steps whose moment partials are held before they are reduced: 64 MiB of them
+// (a step of 65536 workgroups leaves 1 MiB).
+int partial_steps(int nsteps, int nwg) {
+  const size_t per = (size_t)nwg * 2 * sizeof(double);
+  return (int)std::min<size_t>(nsteps, std::max<size_t>(1, ((size_t)64 << 20) / per));
+}
+
 int ensure_partials(fkpm_handle* h, int nsteps) {
   const int nwg = std::max(h->kc[K_MOM].nwg, h->kc[K_MOMT].nwg);
-  CHK(h->partial.ensure((size_t)nsteps * nwg * 2 * sizeof(double)));
+  CHK(h->partial.ensure((size_t)partial_steps(nsteps, nwg) * nwg * 2 * sizeof(double)));
   CHK(h->psum.ensure((size_t)nsteps * 2 * sizeof(double)));
   return 0;
 }
@@ -896,7 +923,7 @@ int timing_end(fkpm_handle* h, double* ms, int* cnt, int launches) {
 
 // ---------------------------------------------------------------------------
 // Autotuner: times every compiled geometry of pass width wmax or wmax/2, three
-// workgroup caps and the nontemporal choice, per kernel kind, on the current
+// workgroup caps (where they differ) and the nontemporal choice, per kernel kind, on the current
 // H and R; keeps the fastest and caches it for this problem shape.
 // ---------------------------------------------------------------------------
 template <class S>
@@ -908,7 +935,7 @@ int tune_t(fkpm_handle* h) {
   CHK(h->Bv[0].ensure(vb));
   CHK(h->xi.ensure(h->accbytes()));
   CHK(h->tune_dacc.ensure((size_t)(h->nnzb > 0 ? h->nnzb : 1) * h->b * h->b * HS * sizeof(double)));
-  CHK(h->partial.ensure((size_t)(h->nb + 3) / 4 * 2 * sizeof(double) + 64));
+  CHK(h->partial.ensure(((size_t)(h->nb + 3) / 4 + 8 * 64) * 2 * sizeof(double)));
   const int* rp = h->rp.as<const int>();
   const int* ci = h->ci.as<const int>();
   const S* hv = h->hv.as<const S>();
@@ -937,7 +964,7 @@ int tune_t(fkpm_handle* h) {
   int step = 0;
   fkd::GeomChoice gs[64];
   const int ng = fkd::geometries_for_block(h->b, gs, 64);
-  static const int caps[] = {1024, 4096, 16384};
+  static const int caps[] = {4096, 16384, 65536};
   static const int nts[] = {0, fkd::NT_LOAD | fkd::NT_STORE};
   static const int sweeps[] = {0, 1, 2, 8};
   // The table kinds are timed on ns slots (at least 512 MB, more than the
@@ -1077,8 +1104,26 @@ int tune_t(fkpm_handle* h) {
                     reps > 6 ? " (final)" : "");
           return 0;
     };
+    // caps that give the same grid are one candidate
+    std::vector<KCfg> distinct;
+    for (KCfg c : cands) {
+      KCfg d = c;
+      if (d.mfma) {
+        d.L = 64;
+        d.KQ = 1;
+      }
+      derive_grid(h->nb, d);
+      bool seen = false;
+      for (const KCfg& o : distinct)
+        seen |= o.L == c.L && o.KQ == c.KQ && o.nt == c.nt && o.mfma == c.mfma &&
+                o.sweep == c.sweep && o.nwg == d.nwg && o.chunk == d.chunk;
+      if (seen) continue;
+      c.nwg = d.nwg;
+      c.chunk = d.chunk;
+      distinct.push_back(c);
+    }
     std::vector<std::pair<float, KCfg>> timed;
-    for (const KCfg& c : cands) {
+    for (const KCfg& c : distinct) {
       float us = 0.f;
       CHK(time_cfg(c, 6, &us));
       timed.push_back({us, h->kc[kind]});
@@ -1402,6 +1447,7 @@ int moments_t(fkpm_handle* h, int M, double* mu) {
   CHK(timing_begin(h));
   {
     LoopRecorder rec(h);
+    const int group = partial_steps(nsteps, kc.nwg);
     for (int m = 0; m < nsteps; m++) {
       // alpha_{m+1} = cx Hs alpha_m + cz alpha_{m-1}
       const S* x = (const S*)h->vec_a(m);
@@ -1410,10 +1456,14 @@ int moments_t(fkpm_handle* h, int M, double* mu) {
       CHK(launch(mom_fn(h, ks, kc), grid, block, h->stream, rp_for(h, kc),
                  h->ci.as<const int>(), h->hv.as<const S>(), x, z, y, h->nb, h->qp, kc.chunk,
                  m == 0 ? 1.0 : 2.0, m == 0 ? 0.0 : -1.0,
-                 h->partial.as<double>() + (size_t)m * kc.nwg * 2, kc.nt, no_rsource<S>()));
+                 h->partial.as<double>() + (size_t)(m % group) * kc.nwg * 2, kc.nt,
+                 no_rsource<S>()));
+      if ((m + 1) % group == 0 || m == nsteps - 1) {
+        const int m0 = m - m % group;
+        CHK(launch(&fkd::k_reduce_partials, dim3(m + 1 - m0), block, h->stream,
+                   (const double*)h->partial.as<double>(), kc.nwg, h->psum.as<double>() + 2 * m0));
+      }
     }
-    CHK(launch(&fkd::k_reduce_partials, dim3(nsteps), block, h->stream,
-               (const double*)h->partial.as<double>(), kc.nwg, h->psum.as<double>()));
     CHK(rec.run());
   }
   CHK(timing_end(h, &h->ms_mom, &h->n_mom, nsteps));

@@ -294,8 +294,9 @@ class HipEngine:
 
     def set_store_alpha(self, mode) -> None:
         """Keep every forward vector for autodiff_matrix (FKPM_OPT_STORE_ALPHA):
-        True / 2 whenever the table fits, 1 automatic (default), False / 0
-        recompute alpha backward."""
+        True / 2 whenever the table fits, 1 (default) the same but for lattices
+        that run the whole-recursion kernels, False / 0 recompute alpha
+        backward."""
         call("fkpm_set_option", self._h, _capi.OPT_STORE_ALPHA,
              2 if mode is True else 0 if mode is False else int(mode))
 

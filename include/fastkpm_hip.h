@@ -189,9 +189,10 @@ int fkpm_moments_noalloc(int device, int prec, int nb, int b, int nnzb, const in
                                    environment variable FKPM_ALPHA_TABLE_BYTES), and
                                    fkpm_autodiff_matrix then reads alpha_{m-1} instead of
                                    recomputing it (one gathered vector per step instead of two);
-                                   1 (default): the same when three vectors exceed the
-                                   32 MB of L2; 0: the three-vector ring and the
-                                   recomputation */
+                                   1 (default): the same, except that lattices small enough
+                                   for the whole-recursion kernels (about 4096 orbital rows)
+                                   run those, with a table of their own; 0: the three-vector
+                                   ring and the recomputation */
 #define FKPM_OPT_SWEEP 4        /* value 0: every kernel kind sweeps the rows per XCD; s in
                                    1..64: as one front in segments of s passes per XCD
                                    (fkpm_get_kernel_sweep); -1 (default): the configuration's
