@@ -474,21 +474,23 @@ void plan(bool single, const Request& r, Layout* L) {
   }
   L->qp = ((need + L->W - 1) / L->W) * L->W;
   L->sp = L->qp * ne;
-  // workgroups per slot: one per 4 block rows up to 2048 (fixed by the
-  // shape); they sweep the slot's rows as one front (chunk -1), or, with the
-  // lattice row order, the sweep positions one range per XCD (chunk > 0).  A
-  // slot's first workgroup sits at any offset of the launch, so workgroup k
-  // of the slot runs on XCD (offset + k) mod 8: the ranges keep to one XCD
-  // each, only which XCD takes which range shifts.
-  int nwg = std::min(std::max((r.nb + 3) / 4, 1), 2048);
+  // Workgroups per slot (fixed by the shape): one pass over the rows, at most
+  // 2048.  While the six vectors of a backward step stay in the last-level cache,
+  // and with the lattice row order, each XCD takes one range of the rows (chunk
+  // > 0), else the workgroups sweep them as one front (chunk -1).  A slot's
+  // first workgroup sits at any offset of the launch, so workgroup k of the
+  // slot runs on XCD (offset + k) mod 8: the ranges keep to one XCD each, only
+  // which XCD takes which range shifts.
+  const int gwg = (fkd::WG / fkd::WAVE) *
+                  (classes(single)[L->cls].mf ? 1 : fkd::WAVE / classes(single)[L->cls].L);
+  int nwg = std::min(std::max((r.nb + gwg - 1) / gwg, 1), 2048);
   int chunk = (r.nb + nwg - 1) / nwg;
-  if (!r.rdesc.empty()) {
-    const int gwg = (fkd::WG / fkd::WAVE) * (fkd::WAVE / classes(single)[L->cls].L);
-    chunk = (chunk + gwg - 1) / gwg * gwg;
-  }
+  const bool ranges = !r.rdesc.empty() ||
+                      (nwg >= 64 && 6 * (size_t)r.n * L->sp * 2 * es <= ((size_t)256 << 20));
+  if (ranges) chunk = (chunk + gwg - 1) / gwg * gwg;
   nwg = (r.nb + chunk - 1) / chunk;
   L->nwg = nwg;
-  L->chunk = r.rdesc.empty() ? -1 : chunk;
+  L->chunk = ranges ? chunk : -1;
   const size_t vec = (size_t)r.n * L->sp * 2 * es;
   const size_t dbl = (size_t)r.nnzb * r.b * r.b * 2 * sizeof(double);
   const size_t h = r.M / 2;
@@ -562,7 +564,7 @@ struct fkpm_batch {
   int peak_slots = 0;
   // graph cache for the current slot set
   long long set_version = 0, graph_version = -1;
-  std::map<int, hipGraphExec_t> graphs;  // by tick count
+  std::map<std::vector<unsigned char>, hipGraphExec_t> graphs;  // by tick_mask
 
   void clear_graphs() {
     for (auto& g : graphs) (void)hipGraphExecDestroy(g.second);
@@ -755,57 +757,90 @@ void upload_tables(fkpm_batch* B) {
   BCHK(hipStreamSynchronize(B->stream));  // host tables are reused next time
 }
 
-void enqueue_ticks(fkpm_batch* B, int T) {
-  const auto& cl = classes(B->single);
-  const int na = (int)B->h_act.size();
-  for (int t = 0; t < T; t++) {
-    for (size_t c = 0; c < cl.size(); c++) {
-      const int ns = (int)B->h_cls_slots[c].size();
-      if (ns == 0) continue;
-      const int grid = B->h_cls_off[c].back();
-      launch_k(cl[c].fwd, grid, B->stream, B->d_slots, B->d_st, B->d_cls_slots[c],
-               B->d_cls_off[c], ns);
-      launch_k(cl[c].bwd, grid, B->stream, B->d_slots, B->d_st, B->d_cls_slots[c],
-               B->d_cls_off[c], ns);
-      launch_k(cl[c].aux, grid, B->stream, B->d_slots, B->d_st, B->d_cls_slots[c],
-               B->d_cls_off[c], ns);
-    }
-    int* st = B->d_st;
-    const int* act = B->d_act;
-    void* argv[] = {(void*)&st, (void*)&act, (void*)&na};
-    BCHK(hipLaunchKernel((const void*)&fkd::k_batch_advance, dim3((na + 255) / 256), dim3(256),
-                         argv, 0, B->stream));
+// What a tick has to launch for one class: its forward kernel when some slot is
+// in its forward phase, and so on.  Every slot advances by one step a tick, so
+// the host knows the phases of all ticks of a run from the step counters it
+// last read.
+constexpr unsigned char kFwd = 1, kBwd = 2, kAux = 4;
+
+std::vector<unsigned char> tick_mask(const fkpm_batch* B, int t) {
+  std::vector<unsigned char> m(classes(B->single).size(), 0);
+  for (const Slot& sl : B->active) {
+    const int step = B->h_st[sl.idx] + t, M = sl.rq->M, h = M / 2;
+    unsigned char& b = m[sl.lay.cls];
+    if (step < h) b |= kFwd;
+    if (step > h && step < M) b |= kBwd;
+    if (step == 0 || step == h || step == M || step == M + 1) b |= kAux;
   }
+  return m;
 }
 
+void enqueue_tick(fkpm_batch* B, const std::vector<unsigned char>& mask) {
+  const auto& cl = classes(B->single);
+  for (size_t c = 0; c < cl.size(); c++) {
+    const int ns = (int)B->h_cls_slots[c].size();
+    if (ns == 0) continue;
+    const int grid = B->h_cls_off[c].back();
+    const struct {
+      unsigned char bit;
+      BatchKernel fn;
+    } phase[] = {{kFwd, cl[c].fwd}, {kBwd, cl[c].bwd}, {kAux, cl[c].aux}};
+    for (const auto& p : phase)
+      if (mask[c] & p.bit)
+        launch_k(p.fn, grid, B->stream, B->d_slots, B->d_st, B->d_cls_slots[c], B->d_cls_off[c],
+                 ns);
+  }
+  int* st = B->d_st;
+  const int* act = B->d_act;
+  const int na = (int)B->h_act.size();
+  void* argv[] = {(void*)&st, (void*)&act, (void*)&na};
+  BCHK(hipLaunchKernel((const void*)&fkd::k_batch_advance, dim3((na + 255) / 256), dim3(256), argv,
+                       0, B->stream));
+}
+
+// kGraphTicks ticks of one mask as a graph (captured once per slot set and mask).
+constexpr int kGraphTicks = 8;
+
+void replay_ticks(fkpm_batch* B, const std::vector<unsigned char>& mask) {
+  if (B->graph_version != B->set_version) {
+    B->clear_graphs();
+    B->graph_version = B->set_version;
+  }
+  auto it = B->graphs.find(mask);
+  if (it == B->graphs.end()) {
+    hipGraph_t g = nullptr;
+    hipGraphExec_t ex = nullptr;
+    BCHK(hipStreamBeginCapture(B->stream, hipStreamCaptureModeThreadLocal));
+    try {
+      for (int t = 0; t < kGraphTicks; t++) enqueue_tick(B, mask);
+    } catch (...) {
+      hipGraph_t junk = nullptr;
+      (void)hipStreamEndCapture(B->stream, &junk);
+      if (junk) (void)hipGraphDestroy(junk);
+      throw;
+    }
+    BCHK(hipStreamEndCapture(B->stream, &g));
+    BCHK(hipGraphInstantiate(&ex, g, nullptr, nullptr, 0));
+    (void)hipGraphDestroy(g);
+    it = B->graphs.emplace(mask, ex).first;
+    B->n_captures++;
+  }
+  BCHK(hipGraphLaunch(it->second, B->stream));
+}
+
+// T ticks: stretches of kGraphTicks ticks with the same work as graphs, the
+// others (a slot changing its phase) launched directly.
 void run_ticks(fkpm_batch* B, int T, bool use_graph) {
-  if (!use_graph) {
-    enqueue_ticks(B, T);
-  } else {
-    if (B->graph_version != B->set_version) {
-      B->clear_graphs();
-      B->graph_version = B->set_version;
+  for (int t = 0; t < T;) {
+    const std::vector<unsigned char> mask = tick_mask(B, t);
+    int n = 1;
+    while (n < kGraphTicks && t + n < T && tick_mask(B, t + n) == mask) n++;
+    if (use_graph && n == kGraphTicks) {
+      replay_ticks(B, mask);
+    } else {
+      for (int k = 0; k < n; k++) enqueue_tick(B, mask);
     }
-    auto it = B->graphs.find(T);
-    if (it == B->graphs.end()) {
-      hipGraph_t g = nullptr;
-      hipGraphExec_t ex = nullptr;
-      BCHK(hipStreamBeginCapture(B->stream, hipStreamCaptureModeThreadLocal));
-      try {
-        enqueue_ticks(B, T);
-      } catch (...) {
-        hipGraph_t junk = nullptr;
-        (void)hipStreamEndCapture(B->stream, &junk);
-        if (junk) (void)hipGraphDestroy(junk);
-        throw;
-      }
-      BCHK(hipStreamEndCapture(B->stream, &g));
-      BCHK(hipGraphInstantiate(&ex, g, nullptr, nullptr, 0));
-      (void)hipGraphDestroy(g);
-      it = B->graphs.emplace(T, ex).first;
-      B->n_captures++;
-    }
-    BCHK(hipGraphLaunch(it->second, B->stream));
+    t += n;
   }
   B->n_ticks += T;
   B->n_replays++;
