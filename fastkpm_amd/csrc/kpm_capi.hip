@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -17,6 +18,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <type_traits>
 #include <vector>
 
@@ -310,6 +312,7 @@ fkd::RSource<S> no_rsource() {
 
 struct fkpm_handle {
   int device = 0;
+  size_t total_bytes = 0;  // memory of the device (0: not asked yet)
   hipStream_t stream = nullptr;
   int dtype = FKPM_C64;
   int prec = FKPM_PREC_FP64;
@@ -322,6 +325,7 @@ struct fkpm_handle {
   DevBuf rp, ci, hv, rowblk, hraw;
   double avg = 0.0, mag = 1.0;
   std::vector<int> h_rp, h_ci;
+  bool pattern_set = false;  // the device holds the pattern of h_rp, h_ci
 
   // --- R and recursion state ---
   int n = 0, s = 0;
@@ -340,7 +344,8 @@ struct fkpm_handle {
   bool rr_force = false;  // FKPM_OPT_MFMA 2: row-resident ones by default wherever they exist
   int stoch_method = FKPM_STOCH_AUTO;
   int stoch_used = -1;  // method the last stoch_matrix ran (FKPM_STOCH_*)
-  DevBuf R, A[3], Bv[3], xi, partial, psum, tune_dacc;
+  DevBuf R, A[3], Bv[3], xi, partial, tune_dacc;
+  PinBuf psum;             // moment sums, written by the reducing kernel
   int alpha_M = 0;  // M of the moments whose final state is held, 0 if none
   DevBuf atab;            // alpha_1 .. alpha_{M/2} of the last moments(M), when it fits
   bool a_stored = false;  // the forward vectors live in atab (else the ring A[3])
@@ -374,6 +379,12 @@ struct fkpm_handle {
   DevBuf dout_f;  // D rounded to float for single-precision engines
   std::vector<int> hd_rp, hd_ci;
 
+  // --- pinned staging of host arrays ---
+  PinBuf stage;             // H values on their way in (upload_H_t)
+  bool stage_busy = false;  // a copy from it may still be queued
+  PinBuf dpin;              // chunks of a large D on their way out (copy_to_host)
+  std::vector<hipEvent_t> dpin_ev;
+
   // --- two-current moments (moments2) ---
   DevBuf j_rp[2], j_ci[2], j_rb[2], j_raw[2], j_val[2], m2_a, m2_b, m2_ring, m2_c, m2_part;
 
@@ -393,7 +404,7 @@ struct fkpm_handle {
     if (stream) (void)hipStreamSynchronize(stream);
     DevBuf* bufs[] = {&rp,    &ci,    &hv,      &rowblk, &hraw, &rraw,  &rcol,     &rval,
                       &rflag, &R,     &A[0],    &A[1],   &A[2], &Bv[0], &Bv[1],    &Bv[2],
-                      &xi,    &partial, &psum,  &tune_dacc, &drp, &dci,  &tpos,     &dacc,
+                      &xi,    &partial, &tune_dacc, &drp, &dci,  &tpos,     &dacc,
                       &dout,  &dout_f, &atab,  &tabc, &rdesc};
     for (DevBuf* d : bufs) d->release();
     DevBuf* m2bufs[] = {&j_rp[0], &j_ci[0], &j_rb[0], &j_raw[0], &j_val[0], &j_rp[1], &j_ci[1],
@@ -402,6 +413,10 @@ struct fkpm_handle {
     DevBuf* rbufs[] = {&res.hval, &res.hoff, &res.atab, &res.btab, &res.xi, &res.coef, &res.part};
     for (DevBuf* d : rbufs) d->release();
     res.pin.release();
+    psum.release();
+    stage.release();
+    dpin.release();
+    for (hipEvent_t e : dpin_ev) (void)hipEventDestroy(e);
     gcache.clear();
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
@@ -1425,12 +1440,15 @@ int moments_t(fkpm_handle* h, int M, double* mu) {
   // memory (or the byte count in FKPM_ALPHA_TABLE_BYTES).
   {
     const size_t need = (size_t)nsteps * h->vbytes();
-    size_t free_b = 0, total_b = 0;
-    HIPCHK(hipMemGetInfo(&free_b, &total_b));
     // default: half of what is free (the table already held counts as free),
     // never more than a quarter of the device, so that other engines and a
     // batch arena on the same device keep room whatever the order of calls
-    size_t budget = std::min(free_b / 2 + h->atab.bytes, total_b / 4);
+    size_t budget = h->total_bytes / 4;
+    if (need > h->atab.bytes || h->total_bytes == 0) {  // else the held table is big enough
+      size_t free_b = 0;
+      HIPCHK(hipMemGetInfo(&free_b, &h->total_bytes));
+      budget = std::min(free_b / 2 + h->atab.bytes, h->total_bytes / 4);
+    }
     if (h->table_cap_mb >= 0) budget = (size_t)h->table_cap_mb << 20;
     if (const char* e = getenv("FKPM_ALPHA_TABLE_BYTES")) budget = (size_t)strtoull(e, nullptr, 10);
     h->a_stored = false;
@@ -1461,19 +1479,75 @@ int moments_t(fkpm_handle* h, int M, double* mu) {
       if ((m + 1) % group == 0 || m == nsteps - 1) {
         const int m0 = m - m % group;
         CHK(launch(&fkd::k_reduce_partials, dim3(m + 1 - m0), block, h->stream,
-                   (const double*)h->partial.as<double>(), kc.nwg, h->psum.as<double>() + 2 * m0));
+                   (const double*)h->partial.as<double>(), kc.nwg, (double*)h->psum.p + 2 * m0));
       }
     }
     CHK(rec.run());
   }
   CHK(timing_end(h, &h->ms_mom, &h->n_mom, nsteps));
   if (h->a_stored) h->tab_K = nsteps;
-  std::vector<double> ps((size_t)nsteps * 2);
-  HIPCHK(hipMemcpyAsync(ps.data(), h->psum.p, ps.size() * sizeof(double), hipMemcpyDeviceToHost,
-                        h->stream));
   HIPCHK(hipStreamSynchronize(h->stream));
-  moments_from_sums(ps.data(), nsteps, mu);
+  moments_from_sums((const double*)h->psum.p, nsteps, mu);
   h->alpha_M = M;
+  return 0;
+}
+
+// A large copy to pageable memory runs at the rate of one core copying out of
+// pinned memory (17 GB/s), a third of the link's: from kBigCopy on, four threads
+// copy chunks out of a ring of pinned buffers while the next chunks arrive
+// (117 MB: 6.9 -> 2.7 ms).
+constexpr size_t kBigCopy = 16 << 20, kCopyChunk = 2 << 20;
+constexpr int kCopyThreads = 4;
+
+int copy_to_host(fkpm_handle* h, void* dst, const void* src, size_t bytes) {
+  if (bytes < kBigCopy) {
+    HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(hipStreamSynchronize(h->stream));
+    return 0;
+  }
+  CHK(h->dpin.ensure(2 * kCopyThreads * kCopyChunk));
+  while (h->dpin_ev.size() < 2 * kCopyThreads) {
+    hipEvent_t e = nullptr;
+    HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    h->dpin_ev.push_back(e);
+  }
+  const size_t n = (bytes + kCopyChunk - 1) / kCopyChunk;
+  std::atomic<int> err{hipSuccess};
+  // thread w takes chunks w, w + kCopyThreads, ..., two of them under way
+  auto work = [&](int w) {
+    auto note = [&](hipError_t e) {
+      if (e != hipSuccess) err = e;
+      return e == hipSuccess;
+    };
+    if (!note(hipSetDevice(h->device))) return;
+    auto slot = [&](size_t i) { return 2 * w + (int)(i / kCopyThreads & 1); };
+    auto len = [&](size_t i) { return std::min(kCopyChunk, bytes - i * kCopyChunk); };
+    auto fetch = [&](size_t i) {
+      return i >= n ||
+             (note(hipMemcpyAsync((char*)h->dpin.p + slot(i) * kCopyChunk,
+                                  (const char*)src + i * kCopyChunk, len(i), hipMemcpyDeviceToHost,
+                                  h->stream)) &&
+              note(hipEventRecord(h->dpin_ev[slot(i)], h->stream)));
+    };
+    if (!fetch(w) || !fetch(w + kCopyThreads)) return;
+    for (size_t i = w; i < n; i += kCopyThreads) {
+      if (!note(hipEventSynchronize(h->dpin_ev[slot(i)]))) return;
+      memcpy((char*)dst + i * kCopyChunk, (const char*)h->dpin.p + slot(i) * kCopyChunk, len(i));
+      if (!fetch(i + 2 * kCopyThreads)) return;
+    }
+  };
+  std::thread pool[kCopyThreads];
+  int started = 1;
+  try {
+    for (; started < kCopyThreads; started++) pool[started] = std::thread(work, started);
+  } catch (const std::exception&) {
+    // no thread to be had: this one takes the remaining chunks below
+  }
+  work(0);
+  for (int w = started; w < kCopyThreads; w++) work(w);
+  for (int w = 1; w < started; w++) pool[w].join();
+  HIPCHK((hipError_t)err.load());
+  HIPCHK(hipStreamSynchronize(h->stream));
   return 0;
 }
 
@@ -1490,9 +1564,7 @@ int copy_D_out(fkpm_handle* h, void* D_val) {
                (const double*)h->dout.as<double>(), h->dout_f.as<float>(), cnt));
     src = h->dout_f.p;
   }
-  HIPCHK(hipMemcpyAsync(D_val, src, bytes, hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(hipStreamSynchronize(h->stream));
-  return 0;
+  return copy_to_host(h, D_val, src, bytes);
 }
 
 int check_D_ready(fkpm_handle* h) {
@@ -2024,11 +2096,23 @@ int moments2_t(fkpm_handle* h, int M, int col_chunk, size_t budget, double* mu) 
   return 0;  // the buffers of moments / autodiff_matrix are untouched
 }
 
+// H values up to this size go through pinned staging, so that set_H returns
+// without waiting for the device.
+constexpr size_t kStageBytes = 512 << 10;
+
 template <class TH, class S, bool CX>
 int upload_H_t(fkpm_handle* h, DevBuf& dst, const void* val, double mag, double shift) {
-  const size_t cnt = (size_t)h->nnzb * h->b * h->b;
-  HIPCHK(hipMemcpyAsync(h->hraw.p, val, cnt * sizeof(TH) * (CX ? 2 : 1), hipMemcpyHostToDevice,
-                        h->stream));
+  const size_t cnt = (size_t)h->nnzb * h->b * h->b, bytes = cnt * sizeof(TH) * (CX ? 2 : 1);
+  if (bytes <= kStageBytes) {
+    if (h->stage_busy) HIPCHK(hipStreamSynchronize(h->stream));
+    CHK(h->stage.ensure(kStageBytes));
+    memcpy(h->stage.p, val, bytes);
+    val = h->stage.p;
+    h->stage_busy = true;
+  } else {
+    h->stage_busy = false;  // set_H waits for the stream
+  }
+  HIPCHK(hipMemcpyAsync(h->hraw.p, val, bytes, hipMemcpyHostToDevice, h->stream));
   return launch(&fkd::k_scale_H<TH, S, CX>, dim3(grid_for(cnt)), dim3(256), h->stream,
                 h->hraw.as<const TH>(), dst.as<S>(), h->rowblk.as<const int>(),
                 h->ci.as<const int>(), h->nnzb, h->b, mag, shift);
@@ -2051,7 +2135,7 @@ int upload_H_s(fkpm_handle* h, DevBuf& dst, const void* val, double mag, double 
 // n1 n2 n3 = nb and every side at least 8.  Fills n[3]; false otherwise.
 bool lattice_dims(int nb, const int* rp, const int* ci, int n[3]) {
   if (nb < 512) return false;
-  std::map<int, long long> cnt;
+  std::vector<int> cnt(nb / 2 + 1, 0);  // blocks at each distance
   for (int i = 0; i < nb; i++)
     for (int p = rp[i]; p < rp[i + 1]; p++) {
       int d = ci[p] - i;
@@ -2060,8 +2144,8 @@ bool lattice_dims(int nb, const int* rp, const int* ci, int n[3]) {
       cnt[std::min(d, nb - d)]++;
     }
   std::vector<int> dist;
-  for (const auto& kv : cnt)
-    if (2 * kv.second >= nb) dist.push_back(kv.first);
+  for (int d = 1; d <= nb / 2; d++)
+    if (2ll * cnt[d] >= nb) dist.push_back(d);
   if (dist.size() != 3 || dist[0] != 1) return false;
   const long long n1 = dist[1], c = dist[2];
   if (c % n1 != 0 || nb % c != 0) return false;
@@ -2101,6 +2185,7 @@ bool lattice_order(int nb, const int* rp, const int* ci, std::vector<int>& order
 
 int upload_pattern(fkpm_handle* h, int nb, int b, int nnzb, const int* row_ptr,
                    const int* col_idx) {
+  h->pattern_set = false;
   h->nb = nb;
   h->b = b;
   h->nnzb = nnzb;
@@ -2138,6 +2223,7 @@ int upload_pattern(fkpm_handle* h, int nb, int b, int nnzb, const int* row_ptr,
   // the async copies above read host arrays owned by the caller (and desc):
   // finish them
   HIPCHK(hipStreamSynchronize(h->stream));
+  h->pattern_set = true;
   return 0;
 }
 
@@ -2396,11 +2482,19 @@ int fkpm_set_H(fkpm_handle* h, int nb, int b, int nnzb, const int* row_ptr, cons
   if (!fkd::block_supported(b)) return fail(FKPM_E_UNSUP, "block size %d has no kernels", b);
   if (!(mag > 0) || !std::isfinite(avg)) return fail(FKPM_E_ARG, "bad energy scale avg=%g mag=%g", avg, mag);
   if (nnzb > 0 && !val) return fail(FKPM_E_ARG, "null H values");
-  CHK(check_pattern("set_H", nb, nnzb, row_ptr, nullptr, col_idx));
-  for (int i = 0; i < nb; i++) {  // engine_cusparse.cpp:716-727: every diagonal block present
-    bool found = false;
-    for (int p = row_ptr[i]; p < row_ptr[i + 1]; p++) found |= (col_idx[p] == i);
-    if (!found) return fail(FKPM_E_ARG, "set_H: diagonal block (%d,%d) is missing", i, i);
+  // The pattern the handle already holds (compared by content, as in a loop
+  // over Hamiltonians on one lattice) has been checked and is on the device.
+  const bool same = h->pattern_set && nb == h->nb && b == h->b && nnzb == h->nnzb && row_ptr &&
+                    (nnzb == 0 || col_idx) &&
+                    memcmp(row_ptr, h->h_rp.data(), sizeof(int) * ((size_t)nb + 1)) == 0 &&
+                    (nnzb == 0 || memcmp(col_idx, h->h_ci.data(), sizeof(int) * (size_t)nnzb) == 0);
+  if (!same) {
+    CHK(check_pattern("set_H", nb, nnzb, row_ptr, nullptr, col_idx));
+    for (int i = 0; i < nb; i++) {  // engine_cusparse.cpp:716-727: every diagonal block present
+      bool found = false;
+      for (int p = row_ptr[i]; p < row_ptr[i + 1]; p++) found |= (col_idx[p] == i);
+      if (!found) return fail(FKPM_E_ARG, "set_H: diagonal block (%d,%d) is missing", i, i);
+    }
   }
   // The kernel choice depends on the block size, the block-row and block
   // counts (grids, tuned-shape key) and on whether every row has at most
@@ -2408,7 +2502,7 @@ int fkpm_set_H(fkpm_handle* h, int nb, int b, int nnzb, const int* row_ptr, cons
   // or at most 7 (their instantiation without a padding slot): a change of any
   // of them picks the kernels again at the next use.
   const int old_b = h->b, old_nb = h->nb, old_nnzb = h->nnzb, old_deg = h->max_deg;
-  CHK(upload_pattern(h, nb, b, nnzb, row_ptr, col_idx));
+  if (!same) CHK(upload_pattern(h, nb, b, nnzb, row_ptr, col_idx));
   const bool geo_change = b != old_b || nb != old_nb || nnzb != old_nnzb ||
                           (old_deg <= kRowResidentMax) != (h->max_deg <= kRowResidentMax) ||
                           (old_deg <= 7) != (h->max_deg <= 7);
@@ -2420,7 +2514,7 @@ int fkpm_set_H(fkpm_handle* h, int nb, int b, int nnzb, const int* row_ptr, cons
     CHK(upload_H_s<float>(h, h->hv, val, mag, avg / mag));
   else
     CHK(upload_H_s<double>(h, h->hv, val, mag, avg / mag));
-  HIPCHK(hipStreamSynchronize(h->stream));
+  if (!h->stage_busy) HIPCHK(hipStreamSynchronize(h->stream));  // the copy reads val itself
   h->h_set = true;
   h->alpha_M = 0;
   h->tab_K = 0;

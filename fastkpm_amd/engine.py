@@ -206,11 +206,12 @@ class HipEngine:
         rp = np.ascontiguousarray(D.row_ptr, dtype=np.int32)
         ri = np.ascontiguousarray(D.row_idx, dtype=np.int32)
         ci = np.ascontiguousarray(D.col_idx, dtype=np.int32)
-        key = (D.n_rows, rp.tobytes(), ci.tobytes())
-        if key != self._d_pattern_key:
+        key = self._d_pattern_key
+        if key is None or key[0] != D.n_rows or not np.array_equal(key[1], rp) \
+                or not np.array_equal(key[2], ci):
             call("fkpm_set_D_pattern", self._h, D.n_rows, D.n_blocks(), _iptr(rp), _iptr(ri),
                  _iptr(ci))
-            self._d_pattern_key = key
+            self._d_pattern_key = (D.n_rows, rp.copy(), ci.copy())
 
     def _D_out(self, D: SpMatBsr, keep_on_device: bool):
         if keep_on_device:

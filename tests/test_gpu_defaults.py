@@ -123,3 +123,27 @@ def test_matrix_core_backward_step_from_the_table(oracle, rows, S, prec):
     assert eng.stoch_method() == "table"
     assert rel_err(D.val, orc.stoch_matrix(c, D)) < tol
     eng.close()
+
+
+@pytest.mark.parametrize("shapes", [((20, 18), (20, 18)), ((20, 18), (18, 20)),
+                                    ((20, 18), (70, 70)), ((70, 70), (20, 18))])
+def test_set_H_arrays_are_free_on_return(oracle, shapes):
+    """H values below and above the staged size, on a held and on a new
+    pattern: the caller's arrays may change as soon as set_H returns."""
+    from fastkpm_amd import EnergyScale, HipEngine, lattice
+    eng = HipEngine("cx_double", "fp64")
+    for k, shape in enumerate(shapes * 2):
+        H = lattice.lattice(shape, b=2, J=1.0 + k, seed=k)
+        rng = np.random.default_rng(k)
+        R = rng.standard_normal((H.n_rows * 2, 3)) + 1j * rng.standard_normal((H.n_rows * 2, 3))
+        orc = oracle.Engine()
+        orc.set_H(H, -12.0, 12.0)
+        orc.set_R(R)
+        want = orc.moments(12)
+        if k % 2:  # values that must not survive
+            eng.set_H(lattice.lattice(shape, b=2, J=9.0, seed=77), EnergyScale(-20.0, 20.0))
+        eng.set_R(R)
+        eng.set_H(H, EnergyScale(-12.0, 12.0))
+        H.val[:] = 1e30
+        assert rel_err(eng.moments(12), want) < 1e-10
+    eng.close()
