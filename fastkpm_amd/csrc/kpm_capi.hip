@@ -906,13 +906,18 @@ int ensure_ready(fkpm_handle* h) {
 // Steps whose moment partials are held before they are reduced: 64 MiB of them
 // (a step of 65536 workgroups leaves 1 MiB).
 int partial_steps(int nsteps, int nwg) {
-  const size_t per = (size_t)nwg * 2 * sizeof(double);
+  const size_t per = (size_t)std::max(nwg, 1) * 2 * sizeof(double);
   return (int)std::min<size_t>(nsteps, std::max<size_t>(1, ((size_t)64 << 20) / per));
 }
 
 int ensure_partials(fkpm_handle* h, int nsteps) {
-  const int nwg = std::max(h->kc[K_MOM].nwg, h->kc[K_MOMT].nwg);
-  CHK(h->partial.ensure((size_t)partial_steps(nsteps, nwg) * nwg * 2 * sizeof(double)));
+  // the wider grid may hold fewer steps and less memory in all
+  size_t rows = 0;
+  for (int kind : {K_MOM, K_MOMT}) {
+    const int nwg = h->kc[kind].nwg;
+    rows = std::max(rows, (size_t)partial_steps(nsteps, nwg) * nwg);
+  }
+  CHK(h->partial.ensure(rows * 2 * sizeof(double)));
   CHK(h->psum.ensure((size_t)nsteps * 2 * sizeof(double)));
   return 0;
 }
