@@ -1191,6 +1191,11 @@ void moments_from_sums(const double* ps, int nsteps, double* mu) {
   }
 }
 
+// Packets of a vector up to which k_table_sums splits the slots (us, split / one
+// thread a packet; 250 slots FP64: 16384 packets 23 / 37, 32768 29 / 40, 65536 69 /
+// 43; 64 slots: 6 / 8, 9 / 12, 19 / 13).
+constexpr size_t kSumsSplit = 32768;
+
 // Weights of the table vectors in stoch_matrix (stoch_table): d_0 .. d_K of v,
 // then e_0 .. e_K of u.
 void stoch_table_weights(int M, const double* c, std::vector<double>& w) {
@@ -1201,6 +1206,25 @@ void stoch_table_weights(int M, const double* c, std::vector<double>& w) {
     w[i] = (i < K ? cm(i) : 0.0) - (i >= 1 ? cm(2 * K - i) : 0.0);  // d_i
     w[K + 1 + i] = i < K ? cm(K + i) : 0.0;                         // e_i
   }
+}
+
+// u, v of stoch_matrix from K table slots of n scalars (k_table_sums).
+template <class S>
+int table_sums(fkpm_handle* h, const S* R, const S* tab, size_t n, int K, const double* d,
+               const double* e, S* u, S* v) {
+  const size_t np = n * sizeof(S) / 16;
+  if (np <= kSumsSplit)
+    return launch(&fkd::k_table_sums<S, 8>, dim3((unsigned)((np + 31) / 32)), dim3(fkd::WG),
+                  h->stream, R, tab, n, K, d, e, u, v, n);
+  return launch(&fkd::k_table_sums<S, 1>, dim3(4096), dim3(fkd::WG), h->stream, R, tab, n, K, d, e,
+                u, v, n);
+}
+
+// out = (add ? out : 0) + the ny rows of part, cnt values each (k_sum_parts).
+int sum_parts(fkpm_handle* h, const double* part, int ny, size_t cnt, double* out, bool add) {
+  const size_t wgs = (cnt + fkd::SUM_X - 1) / fkd::SUM_X;
+  return launch(&fkd::k_sum_parts, dim3((unsigned)std::min<size_t>(std::max<size_t>(wgs, 1), 65536)),
+                dim3(fkd::WG), h->stream, part, ny, cnt, out, add ? 1 : 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1376,8 +1400,7 @@ int res_outer(fkpm_handle* h, const fkd::ResTerms<S>& T, int nterm, double* dst)
   if (h->b == 2) rc = h->cx ? go(&fkd::k_res_outer<S, true, 2>) : go(&fkd::k_res_outer<S, false, 2>);
   if (h->b == 4) rc = h->cx ? go(&fkd::k_res_outer<S, true, 4>) : go(&fkd::k_res_outer<S, false, 4>);
   CHK(rc);
-  return launch(&fkd::k_res_outer_sum, dim3(grid_for(cnt)), block, h->stream,
-                (const double*)h->res.part.as<double>(), (int)ny, cnt, dst);
+  return sum_parts(h, h->res.part.as<const double>(), (int)ny, cnt, dst, false);
 }
 
 // The backward recursion and D from the resident table, into dacc.
@@ -1414,9 +1437,8 @@ int res_stoch(fkpm_handle* h, int M, const double* c, bool table) {
   if (table) {
     stoch_table_weights(M, c, w);
     CHK(res_coef(h, w.data(), (int)w.size()));
-    CHK(launch(&fkd::k_table_sums<S>, dim3(grid_for(slot)), dim3(fkd::WG), h->stream,
-               h->res.atab.as<const S>(), h->res.atab.as<const S>() + slot, slot, K,
-               h->res.coef.as<const double>(), h->res.coef.as<const double>() + K + 1, u, v, slot));
+    CHK(table_sums<S>(h, h->res.atab.as<const S>(), h->res.atab.as<const S>() + slot, slot, K,
+                      h->res.coef.as<const double>(), h->res.coef.as<const double>() + K + 1, u, v));
   } else {
     CHK(res_coef(h, c, M));
   }
@@ -1649,9 +1671,8 @@ int stoch_table(fkpm_handle* h, int M, const double* c, const S** xi_out) {
   S* u = (S*)h->A[0].p;
   S* v = (S*)h->Bv[0].p;
   const size_t n = vb / sizeof(S);
-  CHK(launch(&fkd::k_table_sums<S>, dim3(4096), block, h->stream, (const S*)h->R.p,
-             (const S*)h->atab.p, n, K, (const double*)h->tabc.as<double>(),
-             (const double*)h->tabc.as<double>() + K + 1, u, v, n));
+  CHK(table_sums<S>(h, (const S*)h->R.p, (const S*)h->atab.p, n, K, h->tabc.as<const double>(),
+                    h->tabc.as<const double>() + K + 1, u, v));
   // y_0 = u, y_1 = Hs u, y_{k+1} = 2 Hs y_k - y_{k-1}; the last step writes
   // 2 y_K + v
   fkd::RSource<S> addv = no_rsource<S>();
@@ -1899,7 +1920,7 @@ bool kset_for_width<float>(fkpm_handle* h, int W, fkd::KSet<float>* ks, int* L, 
 
 // C (M x M, FP64, row-major (m1, m2)) = [C +] A^H B for K x M matrices A, B
 // of the storage type (column m at A + m * ld): k_dot_block over slices of
-// 512 k interleaved across about 2048 workgroups, then k_dot_reduce adding
+// 512 k interleaved across about 2048 workgroups, then k_sum_parts adding
 // the grid rows' partial blocks in order (at most 1 GiB of them).
 template <class S>
 int dot_block_acc(fkpm_handle* h, const S* A, const S* B, long long K, long long ld, int M,
@@ -1922,8 +1943,7 @@ int dot_block_acc(fkpm_handle* h, const S* A, const S* B, long long K, long long
   else
     CHK(launch(&fkd::k_dot_block<S, false>, dim3(nblk, (int)ny), dim3(fkd::WG), h->stream, A, B,
                ld, 0LL, K, kslice, M, part));
-  return launch(&fkd::k_dot_reduce, dim3(grid_for(cnt)), dim3(fkd::WG), h->stream,
-                (const double*)part, (int)ny, cnt, h->m2_c.as<double>(), first ? 1 : 0);
+  return sum_parts(h, part, (int)ny, cnt, h->m2_c.as<double>(), !first);
 }
 
 template <class TH, class S, bool CX>

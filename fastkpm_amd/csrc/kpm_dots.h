@@ -185,16 +185,4 @@ __global__ __launch_bounds__(WG) void k_dot_block(const S* __restrict__ A,
       }
 }
 
-// acc[x] = (first ? 0 : acc[x]) + sum over y of part[y * cnt + x], y in order.
-__global__ __launch_bounds__(WG) void k_dot_reduce(const double* __restrict__ part, int ny,
-                                                    size_t cnt, double* __restrict__ acc,
-                                                    int first) {
-  for (size_t x = (size_t)blockIdx.x * blockDim.x + threadIdx.x; x < cnt;
-       x += (size_t)gridDim.x * blockDim.x) {
-    double s = first ? 0.0 : acc[x];
-    for (int y = 0; y < ny; y++) s += part[(size_t)y * cnt + x];
-    acc[x] = s;
-  }
-}
-
 }  // namespace fkd

@@ -1352,52 +1352,110 @@ __global__ __launch_bounds__(WG) void k_copy16(const double2* __restrict__ a,
 // (alpha_0 = R, alpha_i = table slot i-1, slots `slot` scalars apart), one
 // streaming pass over the table with FP64 sums; n scalars per vector, a
 // multiple of the 16-byte packet.  Each thread keeps U slots' loads in flight.
-template <typename S>
+// The slots are cut into SL runs, summed by SL threads a packet: bound by HBM
+// with SL = 1 on large vectors (256^2 x 2 x 64: 5.7 TB/s), by the chain of K / U
+// round trips where one thread a packet leaves most of the chip idle.
+template <typename S, int SL>
 __global__ __launch_bounds__(WG) void k_table_sums(const S* __restrict__ R,
                                                    const S* __restrict__ tab, size_t slot, int K,
                                                    const double* __restrict__ d,
                                                    const double* __restrict__ e,
                                                    S* __restrict__ u, S* __restrict__ v, size_t n) {
   typedef typename Vec16<S>::V VT;
-  constexpr int NS = Vec16<S>::N, U = 8;
+  constexpr int NS = Vec16<S>::N, U = 8, PQ = WG / SL;  // PQ: packets of a workgroup
+  __shared__ double part[SL > 1 ? 2 * NS * WG : 1];
   const size_t np = n / NS;
-  for (size_t q = (size_t)blockIdx.x * WG + threadIdx.x; q < np; q += (size_t)gridDim.x * WG) {
+  const int sl = SL > 1 ? threadIdx.x / PQ : 0;
+  const int per = (K + SL - 1) / SL;
+  const int i1 = min(K, (sl + 1) * per);
+  for (size_t q0 = (size_t)blockIdx.x * PQ; q0 < np; q0 += (size_t)gridDim.x * PQ) {
+    const size_t q = q0 + threadIdx.x % PQ;
     double au[NS], av[NS];
-    {
-      const VT r = __builtin_nontemporal_load(reinterpret_cast<const VT*>(R) + q);
 #pragma unroll
-      for (int t = 0; t < NS; t++) {
-        av[t] = d[0] * (double)r[t];
-        au[t] = K > 0 ? e[0] * (double)r[t] : 0.0;
+    for (int t = 0; t < NS; t++) au[t] = av[t] = 0.0;
+    if (q < np) {
+      if (sl == 0) {
+        const VT r = __builtin_nontemporal_load(reinterpret_cast<const VT*>(R) + q);
+#pragma unroll
+        for (int t = 0; t < NS; t++) {
+          av[t] = d[0] * (double)r[t];
+          au[t] = K > 0 ? e[0] * (double)r[t] : 0.0;
+        }
       }
-    }
-    for (int i0 = 1; i0 <= K; i0 += U) {
-      VT x[U];
+      for (int i0 = 1 + sl * per; i0 <= i1; i0 += U) {
+        VT x[U];
 #pragma unroll
-      for (int k = 0; k < U; k++)
-        if (i0 + k <= K)
-          x[k] = __builtin_nontemporal_load(reinterpret_cast<const VT*>(tab + (size_t)(i0 + k - 1) * slot) + q);
+        for (int k = 0; k < U; k++)
+          if (i0 + k <= i1)
+            x[k] = __builtin_nontemporal_load(reinterpret_cast<const VT*>(tab + (size_t)(i0 + k - 1) * slot) + q);
 #pragma unroll
-      for (int k = 0; k < U; k++) {
-        const int i = i0 + k;
-        if (i <= K) {
-          const double di = d[i], ei = i < K ? e[i] : 0.0;
+        for (int k = 0; k < U; k++) {
+          const int i = i0 + k;
+          if (i <= i1) {
+            const double di = d[i], ei = i < K ? e[i] : 0.0;
 #pragma unroll
-          for (int t = 0; t < NS; t++) {
-            av[t] = fma(di, (double)x[k][t], av[t]);
-            au[t] = fma(ei, (double)x[k][t], au[t]);
+            for (int t = 0; t < NS; t++) {
+              av[t] = fma(di, (double)x[k][t], av[t]);
+              au[t] = fma(ei, (double)x[k][t], au[t]);
+            }
           }
         }
       }
     }
-    VT ou, ov;
+    if constexpr (SL > 1) {
+      __syncthreads();
 #pragma unroll
-    for (int t = 0; t < NS; t++) {
-      ou[t] = (S)au[t];
-      ov[t] = (S)av[t];
+      for (int t = 0; t < NS; t++) {
+        part[(2 * t) * WG + threadIdx.x] = au[t];
+        part[(2 * t + 1) * WG + threadIdx.x] = av[t];
+      }
+      __syncthreads();
+      if (sl == 0)
+        for (int k = 1; k < SL; k++)
+#pragma unroll
+          for (int t = 0; t < NS; t++) {
+            au[t] += part[(2 * t) * WG + k * PQ + threadIdx.x];
+            av[t] += part[(2 * t + 1) * WG + k * PQ + threadIdx.x];
+          }
     }
-    reinterpret_cast<VT*>(u)[q] = ou;
-    reinterpret_cast<VT*>(v)[q] = ov;
+    if (sl == 0 && q < np) {
+      VT ou, ov;
+#pragma unroll
+      for (int t = 0; t < NS; t++) {
+        ou[t] = (S)au[t];
+        ov[t] = (S)av[t];
+      }
+      reinterpret_cast<VT*>(u)[q] = ou;
+      reinterpret_cast<VT*>(v)[q] = ov;
+    }
+  }
+}
+
+// out[x] = (add ? out[x] : 0) + sum over y < ny of part[y * cnt + x], in a fixed
+// order: 16 outputs a workgroup, 16 threads each take every 16th y (eight loads
+// in flight), so that the chain of dependent loads is a 16th of ny (8192 outputs of
+// 2048 rows: 21 us = 6.4 TB/s, one thread per output 800; 10240 of 64: 2.7, 17).
+constexpr int SUM_X = 16, SUM_Y = WG / SUM_X;
+__global__ __launch_bounds__(WG) void k_sum_parts(const double* __restrict__ part, int ny,
+                                                  size_t cnt, double* __restrict__ out, int add) {
+  __shared__ double red[SUM_Y][SUM_X + 1];
+  const int tx = threadIdx.x % SUM_X, ty = threadIdx.x / SUM_X;
+  for (size_t x0 = (size_t)blockIdx.x * SUM_X; x0 < cnt; x0 += (size_t)gridDim.x * SUM_X) {
+    const size_t x = x0 + tx;
+    double s = 0.0;
+    if (x < cnt) {
+#pragma unroll 8
+      for (int y = ty; y < ny; y += SUM_Y) s += part[(size_t)y * cnt + x];
+    }
+    __syncthreads();
+    red[ty][tx] = s;
+    __syncthreads();
+    if (ty == 0 && x < cnt) {
+      double t = add ? out[x] : 0.0;
+#pragma unroll
+      for (int k = 0; k < SUM_Y; k++) t += red[k][tx];
+      out[x] = t;
+    }
   }
 }
 

@@ -576,16 +576,6 @@ __global__ __launch_bounds__(WG) void k_res_outer(const int* __restrict__ drp,
   for (int e = 0; e < NH; e++) o[e] = acc[e];
 }
 
-// dacc[e] = sum_y part[y][e], in order.
-__global__ __launch_bounds__(WG) void k_res_outer_sum(const double* __restrict__ part, int ny,
-                                                      size_t cnt, double* __restrict__ dacc) {
-  for (size_t e = (size_t)blockIdx.x * WG + threadIdx.x; e < cnt; e += (size_t)gridDim.x * WG) {
-    double s = 0.0;
-    for (int y = 0; y < ny; y++) s += part[(size_t)y * cnt + e];
-    dacc[e] = s;
-  }
-}
-
 // n doubles from pinned host memory (the coefficients of a call).
 __global__ __launch_bounds__(WG) void k_res_coef(const double* __restrict__ src,
                                                  double* __restrict__ dst, int n) {
