@@ -182,12 +182,14 @@ __global__ __launch_bounds__(WG) void k_batch_aux(const SlotDev* __restrict__ sd
   const size_t t0 = (size_t)wid.k * WG + threadIdx.x, tstride = (size_t)wid.n * WG;
   if (step == 0) {
     for (size_t e = t0; e < 2 * delem; e += tstride) d.dacc[e] = 0.0;
-  } else if (step == h) {
-    outer_dev<S, S, S, true, B, L, KQ>(wid, rp, d.ci, (const S*)d.R, (const S*)d.R, d.dacc, d.nb,
-                                       d.qp, d.chunk, d.diag);
-  } else if (step == d.M && d.M > 2) {
-    outer_dev<S, S, S, true, B, L, KQ>(wid, rp, d.ci, (const S*)d.A[0], (const S*)d.Bv[1], d.dacc,
-                                       d.nb, d.qp, d.chunk, 1.0);
+  } else if (step == h || (step == d.M && d.M > 2)) {
+    const S* a = (const S*)(step == h ? d.R : d.A[0]);
+    const S* b = (const S*)(step == h ? d.R : d.Bv[1]);
+    const double f = step == h ? d.diag : 1.0;
+    if constexpr (MF >= 1)  // pass widths of 8 and 16 packets
+      mfma_outer_dev<S>(wid, rp, d.ci, a, b, d.dacc, d.nb, d.qp, d.chunk, f);
+    else
+      outer_dev<S, S, S, true, B, L, KQ>(wid, rp, d.ci, a, b, d.dacc, d.nb, d.qp, d.chunk, f);
   } else if (step == d.M + 1) {
     // D_out = ((D + D^+) / 2) / mag on the block pattern (symmetrize + scale)
     for (size_t e = t0; e < delem; e += tstride) {

@@ -1227,6 +1227,23 @@ int sum_parts(fkpm_handle* h, const double* part, int ny, size_t cnt, double* ou
                 dim3(fkd::WG), h->stream, part, ny, cnt, out, add ? 1 : 0);
 }
 
+// dacc += f A B^+ on D's pattern: complex 8x8 blocks on the matrix cores (us, vector
+// units / matrix cores: 32^3 sites, S = 256 FP32 4384 / 1264; 18x15x13, S = 144 FP64
+// 286 / 175).
+template <class S>
+int add_outer(fkpm_handle* h, const S* A, const S* B, double f) {
+  const auto& ks = h->ks<S>(K_OUT);
+  KCfg c = h->kc[K_OUT];
+  auto fn = ks.outer_ss;
+  if (mfma_avail(h, K_AD) && h->qp % (4 * fkd::MO_U) == 0) {
+    fn = ks.mfma_outer;
+    c.L = fkd::WAVE;  // one wave per block row
+    derive_grid(h->nb, c);
+  }
+  return launch(fn, dim3(c.nwg), dim3(fkd::WG), h->stream, h->drp.as<const int>(),
+                h->dci.as<const int>(), A, B, h->dacc.as<double>(), h->nb, h->qp, c.chunk, f);
+}
+
 // ---------------------------------------------------------------------------
 // Whole-recursion kernels of small lattices (kpm_resident.h): moments,
 // autodiff_matrix and stoch_matrix as one launch per recursion.
@@ -1733,12 +1750,8 @@ int stoch_t(fkpm_handle* h, int M, const double* c) {
     CHK(timing_end(h, &h->ms_stoch, &h->n_stoch, launches));
     CHK(zero_doubles(h, h->dacc.p, dcount));
     // D = (1/2) R xi^+ + (1/2) xi R^+
-    CHK(launch(kso.outer_ss, dim3(ko.nwg), block, h->stream, h->drp.as<const int>(),
-               h->dci.as<const int>(), (const S*)h->R.p, xi, h->dacc.as<double>(), h->nb, h->qp,
-               ko.chunk, 0.5));
-    CHK(launch(kso.outer_ss, dim3(ko.nwg), block, h->stream, h->drp.as<const int>(),
-               h->dci.as<const int>(), xi, (const S*)h->R.p, h->dacc.as<double>(), h->nb, h->qp,
-               ko.chunk, 0.5));
+    CHK(add_outer<S>(h, (const S*)h->R.p, xi, 0.5));
+    CHK(add_outer<S>(h, xi, (const S*)h->R.p, 0.5));
   } else {
     // the reference's order: forward recursion, xi accumulated in FP64
     CHK(h->xi.ensure(h->accbytes()));
@@ -1800,15 +1813,11 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
   const dim3 block(fkd::WG);
   const KCfg& ka = h->kc[K_AD];
   const KCfg& kt = h->kc[K_ADS];
-  const KCfg& ko = h->kc[K_OUT];
   const auto& ksa = h->ks<S>(K_AD);
   const auto& kst = h->ks<S>(K_ADS);
-  const auto& kso = h->ks<S>(K_OUT);
   const int* rp = h->rp.as<const int>();
   const int* ci = h->ci.as<const int>();
   const S* hv = h->hv.as<const S>();
-  const int* drp = h->drp.as<const int>();
-  const int* dci = h->dci.as<const int>();
   double* dacc = h->dacc.as<double>();
   const size_t dcount = (size_t)h->nnzbD * h->b * h->b * (h->cx ? 2 : 1);
 
@@ -1820,8 +1829,7 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
   }
   CHK(zero_doubles(h, dacc, dcount));
   // D = diag R R^+
-  CHK(launch(kso.outer_ss, dim3(ko.nwg), block, h->stream, drp, dci, (const S*)h->vec_a(0),
-             (const S*)h->vec_a(0), dacc, h->nb, h->qp, ko.chunk, diag));
+  CHK(add_outer<S>(h, (const S*)h->vec_a(0), (const S*)h->vec_a(0), diag));
   int launches = 0;
   if (M > 2)
     for (int k = 0; k < 3; k++) CHK(h->Bv[k].ensure(h->vbytes()));
@@ -1846,8 +1854,7 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
       const double w = m > 1 ? 2 * c[2 * m - 1] : 0.0;
       if (stored) {
         if (!h->d_fused)  // D += 2 alpha_m beta_{m+1}^+ on D's own pattern
-          CHK(launch(kso.outer_ss, dim3(ko.nwg), block, h->stream, drp, dci, am, first ? am : bm1,
-                     dacc, h->nb, h->qp, ko.chunk, first ? 2.0 * sb : 2.0));
+          CHK(add_outer<S>(h, am, first ? am : bm1, first ? 2.0 * sb : 2.0));
         CHK(launch(h->d_fused ? ads_fn(h, kst, kt) : adsp_fn(kst, kt), dim3(kt.nwg), block,
                    h->stream, rp_for(h, kt), ci, hv, am, am1, bm1, bm2, (const S*)aout, bout, dacc,
                    h->nb, h->qp, kt.chunk, c4, c2, w, sb, sb2, 2.0, kt.nt));
@@ -1857,8 +1864,7 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
                    aout, bout, dacc, h->nb, h->qp, ka.chunk, c4, c2, w, sb, sb2, 2.0, ka.nt));
       } else {
         // D += 2 alpha_m beta_{m+1}^+ on D's own pattern, then the step.
-        CHK(launch(kso.outer_ss, dim3(ko.nwg), block, h->stream, drp, dci, am, first ? am : bm1,
-                   dacc, h->nb, h->qp, ko.chunk, first ? 2.0 * sb : 2.0));
+        CHK(add_outer<S>(h, am, first ? am : bm1, first ? 2.0 * sb : 2.0));
         CHK(launch(adp_fn(ksa, ka), dim3(ka.nwg), block, h->stream, rp_for(h, ka), ci, hv, am, am1,
                    bm1, bm2,
                    aout, bout, dacc, h->nb, h->qp, ka.chunk, c4, c2, w, sb, sb2, 2.0, ka.nt));
@@ -1866,9 +1872,7 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
       launches++;
     }
     // D += alpha_0 beta_1^+ (alpha_0 = R kept, or recomputed into A[0])
-    CHK(launch(kso.outer_ss, dim3(ko.nwg), block, h->stream, drp, dci,
-               (const S*)(stored ? h->vec_a(0) : h->A[0].p), (const S*)h->Bv[1].p, dacc, h->nb,
-               h->qp, ko.chunk, 1.0));
+    CHK(add_outer<S>(h, (const S*)(stored ? h->vec_a(0) : h->A[0].p), (const S*)h->Bv[1].p, 1.0));
   }
   CHK(rec.run());
   CHK(timing_end(h, &h->ms_ad, &h->n_ad, launches));

@@ -79,6 +79,9 @@ struct KSet {
   void (*mfma_ads[6])(const int*, const int*, const S*, const S*, const S*, const S*, const S*,
                       const S*, S*, double*, int, int, int, double, double, double, double, double,
                       double, int) = {};
+  // outer_ss on the matrix cores (padded width a multiple of 8 packets)
+  void (*mfma_outer)(const int*, const int*, const S*, const S*, double*, int, int, int,
+                     double) = nullptr;
   int B = 0, L = 0, KQ = 0;
 };
 

@@ -1334,4 +1334,98 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(3))) void k_
                                       w, sb, sb2, dscale);
 }
 
+// ---------------------------------------------------------------------------
+// Outer product on D's pattern: D_ij += f A_i B_j^+ (the start and the end of
+// autodiff_matrix, and stoch_matrix), complex 8x8 blocks.
+//
+// One wave per D block row.  Lane (g, r) = (lane / 16, lane % 16) loads packet
+// q + g of orbital r % 8 (16 bytes, 64 contiguous bytes a row and instruction)
+// and feeds its real (r < 8) or imaginary part as operand row r: the order of
+// the columns in the K dimension is free as long as A and B share it.  Products
+// and sums in FP64 for both storage types.  On the vector units each of the 128
+// sums of a block is reduced over the lanes by itself: 32^3 sites x 8, S = 256 FP32
+// 4384 us a call, here 1264; 18x15x13 x 8, S = 144 FP64 286 and 175.  Bound: L1 reads
+// (a packet is read by the lanes of both parts) beside the FP64 matrix cores
+// (FP32: 440 us of products, 200 of HBM).
+// ---------------------------------------------------------------------------
+constexpr int MO_G = 4;  // D blocks per pass over the columns
+constexpr int MO_U = 2;  // packets per lane in flight for each of them
+
+template <typename S>
+__device__ __forceinline__ void mfma_outer_dev(WgId wid, const int* __restrict__ drp,
+                                               const int* __restrict__ dci,
+                                               const S* __restrict__ A, const S* __restrict__ Bm,
+                                               double* __restrict__ dacc, int nb, int qp, int chunk,
+                                               double f) {
+  typedef typename Vec16<S>::V VT;
+  constexpr int NS = Vec16<S>::N;
+  const int lane = threadIdx.x & (WAVE - 1);
+  const int g = lane >> 4, r = lane & 15;
+  const bool im = r >= 8;
+  const RowRange rr = wg_rows(nb, chunk, WG / WAVE, wid);
+  const size_t rs = (size_t)qp * NS;
+  const size_t lo = (size_t)(r & 7) * rs + (size_t)g * NS;
+  for (int base = rr.r0; base < rr.r1; base += rr.stride) {
+    const int i = __builtin_amdgcn_readfirstlane(base + (int)(threadIdx.x / WAVE));
+    if (i >= rr.r1) continue;
+    const int p0 = drp[i], p1 = drp[i + 1];
+    const S* a = A + (size_t)8 * i * rs + lo;
+    for (int pb = p0; pb < p1; pb += MO_G) {
+      const S* b[MO_G];
+      dv4 acc[MO_G];
+#pragma unroll
+      for (int k = 0; k < MO_G; k++) {  // a slot past the row's end repeats its last block
+        b[k] = Bm + (size_t)8 * dci[min(pb + k, p1 - 1)] * rs + lo;
+        acc[k] = dv4{0.0, 0.0, 0.0, 0.0};
+      }
+      for (int q = 0; q < qp; q += 4 * MO_U) {
+        VT xa[MO_U], xb[MO_G][MO_U];
+#pragma unroll
+        for (int u = 0; u < MO_U; u++) {
+          const size_t o = (size_t)(q + 4 * u) * NS;
+          xa[u] = *reinterpret_cast<const VT*>(a + o);
+#pragma unroll
+          for (int k = 0; k < MO_G; k++) xb[k][u] = *reinterpret_cast<const VT*>(b[k] + o);
+        }
+#pragma unroll
+        for (int u = 0; u < MO_U; u++)
+#pragma unroll
+          for (int e = 0; e < NS; e += 2) {
+            const double av = (double)(im ? xa[u][e + 1] : xa[u][e]);
+#pragma unroll
+            for (int k = 0; k < MO_G; k++)
+              acc[k] = Mfma<double>::mac(av, (double)(im ? xb[k][u][e + 1] : xb[k][u][e]), acc[k]);
+          }
+      }
+      // Lane (g, r) holds rows g, g + 4, g + 8, g + 12 of column r of the real
+      // 16 x 16 product: r < 8 forms the entry of orbitals (g, r), r >= 8 the one of
+      // (g + 4, r - 8), each with two values of the other lane.
+#pragma unroll
+      for (int k = 0; k < MO_G; k++) {
+        const double v0 = __shfl_xor(im ? acc[k][0] : acc[k][1], 8, WAVE);
+        const double v1 = __shfl_xor(im ? acc[k][2] : acc[k][3], 8, WAVE);
+        if (pb + k >= p1) continue;
+        const double re = im ? v0 + acc[k][3] : acc[k][0] + v1;
+        const double ig = im ? v1 - acc[k][1] : acc[k][2] - v0;
+        double2* d = reinterpret_cast<double2*>(dacc) + (size_t)(pb + k) * 64 + (r & 7) * 8 +
+                     (im ? g + 4 : g);
+        double2 t = *d;
+        t.x = fma(f, re, t.x);
+        t.y = fma(f, ig, t.y);
+        *d = t;
+      }
+    }
+  }
+}
+
+template <typename S>
+__global__ __launch_bounds__(WG) void k_mfma_outer(const int* __restrict__ drp,
+                                                   const int* __restrict__ dci,
+                                                   const S* __restrict__ A,
+                                                   const S* __restrict__ Bm,
+                                                   double* __restrict__ dacc, int nb, int qp,
+                                                   int chunk, double f) {
+  mfma_outer_dev<S>(wg_self(), drp, dci, A, Bm, dacc, nb, qp, chunk, f);
+}
+
 }  // namespace fkd

@@ -147,3 +147,31 @@ def test_set_H_arrays_are_free_on_return(oracle, shapes):
         H.val[:] = 1e30
         assert rel_err(eng.moments(12), want) < 1e-10
     eng.close()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("S", [1, 16, 17, 48, 130])
+def test_matrix_core_outer_product(oracle, S, prec):
+    """stoch_matrix of 8x8 blocks on a D pattern of its own: rows of 0 to 9 blocks
+    (groups of four and their remainders), one column to several passes."""
+    from fastkpm_amd import EnergyScale, HipEngine, lattice
+    H = lattice.lattice((4, 3, 3), b=8, orbital_blocks=True, seed=S)
+    nb = H.n_rows
+    rng = np.random.default_rng(S)
+    rows = np.repeat(np.arange(nb), np.arange(nb) % 10)
+    cols = np.concatenate([rng.choice(nb, k % 10, replace=False) for k in range(nb)])
+    D = lattice.coo_to_bsr(nb, 8, rows, cols, np.zeros((len(rows), 8, 8)))
+    R = rng.standard_normal((nb * 8, S)) + 1j * rng.standard_normal((nb * 8, S))
+    M = 6
+    c = 1.0 / (1.0 + np.arange(M))
+    bound = float(np.abs(np.linalg.eigvalsh(H.to_dense())).max()) * 1.01
+    eng = HipEngine("cx_double", prec)
+    eng.set_R(R)
+    eng.set_H(H, EnergyScale(-bound, bound))
+    orc = oracle.Engine()
+    orc.set_H(H, -bound, bound)
+    orc.set_R(R)
+    eng.stoch_matrix(c, D)
+    want = orc.stoch_matrix(c, D)
+    assert rel_err(D.val, want) < (1e-10 if prec == "fp64" else M * 16 * 2.0 ** -24)
+    eng.close()
