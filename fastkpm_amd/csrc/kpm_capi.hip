@@ -1273,6 +1273,29 @@ bool find_res(fkpm_handle* h, int rpt) {
 size_t res_count(const fkpm_handle* h) { return (size_t)h->n * h->s * (h->cx ? 2 : 1); }
 size_t res_slot(const fkpm_handle* h) { return (res_count(h) + 63) / 64 * 64; }
 
+template <class S>
+size_t res_lds(fkpm_handle* h) {
+  return 2 * (((size_t)(h->nb + 1) * h->rset<S>().elem_bytes + 15) / 16 * 16);
+}
+
+// The backward recursion's kernel: the thread's rows of the forward vectors in
+// registers where the whole of H still fits beside them, else in LDS where
+// four buffers fit (autodiff_matrix of M = 128, us, registers / LDS: 45x42 x 2 FP32 272 /
+// 253, 35x36 x 2 FP64 534 / 439, 50x50 x 1 510 / 421, 15^3 x 1 real 422 / 354, 8^3 x 4 FP32
+// 331 / 261, FP64 663 / 602).
+struct ResBwd {
+  int st, la;  // some blocks streamed; forward vectors in LDS
+  size_t lds;
+};
+
+template <class S>
+ResBwd res_bwd(fkpm_handle* h) {
+  const fkd::ResSet<S>& rs = h->rset<S>();
+  const size_t lds = res_lds<S>(h);
+  const int la = h->max_deg > rs.dreg_bwd[0][0] && 2 * lds <= kLdsBytes;
+  return ResBwd{h->max_deg > rs.dreg_bwd[0][la], la, la ? 2 * lds : lds};
+}
+
 // Whether the whole-recursion kernels run for the current H and R: the
 // defaults of every switch that names a step kernel or the table (a forced
 // geometry, sweep, order, graph or table mode asks for the step kernels), and a
@@ -1291,8 +1314,9 @@ bool res_wanted(fkpm_handle* h) {
   const fkd::ResSet<S>& rs = h->rset<S>();
   if (2 * ((size_t)(h->nb + 1) * rs.elem_bytes + 16) > kLdsBytes) return false;
   const int threads = ((h->nb + rpt - 1) / rpt + 63) / 64 * 64;
-  if (h->max_deg > rs.dreg_bwd[0]) {
-    const int d = h->max_deg - rs.dreg_bwd[1];
+  const ResBwd rb = res_bwd<S>(h);
+  if (rb.st) {
+    const int d = h->max_deg - rs.dreg_bwd[1][rb.la];
     if ((size_t)d * (rs.block_bytes + 4) * h->nb > kResStream) return false;
   }
   if (rpt != h->res.rpt || threads != h->res.threads) h->res.packed = false;
@@ -1343,11 +1367,6 @@ int res_pack(fkpm_handle* h) {
                h->res.hval.as<S>(), h->res.hoff.as<int>()));
   h->res.packed = true;
   return 0;
-}
-
-template <class S>
-size_t res_lds(fkpm_handle* h) {
-  return 2 * (((size_t)(h->nb + 1) * h->rset<S>().elem_bytes + 15) / 16 * 16);
 }
 
 // Coefficients to the device: pinned memory, read by a kernel on the stream.
@@ -1429,7 +1448,8 @@ int res_autodiff(fkpm_handle* h, int M, const double* c, double diag) {
   CHK(timing_begin(h));
   if (M2 > 1) {
     CHK(res_coef(h, c, M));
-    CHK(launch_lds(rs.bwd[h->max_deg > rs.dreg_bwd[0]], dim3(h->s), dim3(h->res.threads), res_lds<S>(h), h->stream,
+    const ResBwd rb = res_bwd<S>(h);
+    CHK(launch_lds(rs.bwd[rb.st][rb.la], dim3(h->s), dim3(h->res.threads), rb.lds, h->stream,
                    res_H<S>(h), h->res.atab.as<const S>(), h->res.btab.as<S>(), slot, M2,
                    h->res.coef.as<const double>(), 2 * c[M - 1]));
   }

@@ -49,6 +49,10 @@ struct ResGeo {
   }
 };
 constexpr int RES_VL_FWD = 2, RES_VL_XI = 2, RES_VL_BWD = 5;
+// FP64 with streamed blocks keeps the registers of one more vector free: 9^3 x 2
+// (two rows a thread) streamed two blocks of seven slower than three.
+template <typename S, bool ST>
+constexpr int RES_VL_BWD_LA = ST && sizeof(S) == 8 ? 3 : 2;
 
 // N scalars at p (16-byte packets where the size allows; a smaller element is
 // one access).
@@ -310,8 +314,11 @@ __global__ __launch_bounds__(RES_T) void k_res_forward(ResH<S> H, const S* __res
 //   beta_m = 2 Hs beta_{m+1} - beta_{m+2} + 4 c_{2m} alpha_m
 //            + 2 c_{2m+1} alpha_{m+1} + 2 c_{2m-1} alpha_{m-1} (m > 1)
 // into slots m = M2-1 .. 1 of btab, with beta_{M2} = sb alpha_{M2-1} kept
-// virtual (the first step scales its product).
-template <typename S, bool CX, int B, int RPT, bool ST>
+// virtual (the first step scales its product).  The thread's rows of alpha_m and
+// alpha_{m+1} stay in registers, or (LA) in two more LDS buffers, which leaves
+// the registers of three vectors to blocks of H (45x42 x 2 FP32: all of it, 2.7 ->
+// 2.4 us a step).
+template <typename S, bool CX, int B, int RPT, bool ST, bool LA>
 __global__ __launch_bounds__(RES_T) void k_res_backward(ResH<S> H, const S* __restrict__ tab,
                                                         S* __restrict__ btab, size_t slot, int M2,
                                                         const double* __restrict__ c, double sb) {
@@ -320,15 +327,21 @@ __global__ __launch_bounds__(RES_T) void k_res_backward(ResH<S> H, const S* __re
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int bufb = res_buf_bytes<GE::BYTES>(H.nb);
   const size_t col = (size_t)blockIdx.x * H.nb * NV;
-  ResRegs<S, CX, B, RPT, RES_VL_BWD, ST> G;
+  ResRegs<S, CX, B, RPT, LA ? RES_VL_BWD_LA<S, ST> : RES_VL_BWD, ST> G;
   G.load(H);
-  S ai[RPT][NV], a1[RPT][NV];
+  S ai[LA ? 1 : RPT][NV], a1[LA ? 1 : RPT][NV];
 #pragma unroll
   for (int k = 0; k < RPT; k++) {
     const int i = min((int)(k * blockDim.x + threadIdx.x), H.nb - 1);
-    ldn<S, NV>(tab + (size_t)(M2 - 1) * slot + col + (size_t)i * NV, ai[k]);
-    ldn<S, NV>(tab + (size_t)M2 * slot + col + (size_t)i * NV, a1[k]);
-    stn<S, NV>(reinterpret_cast<S*>(lds + i * GE::BYTES), ai[k]);  // clamped rows: the same value
+    S(&t)[NV] = ai[LA ? 0 : k], (&t1)[NV] = a1[LA ? 0 : k];
+    ldn<S, NV>(tab + (size_t)(M2 - 1) * slot + col + (size_t)i * NV, t);
+    ldn<S, NV>(tab + (size_t)M2 * slot + col + (size_t)i * NV, t1);
+    // clamped rows: the same value
+    stn<S, NV>(reinterpret_cast<S*>(lds + i * GE::BYTES), t);
+    if constexpr (LA) {
+      stn<S, NV>(reinterpret_cast<S*>(lds + 2 * bufb + i * GE::BYTES), t);
+      stn<S, NV>(reinterpret_cast<S*>(lds + 3 * bufb + i * GE::BYTES), t1);
+    }
   }
   res_zero_block<S, B, RPT, NV>(lds, H.nb, bufb);
   __syncthreads();
@@ -346,6 +359,8 @@ __global__ __launch_bounds__(RES_T) void k_res_backward(ResH<S> H, const S* __re
     }
     const char* xb = lds + q * bufb;
     char* yb = lds + (q ^ 1) * bufb;  // holds beta_{m+2}
+    const char* ab = lds + (2 + q) * bufb;      // LA: alpha_m
+    char* a1b = lds + (2 + (q ^ 1)) * bufb;     // LA: alpha_{m+1}, then alpha_{m-1}
     S acc[RPT][NV];
     G.mul(H, xb, acc);
     S* out = btab + (size_t)m * slot + col;
@@ -354,19 +369,28 @@ __global__ __launch_bounds__(RES_T) void k_res_backward(ResH<S> H, const S* __re
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
       const int i = k * blockDim.x + threadIdx.x;
+      S(&t)[NV] = ai[LA ? 0 : k], (&t1)[NV] = a1[LA ? 0 : k];
+      if constexpr (LA) {
+        const int o = min(i, H.nb - 1) * GE::BYTES;
+        ldn<S, NV>(reinterpret_cast<const S*>(ab + o), t);
+        ldn<S, NV>(reinterpret_cast<const S*>(a1b + o), t1);
+      }
 #pragma unroll
       for (int e = 0; e < NV; e++) {
-        const S b2 = first || second ? asb2 * a1[k][e] : y[k][e];
+        const S b2 = first || second ? asb2 * t1[e] : y[k][e];
         S v = fma(ab2, acc[k][e], -b2);
-        v = fma(ac4, ai[k][e], v);
-        v = fma(ac2, a1[k][e], v);
+        v = fma(ac4, t[e], v);
+        v = fma(ac2, t1[e], v);
         y[k][e] = fma(aw, an[k][e], v);
-        a1[k][e] = ai[k][e];
-        ai[k][e] = an[k][e];
+        if constexpr (!LA) {
+          t1[e] = t[e];
+          t[e] = an[k][e];
+        }
       }
       if (i < H.nb) {
         stn<S, NV>(reinterpret_cast<S*>(yb + i * GE::BYTES), y[k]);
         stn<S, NV>(out + (size_t)i * NV, y[k]);
+        if constexpr (LA) stn<S, NV>(reinterpret_cast<S*>(a1b + i * GE::BYTES), an[k]);
       }
     }
     __syncthreads();
@@ -591,9 +615,10 @@ template <class S>
 struct ResSet {
   void (*pack)(const int*, const int*, const S*, int, int, int, S*, int*) = nullptr;
   void (*fwd[2])(ResH<S>, const S*, int, S*, size_t, int) = {};
-  void (*bwd[2])(ResH<S>, const S*, S*, size_t, int, const double*, double) = {};
+  // second index 1: own rows of alpha in LDS (four buffers instead of two)
+  void (*bwd[2][2])(ResH<S>, const S*, S*, size_t, int, const double*, double) = {};
   void (*xi[2])(ResH<S>, const S*, int, const S*, const S*, const double*, int, S*, S*) = {};
-  int dreg_fwd[2] = {}, dreg_bwd[2] = {}, dreg_xi[2] = {};
+  int dreg_fwd[2] = {}, dreg_bwd[2][2] = {}, dreg_xi[2] = {};
   int elem_bytes = 0;   // one block row of one column
   int block_bytes = 0;  // one H block
 };
