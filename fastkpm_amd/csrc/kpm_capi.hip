@@ -348,8 +348,10 @@ struct fkpm_handle {
   PinBuf psum;             // moment sums, written by the reducing kernel
   int alpha_M = 0;  // M of the moments whose final state is held, 0 if none
   DevBuf atab;            // alpha_1 .. alpha_{M/2} of the last moments(M), when it fits
-  bool a_stored = false;  // the forward vectors live in atab (else the ring A[3])
-  int tab_K = 0;          // atab holds alpha_1 .. alpha_tab_K of the current H and R
+  int a_slots = 0;        // moments state: alpha_1 .. alpha_{a_slots} live in atab, later ones
+                          // in the ring A[3]
+  int tab_K = 0;          // atab holds alpha_1 .. alpha_tab_K of the current H and R,
+  int tab_M = 0;          // kept by moments(tab_M)
   DevBuf tabc;            // stoch_matrix weights of the table vectors
   std::vector<double> tabc_host;
   int store_alpha = 1;    // FKPM_OPT_STORE_ALPHA: 0 never, 1 auto, 2 whenever the table fits
@@ -426,11 +428,11 @@ struct fkpm_handle {
   size_t vbytes() const { return (size_t)n * sp * (cx ? 2 : 1) * (single ? 4 : 8); }
   size_t accbytes() const { return (size_t)n * sp * (cx ? 2 : 1) * 8; }
   int ne() const { return (single ? 4 : 2) / (cx ? 2 : 1); }  // elements per 16-byte packet
-  // forward-phase alpha_k: R, then the table of every alpha_k (a_stored) or
-  // the ring of three
+  // forward-phase alpha_k: R, then the table's alpha_1 .. alpha_{a_slots}, then the
+  // ring of three
   void* vec_a(int k) {
     if (k == 0) return R.p;
-    if (a_stored) return static_cast<char*>(atab.p) + (size_t)(k - 1) * vbytes();
+    if (k <= a_slots) return static_cast<char*>(atab.p) + (size_t)(k - 1) * vbytes();
     return A[k % 3].p;
   }
   template <class S>
@@ -1208,16 +1210,16 @@ void stoch_table_weights(int M, const double* c, std::vector<double>& w) {
   }
 }
 
-// u, v of stoch_matrix from K table slots of n scalars (k_table_sums).
-template <class S>
-int table_sums(fkpm_handle* h, const S* R, const S* tab, size_t n, int K, const double* d,
-               const double* e, S* u, S* v) {
+// The NO sums of stoch_matrix from K table slots of n scalars (k_table_sums).
+template <class S, int NO>
+int table_sums(fkpm_handle* h, const S* R, const S* tab, size_t n, int K, const double* w, S* o0,
+               S* o1, S* o2 = nullptr) {
   const size_t np = n * sizeof(S) / 16;
   if (np <= kSumsSplit)
-    return launch(&fkd::k_table_sums<S, 8>, dim3((unsigned)((np + 31) / 32)), dim3(fkd::WG),
-                  h->stream, R, tab, n, K, d, e, u, v, n);
-  return launch(&fkd::k_table_sums<S, 1>, dim3(4096), dim3(fkd::WG), h->stream, R, tab, n, K, d, e,
-                u, v, n);
+    return launch(&fkd::k_table_sums<S, 8, NO>, dim3((unsigned)((np + 31) / 32)), dim3(fkd::WG),
+                  h->stream, R, tab, n, K, w, o0, o1, o2, n);
+  return launch(&fkd::k_table_sums<S, 1, NO>, dim3(4096), dim3(fkd::WG), h->stream, R, tab, n, K, w,
+                o0, o1, o2, n);
 }
 
 // out = (add ? out : 0) + the ny rows of part, cnt values each (k_sum_parts).
@@ -1242,6 +1244,23 @@ int add_outer(fkpm_handle* h, const S* A, const S* B, double f) {
   }
   return launch(fn, dim3(c.nwg), dim3(fkd::WG), h->stream, h->drp.as<const int>(),
                 h->dci.as<const int>(), A, B, h->dacc.as<double>(), h->nb, h->qp, c.chunk, f);
+}
+
+// Weights of the table vectors where the table holds a third of the orders
+// (stoch_table3, K = ceil(M/3)): v, w_1, w_2.
+void stoch_table3_weights(int M, const double* c, std::vector<double>& w) {
+  const int K = (M + 2) / 3, n = K + 1;
+  std::vector<double> a(3 * (size_t)K, 0.0);  // coefficients of T_{jK+i} at j K + i
+  std::copy(c, c + M, a.begin());
+  w.assign(3 * (size_t)n, 0.0);
+  for (int j = 2; j >= 1; j--) {
+    w[j * n] = a[j * K];
+    for (int i = 1; i < K; i++) {
+      w[j * n + i] = 2 * a[j * K + i];
+      a[(j - 1) * K + K - i] -= a[j * K + i];
+    }
+  }
+  for (int i = 0; i < K; i++) w[i] = a[i] - w[2 * n + i];
 }
 
 // ---------------------------------------------------------------------------
@@ -1407,7 +1426,7 @@ int res_moments(fkpm_handle* h, int M, double* mu, bool* done) {
   moments_from_sums(ps, nsteps, mu);
   h->res.K = nsteps;
   h->res.state = true;
-  h->a_stored = false;
+  h->a_slots = 0;
   h->alpha_M = M;
   *done = true;
   return 0;
@@ -1474,8 +1493,8 @@ int res_stoch(fkpm_handle* h, int M, const double* c, bool table) {
   if (table) {
     stoch_table_weights(M, c, w);
     CHK(res_coef(h, w.data(), (int)w.size()));
-    CHK(table_sums<S>(h, h->res.atab.as<const S>(), h->res.atab.as<const S>() + slot, slot, K,
-                      h->res.coef.as<const double>(), h->res.coef.as<const double>() + K + 1, u, v));
+    CHK((table_sums<S, 2>(h, h->res.atab.as<const S>(), h->res.atab.as<const S>() + slot, slot, K,
+                          h->res.coef.as<const double>(), v, u)));
   } else {
     CHK(res_coef(h, c, M));
   }
@@ -1499,11 +1518,14 @@ int moments_t(fkpm_handle* h, int M, double* mu) {
   }
   h->res.state = false;
   CHK(ensure_partials(h, nsteps));
-  // keep every alpha_k for autodiff_matrix (no backward recomputation of
-  // alpha) when wanted (table_wanted) and the table fits half the free device
-  // memory (or the byte count in FKPM_ALPHA_TABLE_BYTES).
+  // Keep the alpha_k for autodiff_matrix (no backward recomputation of alpha) and
+  // stoch_matrix when wanted (table_wanted): all of them where the table fits
+  // half the free device memory (or the byte count in FKPM_ALPHA_TABLE_BYTES),
+  // else as many as fit from a third of M on, the first ones (64^3 x 2 FP64, S = 128,
+  // M = 160, 67 of 80 kept: moments + autodiff_matrix + stoch_matrix 305 -> 258 ms).
   {
-    const size_t need = (size_t)nsteps * h->vbytes();
+    const size_t vb = h->vbytes(), need = (size_t)nsteps * vb;
+    const int least = (M + 2) / 3;
     // default: half of what is free (the table already held counts as free),
     // never more than a quarter of the device, so that other engines and a
     // batch arena on the same device keep room whatever the order of calls
@@ -1515,41 +1537,48 @@ int moments_t(fkpm_handle* h, int M, double* mu) {
     }
     if (h->table_cap_mb >= 0) budget = (size_t)h->table_cap_mb << 20;
     if (const char* e = getenv("FKPM_ALPHA_TABLE_BYTES")) budget = (size_t)strtoull(e, nullptr, 10);
-    h->a_stored = false;
-    if (table_wanted(h) && need <= budget) {
+    size_t slots = std::min<size_t>(budget / vb, nsteps);
+    // a held table that serves is not grown for a few slots more
+    if (slots < (size_t)nsteps && h->atab.bytes / vb >= (size_t)least)
+      slots = std::min(slots, h->atab.bytes / vb);
+    h->a_slots = 0;
+    if (table_wanted(h) && slots >= (size_t)std::min(least, nsteps)) {
       h->tab_K = 0;  // rewritten below (and lost if the table grows)
-      CHK(h->atab.ensure(need));
-      h->a_stored = true;
+      CHK(h->atab.ensure(slots * vb));
+      h->a_slots = (int)slots;
     }
   }
-  const int kind = h->a_stored ? K_MOMT : K_MOM;
-  const KCfg& kc = h->kc[kind];
-  const auto& ks = h->ks<S>(kind);
-  const dim3 grid(kc.nwg), block(fkd::WG);
+  const dim3 block(fkd::WG);
   CHK(timing_begin(h));
   {
     LoopRecorder rec(h);
-    const int group = partial_steps(nsteps, kc.nwg);
-    for (int m = 0; m < nsteps; m++) {
-      // alpha_{m+1} = cx Hs alpha_m + cz alpha_{m-1}
-      const S* x = (const S*)h->vec_a(m);
-      const S* z = m == 0 ? nullptr : (const S*)h->vec_a(m - 1);
-      S* y = (S*)h->vec_a(m + 1);
-      CHK(launch(mom_fn(h, ks, kc), grid, block, h->stream, rp_for(h, kc),
-                 h->ci.as<const int>(), h->hv.as<const S>(), x, z, y, h->nb, h->qp, kc.chunk,
-                 m == 0 ? 1.0 : 2.0, m == 0 ? 0.0 : -1.0,
-                 h->partial.as<double>() + (size_t)(m % group) * kc.nwg * 2, kc.nt,
-                 no_rsource<S>()));
-      if ((m + 1) % group == 0 || m == nsteps - 1) {
-        const int m0 = m - m % group;
-        CHK(launch(&fkd::k_reduce_partials, dim3(m + 1 - m0), block, h->stream,
-                   (const double*)h->partial.as<double>(), kc.nwg, (double*)h->psum.p + 2 * m0));
+    // alpha_{m+1} = cx Hs alpha_m + cz alpha_{m-1}, into the table, then the ring
+    for (int m0 = 0; m0 < nsteps;) {
+      const int kind = m0 < h->a_slots ? K_MOMT : K_MOM;
+      const KCfg& kc = h->kc[kind];
+      const auto& ks = h->ks<S>(kind);
+      const int m1 = std::min(m0 + partial_steps(nsteps, kc.nwg), kind == K_MOMT ? h->a_slots : nsteps);
+      for (int m = m0; m < m1; m++) {
+        const S* x = (const S*)h->vec_a(m);
+        const S* z = m == 0 ? nullptr : (const S*)h->vec_a(m - 1);
+        S* y = (S*)h->vec_a(m + 1);
+        CHK(launch(mom_fn(h, ks, kc), dim3(kc.nwg), block, h->stream, rp_for(h, kc),
+                   h->ci.as<const int>(), h->hv.as<const S>(), x, z, y, h->nb, h->qp, kc.chunk,
+                   m == 0 ? 1.0 : 2.0, m == 0 ? 0.0 : -1.0,
+                   h->partial.as<double>() + (size_t)(m - m0) * kc.nwg * 2, kc.nt,
+                   no_rsource<S>()));
       }
+      CHK(launch(&fkd::k_reduce_partials, dim3(m1 - m0), block, h->stream,
+                 (const double*)h->partial.as<double>(), kc.nwg, (double*)h->psum.p + 2 * m0));
+      m0 = m1;
     }
     CHK(rec.run());
   }
   CHK(timing_end(h, &h->ms_mom, &h->n_mom, nsteps));
-  if (h->a_stored) h->tab_K = nsteps;
+  if (h->a_slots > 0) {
+    h->tab_K = h->a_slots;
+    h->tab_M = M;
+  }
   HIPCHK(hipStreamSynchronize(h->stream));
   moments_from_sums((const double*)h->psum.p, nsteps, mu);
   h->alpha_M = M;
@@ -1683,6 +1712,32 @@ int stoch_clenshaw(fkpm_handle* h, int M, const double* c, const S** xi_out) {
   return launches + 1;
 }
 
+// f T_K(Hs) x + add for the vector x in A[*slot], by K Chebyshev steps
+// (y_0 = x, y_1 = Hs x, y_{k+1} = 2 Hs y_k - y_{k-1}, the last one scaled by f with
+// `add` as its source); *slot is then the result's place in the ring.
+template <class S>
+int chebyshev_of(fkpm_handle* h, int K, double f, const S* add, int* slot) {
+  const KCfg& kc = h->kc[K_MOM];
+  const auto& ks = h->ks<S>(K_MOM);
+  fkd::RSource<S> src = no_rsource<S>();
+  src.rd = add;
+  src.cr = 1.0;
+  const S* x = (const S*)h->A[*slot].p;
+  const S* z = nullptr;
+  for (int k = 0; k < K; k++) {
+    *slot = (*slot + 1) % 3;
+    S* y = (S*)h->A[*slot].p;
+    const double g = k == K - 1 ? f : 1.0;
+    CHK(launch(mom_fn(h, ks, kc), dim3(kc.nwg), dim3(fkd::WG), h->stream, rp_for(h, kc),
+               h->ci.as<const int>(), h->hv.as<const S>(), x, z, y, h->nb, h->qp, kc.chunk,
+               (k == 0 ? 1.0 : 2.0) * g, k == 0 ? 0.0 : -g, (double*)nullptr, kc.nt,
+               k == K - 1 ? src : no_rsource<S>()));
+    z = x;
+    x = y;
+  }
+  return 0;
+}
+
 // xi from the kept forward vectors alpha_0 .. alpha_K (K = ceil(M/2), coefficients
 // padded with zeros to 2K): by T_{K+j} = 2 T_K T_j - T_{K-j},
 //   xi = sum_{m<2K} c_m T_m(Hs) R = v + 2 T_K(Hs) u,
@@ -1695,48 +1750,53 @@ int stoch_clenshaw(fkpm_handle* h, int M, const double* c, const S** xi_out) {
 template <class S>
 int stoch_table(fkpm_handle* h, int M, const double* c, const S** xi_out) {
   const int K = (M + 1) / 2;
-  const KCfg& kc = h->kc[K_MOM];
-  const auto& ks = h->ks<S>(K_MOM);
-  const dim3 grid(kc.nwg), block(fkd::WG);
-  const size_t vb = h->vbytes();
+  const size_t n = h->vbytes() / sizeof(S);
   std::vector<double>& w = h->tabc_host;
   stoch_table_weights(M, c, w);
   CHK(h->tabc.ensure(w.size() * sizeof(double)));
   HIPCHK(hipMemcpyAsync(h->tabc.p, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice,
                         h->stream));
-  CHK(h->Bv[0].ensure(vb));
+  CHK(h->Bv[0].ensure(h->vbytes()));
   S* u = (S*)h->A[0].p;
   S* v = (S*)h->Bv[0].p;
-  const size_t n = vb / sizeof(S);
-  CHK(table_sums<S>(h, (const S*)h->R.p, (const S*)h->atab.p, n, K, h->tabc.as<const double>(),
-                    h->tabc.as<const double>() + K + 1, u, v));
-  // y_0 = u, y_1 = Hs u, y_{k+1} = 2 Hs y_k - y_{k-1}; the last step writes
-  // 2 y_K + v
-  fkd::RSource<S> addv = no_rsource<S>();
-  addv.rd = v;
-  addv.cr = 1.0;
-  const S* x = u;
-  const S* z = nullptr;
-  int slot = 1;
-  for (int k = 0; k < K; k++) {
-    S* y = (S*)h->A[slot].p;
-    slot = (slot + 1) % 3;
-    const bool last = (k == K - 1);
-    const double cx = (k == 0 ? 1.0 : 2.0) * (last ? 2.0 : 1.0);
-    const double cz = k == 0 ? 0.0 : (last ? -2.0 : -1.0);
-    CHK(launch(mom_fn(h, ks, kc), grid, block, h->stream, rp_for(h, kc),
-               h->ci.as<const int>(), h->hv.as<const S>(), x, z, y, h->nb, h->qp, kc.chunk, cx,
-               cz, (double*)nullptr, kc.nt, last ? addv : no_rsource<S>()));
-    z = x;
-    x = y;
-  }
-  *xi_out = x;
+  CHK((table_sums<S, 2>(h, (const S*)h->R.p, (const S*)h->atab.p, n, K, h->tabc.as<const double>(),
+                        v, u)));
+  int slot = 0;
+  CHK(chebyshev_of<S>(h, K, 2.0, v, &slot));
+  *xi_out = (const S*)h->A[slot].p;
   return K + 1;
+}
+
+// xi from the first forward vectors alpha_0 .. alpha_{K-1} only, K = ceil(M/3)
+// (coefficients padded with zeros to 3K): by T_{jK+i} = 2 T_{jK} T_i - T_{(j-1)K+(K-i)},
+// from j = 2 down,
+//   xi = w_0 + T_K(Hs) w_1 + T_{2K}(Hs) w_2 = (w_0 - w_2) + T_K(Hs) (w_1 + 2 T_K(Hs) w_2),
+// w_j sums of the alpha_i: 2K steps and one pass over K vectors instead of M - 1
+// steps.  Returns xi's buffer.
+template <class S>
+int stoch_table3(fkpm_handle* h, int M, const double* c, const S** xi_out) {
+  const int K = (M + 2) / 3;
+  const size_t n = h->vbytes() / sizeof(S);
+  std::vector<double>& w = h->tabc_host;
+  stoch_table3_weights(M, c, w);
+  CHK(h->tabc.ensure(w.size() * sizeof(double)));
+  HIPCHK(hipMemcpyAsync(h->tabc.p, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice,
+                        h->stream));
+  for (int k = 0; k < 2; k++) CHK(h->Bv[k].ensure(h->vbytes()));
+  S* v = (S*)h->Bv[0].p;
+  S* w1 = (S*)h->Bv[1].p;
+  CHK((table_sums<S, 3>(h, (const S*)h->R.p, (const S*)h->atab.p, n, K, h->tabc.as<const double>(),
+                        v, w1, (S*)h->A[0].p)));
+  int slot = 0;
+  CHK(chebyshev_of<S>(h, K, 2.0, w1, &slot));
+  CHK(chebyshev_of<S>(h, K, 1.0, v, &slot));
+  *xi_out = (const S*)h->A[slot].p;
+  return 2 * K + 1;
 }
 
 template <class S>
 int stoch_t(fkpm_handle* h, int M, const double* c) {
-  h->a_stored = false;  // the forward method's alpha_k go to the ring
+  h->a_slots = 0;  // the forward method's alpha_k go to the ring
   const dim3 block(fkd::WG);
   const int* rp = h->rp.as<const int>();
   const int* ci = h->ci.as<const int>();
@@ -1755,7 +1815,10 @@ int stoch_t(fkpm_handle* h, int M, const double* c) {
   }
   CHK(timing_begin(h));
   const bool table = h->stoch_method == FKPM_STOCH_AUTO && h->tab_K >= (M + 1) / 2;
-  h->stoch_used = table ? FKPM_STOCH_TABLE
+  // a table cut short by the memory, up to the order it was kept for
+  const bool table3 = !table && h->stoch_method == FKPM_STOCH_AUTO && M <= h->tab_M &&
+                      h->tab_K >= (M + 2) / 3;
+  h->stoch_used = table || table3 ? FKPM_STOCH_TABLE
                         : h->stoch_method == FKPM_STOCH_FORWARD ? FKPM_STOCH_FORWARD
                                                                 : FKPM_STOCH_CLENSHAW;
   if (h->stoch_used != FKPM_STOCH_FORWARD) {
@@ -1763,7 +1826,9 @@ int stoch_t(fkpm_handle* h, int M, const double* c) {
     int launches = 0;
     {
       LoopRecorder rec(h);
-      launches = table ? stoch_table<S>(h, M, c, &xi) : stoch_clenshaw<S>(h, M, c, &xi);
+      launches = table    ? stoch_table<S>(h, M, c, &xi)
+                 : table3 ? stoch_table3<S>(h, M, c, &xi)
+                          : stoch_clenshaw<S>(h, M, c, &xi);
       if (launches < 0) return launches;
       CHK(rec.run());
     }
@@ -1857,12 +1922,11 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
   LoopRecorder rec(h);
   if (M > 2) {
     const double sb = 2 * c[M - 1];  // beta_{M/2} = 2 c_{M-1} alpha_{M/2-1}
-    const bool stored = h->a_stored;
     for (int m = M / 2 - 1; m >= 1; m--) {
-      // alpha_m, alpha_{m+1} and alpha_{m-1}: from the table, or the ring with
-      // alpha_{m-1} recomputed by the step
-      const S* am = (const S*)(stored ? h->vec_a(m) : h->A[m % 3].p);
-      const S* am1 = (const S*)(stored ? h->vec_a(m + 1) : h->A[(m + 1) % 3].p);
+      // alpha_{m-1}: from the table, or recomputed into the ring by the step
+      const bool stored = h->a_slots > 0 && m - 1 <= h->a_slots;
+      const S* am = (const S*)h->vec_a(m);
+      const S* am1 = (const S*)h->vec_a(m + 1);
       S* aout = stored ? (S*)h->vec_a(m - 1) : (S*)h->A[(m - 1) % 3].p;
       const bool first = (m == M / 2 - 1);
       const bool second = (m == M / 2 - 2);
@@ -1892,7 +1956,7 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
       launches++;
     }
     // D += alpha_0 beta_1^+ (alpha_0 = R kept, or recomputed into A[0])
-    CHK(add_outer<S>(h, (const S*)(stored ? h->vec_a(0) : h->A[0].p), (const S*)h->Bv[1].p, 1.0));
+    CHK(add_outer<S>(h, (const S*)(h->a_slots > 0 ? h->R.p : h->A[0].p), (const S*)h->Bv[1].p, 1.0));
   }
   CHK(rec.run());
   CHK(timing_end(h, &h->ms_ad, &h->n_ad, launches));
@@ -2780,7 +2844,7 @@ int fkpm_get_kernel_mfma(fkpm_handle* h, int kind, int* mfma) {
 
 int fkpm_get_alpha_table(fkpm_handle* h, int* stored) {
   if (!h || !stored) return fail(FKPM_E_ARG, "null argument");
-  *stored = (h->a_stored && h->alpha_M > 0) ? 1 : 0;
+  *stored = (h->a_slots > 0 && h->alpha_M > 0) ? 1 : 0;
   return 0;
 }
 
@@ -2864,7 +2928,7 @@ int fkpm_set_option(fkpm_handle* h, int option, int value) {
       if (value < 0 || value > 2) return fail(FKPM_E_ARG, "bad store-alpha mode %d", value);
       h->store_alpha = value;
       h->alpha_M = 0;  // moments(M) again before autodiff_matrix
-      h->a_stored = false;
+      h->a_slots = 0;
       return 0;
     case FKPM_OPT_SWEEP:
       if (value < -1 || value > 64) return fail(FKPM_E_ARG, "bad sweep %d", value);

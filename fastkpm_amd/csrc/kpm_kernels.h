@@ -1347,40 +1347,41 @@ __global__ __launch_bounds__(WG) void k_copy16(const double2* __restrict__ a,
     b[k] = a[k];
 }
 
-// Weighted sums of the kept forward vectors for stoch_matrix:
-//   v = sum_{i=0..K} d_i alpha_i,   u = sum_{i=0..K-1} e_i alpha_i
+// NO weighted sums of the kept forward vectors for stoch_matrix,
+//   o_k = sum_{i=0..K} w[k (K + 1) + i] alpha_i
 // (alpha_0 = R, alpha_i = table slot i-1, slots `slot` scalars apart), one
 // streaming pass over the table with FP64 sums; n scalars per vector, a
 // multiple of the 16-byte packet.  Each thread keeps U slots' loads in flight.
 // The slots are cut into SL runs, summed by SL threads a packet: bound by HBM
 // with SL = 1 on large vectors (256^2 x 2 x 64: 5.7 TB/s), by the chain of K / U
 // round trips where one thread a packet leaves most of the chip idle.
-template <typename S, int SL>
+template <typename S, int SL, int NO>
 __global__ __launch_bounds__(WG) void k_table_sums(const S* __restrict__ R,
                                                    const S* __restrict__ tab, size_t slot, int K,
-                                                   const double* __restrict__ d,
-                                                   const double* __restrict__ e,
-                                                   S* __restrict__ u, S* __restrict__ v, size_t n) {
+                                                   const double* __restrict__ w,
+                                                   S* __restrict__ o0, S* __restrict__ o1,
+                                                   S* __restrict__ o2, size_t n) {
   typedef typename Vec16<S>::V VT;
   constexpr int NS = Vec16<S>::N, U = 8, PQ = WG / SL;  // PQ: packets of a workgroup
-  __shared__ double part[SL > 1 ? 2 * NS * WG : 1];
+  __shared__ double part[SL > 1 ? NO * NS * WG : 1];
   const size_t np = n / NS;
   const int sl = SL > 1 ? threadIdx.x / PQ : 0;
   const int per = (K + SL - 1) / SL;
   const int i1 = min(K, (sl + 1) * per);
   for (size_t q0 = (size_t)blockIdx.x * PQ; q0 < np; q0 += (size_t)gridDim.x * PQ) {
     const size_t q = q0 + threadIdx.x % PQ;
-    double au[NS], av[NS];
+    double acc[NO][NS];
 #pragma unroll
-    for (int t = 0; t < NS; t++) au[t] = av[t] = 0.0;
+    for (int o = 0; o < NO; o++)
+#pragma unroll
+      for (int t = 0; t < NS; t++) acc[o][t] = 0.0;
     if (q < np) {
       if (sl == 0) {
         const VT r = __builtin_nontemporal_load(reinterpret_cast<const VT*>(R) + q);
 #pragma unroll
-        for (int t = 0; t < NS; t++) {
-          av[t] = d[0] * (double)r[t];
-          au[t] = K > 0 ? e[0] * (double)r[t] : 0.0;
-        }
+        for (int o = 0; o < NO; o++)
+#pragma unroll
+          for (int t = 0; t < NS; t++) acc[o][t] = w[o * (K + 1)] * (double)r[t];
       }
       for (int i0 = 1 + sl * per; i0 <= i1; i0 += U) {
         VT x[U];
@@ -1392,11 +1393,11 @@ __global__ __launch_bounds__(WG) void k_table_sums(const S* __restrict__ R,
         for (int k = 0; k < U; k++) {
           const int i = i0 + k;
           if (i <= i1) {
-            const double di = d[i], ei = i < K ? e[i] : 0.0;
 #pragma unroll
-            for (int t = 0; t < NS; t++) {
-              av[t] = fma(di, (double)x[k][t], av[t]);
-              au[t] = fma(ei, (double)x[k][t], au[t]);
+            for (int o = 0; o < NO; o++) {
+              const double wi = w[o * (K + 1) + i];
+#pragma unroll
+              for (int t = 0; t < NS; t++) acc[o][t] = fma(wi, (double)x[k][t], acc[o][t]);
             }
           }
         }
@@ -1405,28 +1406,27 @@ __global__ __launch_bounds__(WG) void k_table_sums(const S* __restrict__ R,
     if constexpr (SL > 1) {
       __syncthreads();
 #pragma unroll
-      for (int t = 0; t < NS; t++) {
-        part[(2 * t) * WG + threadIdx.x] = au[t];
-        part[(2 * t + 1) * WG + threadIdx.x] = av[t];
-      }
+      for (int o = 0; o < NO; o++)
+#pragma unroll
+        for (int t = 0; t < NS; t++) part[(o * NS + t) * WG + threadIdx.x] = acc[o][t];
       __syncthreads();
       if (sl == 0)
         for (int k = 1; k < SL; k++)
 #pragma unroll
-          for (int t = 0; t < NS; t++) {
-            au[t] += part[(2 * t) * WG + k * PQ + threadIdx.x];
-            av[t] += part[(2 * t + 1) * WG + k * PQ + threadIdx.x];
-          }
+          for (int o = 0; o < NO; o++)
+#pragma unroll
+            for (int t = 0; t < NS; t++)
+              acc[o][t] += part[(o * NS + t) * WG + k * PQ + threadIdx.x];
     }
     if (sl == 0 && q < np) {
-      VT ou, ov;
+      S* const out[3] = {o0, o1, o2};
 #pragma unroll
-      for (int t = 0; t < NS; t++) {
-        ou[t] = (S)au[t];
-        ov[t] = (S)av[t];
+      for (int o = 0; o < NO; o++) {
+        VT v;
+#pragma unroll
+        for (int t = 0; t < NS; t++) v[t] = (S)acc[o][t];
+        reinterpret_cast<VT*>(out[o])[q] = v;
       }
-      reinterpret_cast<VT*>(u)[q] = ou;
-      reinterpret_cast<VT*>(v)[q] = ov;
     }
   }
 }

@@ -189,6 +189,8 @@ int fkpm_moments_noalloc(int device, int prec, int nb, int b, int nnzb, const in
                                    environment variable FKPM_ALPHA_TABLE_BYTES), and
                                    fkpm_autodiff_matrix then reads alpha_{m-1} instead of
                                    recomputing it (one gathered vector per step instead of two);
+                                   where only some fit, from alpha_{ceil(M/3)} on, it keeps the
+                                   first ones and autodiff_matrix recomputes down to them;
                                    1 (default): the same, except that lattices small enough
                                    for the whole-recursion kernels (about 4096 orbital rows)
                                    run those, with a table of their own; 0: the three-vector
@@ -196,7 +198,8 @@ int fkpm_moments_noalloc(int device, int prec, int nb, int b, int nnzb, const in
 #define FKPM_OPT_SWEEP 4        /* value 0: every kernel kind sweeps the rows per XCD; s in
                                    1..64: as one front in segments of s passes per XCD
                                    (fkpm_get_kernel_sweep); -1 (default): the configuration's
-                                   own (the tuner's choice, else one front with s = 2) */
+                                   own (the tuner's choice, else per XCD while the vectors of
+                                   a step stay in the last-level cache, one front past it) */
 #define FKPM_OPT_SLICE 6        /* value 1: the vector-unit step kernels sweep all their block
                                    rows once per column pass (the probe columns of a row in
                                    slices of one pass width), so the rows an XCD gathers
@@ -235,9 +238,12 @@ int fkpm_moments_noalloc(int device, int prec, int nb, int b, int nnzb, const in
 #define FKPM_STOCH_TABLE 2      /* (reported only) xi from the forward vectors a preceding
                                    fkpm_moments kept (FKPM_OPT_STORE_ALPHA), by
                                    T_{K+j} = 2 T_K T_j - T_{K-j}: one pass over the table and
-                                   K = ceil(M/2) Chebyshev steps instead of M - 1 */
+                                   K = ceil(M/2) Chebyshev steps instead of M - 1, or 2K steps
+                                   with K = ceil(M/3) where the table was cut short */
 #define FKPM_STOCH_AUTO 3       /* FKPM_STOCH_TABLE when the held forward vectors (same H and
-                                   R) reach alpha_K, else FKPM_STOCH_CLENSHAW */
+                                   R) reach alpha_{ceil(M/2)}, or, cut short by the memory,
+                                   alpha_{ceil(M/3)} and M is at most the order they were kept
+                                   for; else FKPM_STOCH_CLENSHAW */
 int fkpm_set_option(fkpm_handle* h, int option, int value);
 
 /* Kernel kinds of fkpm_get_kernel_config. */

@@ -175,3 +175,47 @@ def test_matrix_core_outer_product(oracle, S, prec):
     want = orc.stoch_matrix(c, D)
     assert rel_err(D.val, want) < (1e-10 if prec == "fp64" else M * 16 * 2.0 ** -24)
     eng.close()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("b,S", [(1, 5), (2, 17), (4, 6), (8, 20)])
+@pytest.mark.parametrize("M", [14, 16, 18])
+def test_first_forward_vectors_kept(oracle, monkeypatch, M, b, S, prec):
+    """A table too small for every forward vector keeps the first ones from a
+    third of the orders on: autodiff_matrix recomputes down to them and reads
+    the rest (D on H's pattern and on the diagonal), stoch_matrix starts from
+    them up to the order they were kept for."""
+    from fastkpm_amd import EnergyScale, HipEngine, lattice
+    H = lattice.lattice((4, 3, 3), b=b, orbital_blocks=b > 2, W=1.0, J=1.0 if b == 2 else 0.0,
+                        seed=S)
+    bound = float(np.abs(np.linalg.eigvalsh(H.to_dense())).max()) * 1.01
+    nb = H.n_rows
+    rng = np.random.default_rng(S)
+    R = rng.standard_normal((nb * b, S)) + 1j * rng.standard_normal((nb * b, S))
+    Dd = lattice.coo_to_bsr(nb, b, np.arange(nb), np.arange(nb), np.zeros((nb, b, b)))
+    c = 1.0 / (1.0 + np.arange(M + 2))
+    orc = oracle.Engine()
+    orc.set_H(H, -bound, bound)
+    orc.set_R(R)
+    tol = 1e-10 if prec == "fp64" else M * 16 * 2.0 ** -24
+    least = -(-M // 3)
+    for slots in (least - 1, least, least + 1, M // 2 - 1):
+        eng = HipEngine("cx_double", prec)
+        eng.set_store_alpha(2)
+        eng.set_R(R)
+        eng.set_H(H, EnergyScale(-bound, bound))
+        eng.moments(2)  # the padded width
+        vb = nb * b * eng.config()["s_padded"] * (16 if prec == "fp64" else 8)
+        monkeypatch.setenv("FKPM_ALPHA_TABLE_BYTES", str(slots * vb))
+        for D in (H.like(), Dd):
+            assert rel_err(eng.moments(M), orc.moments(M)) < tol
+            assert eng.alpha_table() == (slots >= least)
+            eng.autodiff_matrix(c[:M], D)
+            assert rel_err(D.val, orc.autodiff_matrix(c[:M], D)) < tol
+        for m in (M, M - 1, M - 2, 3, M + 2):
+            eng.stoch_matrix(c[:m], D)
+            kept = slots >= least and m <= M or m <= 2 * slots and slots >= least
+            assert eng.stoch_method() == ("table" if kept else "clenshaw"), (slots, m)
+            assert rel_err(D.val, orc.stoch_matrix(c[:m], D)) < tol
+        monkeypatch.delenv("FKPM_ALPHA_TABLE_BYTES")
+        eng.close()
