@@ -694,7 +694,10 @@ void admit_one(fkpm_batch* B, Slot& sl) {
   d.psum = (double*)P(B_PSUM);
   d.c = (const double*)P(B_C);
   d.rord = r.rdesc.empty() ? nullptr : (const int*)P(B_RD);
-  d.nt = r.rdesc.empty() ? 0 : fkd::NT_ORDER;
+  d.nt = !r.rdesc.empty()                              ? fkd::NT_ORDER
+         : (long long)r.nb * r.max_deg == r.nnzb && r.max_deg < 1 << 16
+             ? r.max_deg << fkd::NT_DEG
+             : 0;
   d.nb = r.nb;
   d.qp = L.qp;
   d.chunk = L.chunk;

@@ -618,6 +618,14 @@ const int* rp_for(const fkpm_handle* h, const KCfg& c) {
   return (c.nt & fkd::NT_ORDER) ? h->rdesc.as<const int>() : h->rp.as<const int>();
 }
 
+// The nt argument of a step kernel on H's pattern: the configuration's, with the
+// row length where all rows share one (row_ptr).
+int nt_for(const fkpm_handle* h, const KCfg& c) {
+  const bool same = !(c.nt & fkd::NT_ORDER) && (long long)h->nb * h->max_deg == h->nnzb &&
+                    h->max_deg < 1 << 16;
+  return same ? c.nt | h->max_deg << fkd::NT_DEG : c.nt;
+}
+
 // Kernel entry of a kind under its configuration.
 template <class S>
 auto mom_fn(const fkpm_handle* h, const fkd::KSet<S>& ks, const KCfg& c) {
@@ -1074,7 +1082,7 @@ int tune_t(fkpm_handle* h) {
               return launch(mom_fn(h, ks, k), dim3(k.nwg), dim3(fkd::WG), h->stream, rp_for(h, k), ci, hv,
                             (const S*)slot((t + 1) % ns), (const S*)slot(t % ns),
                             slot((t + 2) % ns), h->nb, h->qp, k.chunk, 2.0, -1.0,
-                            h->partial.as<double>(), k.nt, no_rsource<S>());
+                            h->partial.as<double>(), nt_for(h, k), no_rsource<S>());
             }
             if (kind == K_ADS) {  // backward over slots ns-2 .. 1, beta in the ring
               const int t = tstep++;
@@ -1083,7 +1091,7 @@ int tune_t(fkpm_handle* h) {
                             hv, (const S*)slot(m), (const S*)slot(m + 1),
                             (const S*)bring[(t + 1) % 3], (const S*)bring[t % 3],
                             (const S*)slot(m - 1), bring[(t + 2) % 3], h->tune_dacc.as<double>(),
-                            h->nb, h->qp, k.chunk, 0.1, 0.1, 0.1, 1.0, 0.0, 2.0, k.nt);
+                            h->nb, h->qp, k.chunk, 0.1, 0.1, 0.1, 1.0, 0.0, 2.0, nt_for(h, k));
             }
             const int t = step++;
             S* x = ring[(t + 1) % 3];
@@ -1097,19 +1105,19 @@ int tune_t(fkpm_handle* h) {
               const bool cl = t & 1;
               return launch(mom_fn(h, ks, k), dim3(k.nwg), dim3(fkd::WG), h->stream, rp_for(h, k), ci, hv,
                             (const S*)x, (const S*)z, y, h->nb, h->qp, k.chunk, 2.0, -1.0,
-                            cl ? (double*)nullptr : h->partial.as<double>(), k.nt,
+                            cl ? (double*)nullptr : h->partial.as<double>(), nt_for(h, k),
                             cl ? rsource<S>(h, 0.25) : no_rsource<S>());
             }
             if (kind == K_XI)
               return launch(ks.xi, dim3(k.nwg), dim3(fkd::WG), h->stream, rp_for(h, k), ci, hv, (const S*)x,
                             (const S*)z, y, h->xi.as<double>(), h->nb, h->qp, k.chunk, 2.0, -1.0,
-                            0.0, 0.5, t == 0 ? 1 : 0, k.nt);
+                            0.0, 0.5, t == 0 ? 1 : 0, nt_for(h, k));
             // backward step: reads alpha_m, alpha_{m+1}, beta_{m+1}, beta_{m+2};
             // writes alpha_{m-1}, beta_m into the third buffers
             return launch(adf_fn(h, ks, k), dim3(k.nwg), dim3(fkd::WG), h->stream, rp_for(h, k), ci, hv,
                           (const S*)x, (const S*)z, (const S*)bring[(t + 1) % 3],
                           (const S*)bring[t % 3], y, bring[(t + 2) % 3], h->tune_dacc.as<double>(),
-                          h->nb, h->qp, k.chunk, 0.1, 0.1, 0.1, 1.0, 0.0, 2.0, k.nt);
+                          h->nb, h->qp, k.chunk, 0.1, 0.1, 0.1, 1.0, 0.0, 2.0, nt_for(h, k));
           };
           CHK(run());
           HIPCHK(hipEventRecord(h->ev0, h->stream));
@@ -1565,7 +1573,7 @@ int moments_t(fkpm_handle* h, int M, double* mu) {
         CHK(launch(mom_fn(h, ks, kc), dim3(kc.nwg), block, h->stream, rp_for(h, kc),
                    h->ci.as<const int>(), h->hv.as<const S>(), x, z, y, h->nb, h->qp, kc.chunk,
                    m == 0 ? 1.0 : 2.0, m == 0 ? 0.0 : -1.0,
-                   h->partial.as<double>() + (size_t)(m - m0) * kc.nwg * 2, kc.nt,
+                   h->partial.as<double>() + (size_t)(m - m0) * kc.nwg * 2, nt_for(h, kc),
                    no_rsource<S>()));
       }
       CHK(launch(&fkd::k_reduce_partials, dim3(m1 - m0), block, h->stream,
@@ -1696,7 +1704,7 @@ int stoch_clenshaw(fkpm_handle* h, int M, const double* c, const S** xi_out) {
   auto step = [&](double xfac, double cr, S* y) -> int {
     return launch(mom_fn(h, ks, kc), grid, block, h->stream, rp_for(h, kc), h->ci.as<const int>(),
                   h->hv.as<const S>(), b1.p, b2.p, y, h->nb, h->qp, kc.chunk, xfac * b1.s,
-                  b2.p ? -b2.s : 0.0, (double*)nullptr, kc.nt, rsource<S>(h, cr));
+                  b2.p ? -b2.s : 0.0, (double*)nullptr, nt_for(h, kc), rsource<S>(h, cr));
   };
   for (int k = M - 2; k >= 1; k--) {
     S* y = (S*)h->A[slot].p;
@@ -1730,7 +1738,7 @@ int chebyshev_of(fkpm_handle* h, int K, double f, const S* add, int* slot) {
     const double g = k == K - 1 ? f : 1.0;
     CHK(launch(mom_fn(h, ks, kc), dim3(kc.nwg), dim3(fkd::WG), h->stream, rp_for(h, kc),
                h->ci.as<const int>(), h->hv.as<const S>(), x, z, y, h->nb, h->qp, kc.chunk,
-               (k == 0 ? 1.0 : 2.0) * g, k == 0 ? 0.0 : -g, (double*)nullptr, kc.nt,
+               (k == 0 ? 1.0 : 2.0) * g, k == 0 ? 0.0 : -g, (double*)nullptr, nt_for(h, kc),
                k == K - 1 ? src : no_rsource<S>()));
     z = x;
     x = y;
@@ -1848,13 +1856,13 @@ int stoch_t(fkpm_handle* h, int M, const double* c) {
       // alpha_1 = Hs R, xi = c0 R + c1 alpha_1
       CHK(launch(ksx.xi, grid, block, h->stream, rp_for(h, kx), ci, hv, (const S*)h->vec_a(0),
                  (const S*)nullptr, (S*)h->vec_a(1), h->xi.as<double>(), h->nb, h->qp, kx.chunk,
-                 1.0, 0.0, c[0], c[1], 1, kx.nt));
+                 1.0, 0.0, c[0], c[1], 1, nt_for(h, kx)));
       for (int m = 2; m < M; m++) {
         // alpha_m = 2 Hs alpha_{m-1} - alpha_{m-2}; xi += c_m alpha_m
         CHK(launch(ksx.xi, grid, block, h->stream, rp_for(h, kx), ci, hv,
                    (const S*)h->vec_a(m - 1),
                    (const S*)h->vec_a(m - 2), (S*)h->vec_a(m), h->xi.as<double>(), h->nb, h->qp,
-                   kx.chunk, 2.0, -1.0, 0.0, c[m], 0, kx.nt));
+                   kx.chunk, 2.0, -1.0, 0.0, c[m], 0, nt_for(h, kx)));
       }
       CHK(rec.run());
     }
@@ -1941,17 +1949,17 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
           CHK(add_outer<S>(h, am, first ? am : bm1, first ? 2.0 * sb : 2.0));
         CHK(launch(h->d_fused ? ads_fn(h, kst, kt) : adsp_fn(kst, kt), dim3(kt.nwg), block,
                    h->stream, rp_for(h, kt), ci, hv, am, am1, bm1, bm2, (const S*)aout, bout, dacc,
-                   h->nb, h->qp, kt.chunk, c4, c2, w, sb, sb2, 2.0, kt.nt));
+                   h->nb, h->qp, kt.chunk, c4, c2, w, sb, sb2, 2.0, nt_for(h, kt)));
       } else if (h->d_fused) {
         CHK(launch(adf_fn(h, ksa, ka), dim3(ka.nwg), block, h->stream, rp_for(h, ka), ci, hv, am, am1,
                    bm1, bm2,
-                   aout, bout, dacc, h->nb, h->qp, ka.chunk, c4, c2, w, sb, sb2, 2.0, ka.nt));
+                   aout, bout, dacc, h->nb, h->qp, ka.chunk, c4, c2, w, sb, sb2, 2.0, nt_for(h, ka)));
       } else {
         // D += 2 alpha_m beta_{m+1}^+ on D's own pattern, then the step.
         CHK(add_outer<S>(h, am, first ? am : bm1, first ? 2.0 * sb : 2.0));
         CHK(launch(adp_fn(ksa, ka), dim3(ka.nwg), block, h->stream, rp_for(h, ka), ci, hv, am, am1,
                    bm1, bm2,
-                   aout, bout, dacc, h->nb, h->qp, ka.chunk, c4, c2, w, sb, sb2, 2.0, ka.nt));
+                   aout, bout, dacc, h->nb, h->qp, ka.chunk, c4, c2, w, sb, sb2, 2.0, nt_for(h, ka)));
       }
       launches++;
     }
@@ -2168,9 +2176,12 @@ int moments2_t(fkpm_handle* h, int M, int col_chunk, size_t budget, double* mu) 
   const dim3 grid(c.nwg), block(fkd::WG);
   auto step = [&](const int* rp_, const int* ci_, const S* hv_, const S* x, const S* z, S* y,
                   double cx, double cz) {
-    // the row order belongs to H's pattern; the currents' products sweep rows
+    // the row order and the row length belong to H's pattern
+    KCfg rows = c;
+    rows.nt &= ~fkd::NT_ORDER;
     return launch(ks.mom, grid, block, h->stream, rp_, ci_, hv_, x, z, y, h->nb, qpc, c.chunk,
-                  cx, cz, (double*)nullptr, c.nt & ~fkd::NT_ORDER, no_rsource<S>());
+                  cx, cz, (double*)nullptr, rp_ == rp ? nt_for(h, rows) : rows.nt,
+                  no_rsource<S>());
   };
   const int* j1rp = h->j_rp[0].as<const int>();
   const int* j1ci = h->j_ci[0].as<const int>();

@@ -112,6 +112,7 @@ __device__ __forceinline__ void stv_nt(T* __restrict__ p, const A* v, bool nt) {
 // Bits of the `nt` kernel argument.
 constexpr int NT_LOAD = 1;   // loads of the operands read once per step
 constexpr int NT_STORE = 2;  // stores of the step's outputs
+constexpr int NT_DEG = 8;    // first bit of the row length all rows share (0: none)
 // Loop order of the step kernels: without NT_SLICE a lane group finishes
 // every column pass of a block row before the next row; with it the
 // workgroups sweep all their rows once per column pass (L*KQ packets), so the
@@ -312,6 +313,10 @@ struct Geo {
   // take 64 (up to 8 blocks: a 2-D lattice row in one batch on 64 lanes,
   // FP64 forward step 80 -> 79 us at C2; the autodiff step lost a wave per
   // SIMD and 4 us with it).
+  // On fewer lanes the registers of FP64 vectors and per-lane H blocks leave two
+  // waves per SIMD either way, and 40 is the better budget (128^2 x 2 15.7 -> 15.1 us,
+  // 200^2 x 1 11.5 -> 10.5; on 64 lanes 256^2 x 2 80 -> 83; FP32 kept 64: 96 and 128 lost
+  // up to 10 %).
   template <int NX, int BUDGET = 48>
   static constexpr int batch() {
     constexpr int per = NX * B * KQ * NS + B * B * HS;
@@ -374,7 +379,10 @@ __device__ __forceinline__ RowRange wg_rows(int nb, int chunk, int step, WgId wi
 }
 
 // The block row at sweep position i and its block range: row i and rp[i],
-// rp[i+1], or with NT_ORDER the descriptor rp[3i .. 3i+2] (empty past r1).
+// rp[i+1], or with NT_ORDER the descriptor rp[3i .. 3i+2] (empty past r1).  Bits
+// NT_DEG and up of nt hold the blocks of every row where all rows have as many (a
+// lattice): the range then needs no load, one round trip less before a row's
+// gather (forward step 128^2 x 2 FP64 14.4 -> 13.7 us, 200^2 x 1 9.2 -> 8.7).
 // The row loops load the next position's entry before working on the current
 // row.
 struct RowPtr {
@@ -384,6 +392,7 @@ struct RowPtr {
 __device__ __forceinline__ RowPtr row_ptr(const int* __restrict__ rp, int i, int r1, int nt) {
   if (i >= r1) return RowPtr{i, 0, 0};
   if (nt & NT_ORDER) return RowPtr{rp[3 * i], rp[3 * i + 1], rp[3 * i + 2]};
+  if (const int deg = nt >> NT_DEG) return RowPtr{i, i * deg, (i + 1) * deg};
   return RowPtr{i, rp[i], rp[i + 1]};
 }
 
@@ -498,7 +507,8 @@ __device__ __forceinline__ void gather_row(const int* __restrict__ ci, const S* 
   const A none[KQ][B][Vec16<S>::N] = {};
   auto nopre = [](int) { return NoPre{}; };
   auto blk4 = [&](int p, int jb, auto& xv, NoPre) { blk(p, jb, xv); };
-  gather_row_pre<S, A, CX, B, L, KQ, NX, false, decltype(blk4)&, decltype(nopre)&, 64>(
+  constexpr int BUD = sizeof(S) == 8 && L < WAVE ? 40 : 64;
+  gather_row_pre<S, A, CX, B, L, KQ, NX, false, decltype(blk4)&, decltype(nopre)&, BUD>(
       ci, hv, X, rs, qo, p0, p1, acc, blk4, nopre, -1, none);
 }
 
@@ -626,6 +636,11 @@ __device__ __forceinline__ void step_moments_dev(
     const int p0 = cur.p0, p1 = cur.p1;
     for (int q0 = qs; q0 < qs + qw; q0 += L * KQ) {
       const size_t qo = (size_t)(q0 + l) * NS;
+      // own rows of z with the gather's first loads, where they take few registers
+      constexpr bool EARLY = KQ <= 2;
+      A out[KQ][B][NS];
+      if constexpr (EARLY)
+        if (z != nullptr) load_rows_nt<S, A, B, L, KQ>(z, i, rs, qo, out, nt & NT_LOAD);
       A xd[KQ][B][NS];
       A acc[1][KQ][B][NS];
       // the own rows of x (for the dots) arrive with the diagonal block of
@@ -650,9 +665,8 @@ __device__ __forceinline__ void step_moments_dev(
                                                for (int e = 0; e < NS; e++)
                                                  xd[k][bi][e] = xv[0][bi][k][e];
                                          });
-      A out[KQ][B][NS];
       if (z != nullptr) {
-        load_rows_nt<S, A, B, L, KQ>(z, i, rs, qo, out, nt & NT_LOAD);
+        if constexpr (!EARLY) load_rows_nt<S, A, B, L, KQ>(z, i, rs, qo, out, nt & NT_LOAD);
 #pragma unroll
         for (int k = 0; k < KQ; k++)
 #pragma unroll
