@@ -1305,13 +1305,20 @@ size_t res_lds(fkpm_handle* h) {
   return 2 * (((size_t)(h->nb + 1) * h->rset<S>().elem_bytes + 15) / 16 * 16);
 }
 
+// The kernel for rows of at most `deg` blocks, from the blocks each keeps.
+int res_mode(int deg, const int (&dreg)[3]) {
+  return deg <= dreg[fkd::RES_OWN] ? fkd::RES_OWN
+         : deg <= dreg[fkd::RES_REG] ? fkd::RES_REG
+                                     : fkd::RES_ST;
+}
+
 // The backward recursion's kernel: the thread's rows of the forward vectors in
 // registers where the whole of H still fits beside them, else in LDS where
 // four buffers fit (autodiff_matrix of M = 128, us, registers / LDS: 45x42 x 2 FP32 272 /
 // 253, 35x36 x 2 FP64 534 / 439, 50x50 x 1 510 / 421, 15^3 x 1 real 422 / 354, 8^3 x 4 FP32
 // 331 / 261, FP64 663 / 602).
 struct ResBwd {
-  int st, la;  // some blocks streamed; forward vectors in LDS
+  int mode, la;  // fkd::ResMode; forward vectors in LDS
   size_t lds;
 };
 
@@ -1319,8 +1326,10 @@ template <class S>
 ResBwd res_bwd(fkpm_handle* h) {
   const fkd::ResSet<S>& rs = h->rset<S>();
   const size_t lds = res_lds<S>(h);
-  const int la = h->max_deg > rs.dreg_bwd[0][0] && 2 * lds <= kLdsBytes;
-  return ResBwd{h->max_deg > rs.dreg_bwd[0][la], la, la ? 2 * lds : lds};
+  if (h->max_deg <= rs.dreg_bwd[fkd::RES_OWN][0]) return ResBwd{fkd::RES_OWN, 0, lds};
+  const int la = h->max_deg > rs.dreg_bwd[fkd::RES_REG][0] && 2 * lds <= kLdsBytes;
+  return ResBwd{h->max_deg > rs.dreg_bwd[fkd::RES_REG][la] ? fkd::RES_ST : fkd::RES_REG, la,
+                la ? 2 * lds : lds};
 }
 
 // Whether the whole-recursion kernels run for the current H and R: the
@@ -1342,8 +1351,8 @@ bool res_wanted(fkpm_handle* h) {
   if (2 * ((size_t)(h->nb + 1) * rs.elem_bytes + 16) > kLdsBytes) return false;
   const int threads = ((h->nb + rpt - 1) / rpt + 63) / 64 * 64;
   const ResBwd rb = res_bwd<S>(h);
-  if (rb.st) {
-    const int d = h->max_deg - rs.dreg_bwd[1][rb.la];
+  if (rb.mode == fkd::RES_ST) {
+    const int d = h->max_deg - rs.dreg_bwd[fkd::RES_ST][rb.la];
     if ((size_t)d * (rs.block_bytes + 4) * h->nb > kResStream) return false;
   }
   if (rpt != h->res.rpt || threads != h->res.threads) h->res.packed = false;
@@ -1422,7 +1431,7 @@ int res_moments(fkpm_handle* h, int M, double* mu, bool* done) {
   CHK(h->partial.ensure((size_t)nsteps * ny * 2 * sizeof(double)));
   CHK(h->res.pin.ensure((size_t)nsteps * 2 * sizeof(double)));
   CHK(timing_begin(h));
-  CHK(launch_lds(rs.fwd[h->max_deg > rs.dreg_fwd[0]], dim3(h->s), dim3(h->res.threads), res_lds<S>(h), h->stream,
+  CHK(launch_lds(rs.fwd[res_mode(h->max_deg, rs.dreg_fwd)], dim3(h->s), dim3(h->res.threads), res_lds<S>(h), h->stream,
                  res_H<S>(h), h->R.as<const S>(), h->sp, h->res.atab.as<S>(), slot, nsteps));
   CHK(timing_end(h, &h->ms_mom, &h->n_mom, nsteps));
   CHK(launch(&fkd::k_res_dots<S>, dim3(nsteps, ny), dim3(fkd::WG), h->stream,
@@ -1476,7 +1485,7 @@ int res_autodiff(fkpm_handle* h, int M, const double* c, double diag) {
   if (M2 > 1) {
     CHK(res_coef(h, c, M));
     const ResBwd rb = res_bwd<S>(h);
-    CHK(launch_lds(rs.bwd[rb.st][rb.la], dim3(h->s), dim3(h->res.threads), rb.lds, h->stream,
+    CHK(launch_lds(rs.bwd[rb.mode][rb.la], dim3(h->s), dim3(h->res.threads), rb.lds, h->stream,
                    res_H<S>(h), h->res.atab.as<const S>(), h->res.btab.as<S>(), slot, M2,
                    h->res.coef.as<const double>(), 2 * c[M - 1]));
   }
@@ -1507,7 +1516,7 @@ int res_stoch(fkpm_handle* h, int M, const double* c, bool table) {
     CHK(res_coef(h, c, M));
   }
   const S* r0 = table ? h->res.atab.as<const S>() : u;
-  CHK(launch_lds(rs.xi[h->max_deg > rs.dreg_xi[0]], dim3(h->s), dim3(h->res.threads), res_lds<S>(h), h->stream,
+  CHK(launch_lds(rs.xi[res_mode(h->max_deg, rs.dreg_xi)], dim3(h->s), dim3(h->res.threads), res_lds<S>(h), h->stream,
                  res_H<S>(h), h->R.as<const S>(), h->sp, (const S*)(table ? u : nullptr),
                  (const S*)v, h->res.coef.as<const double>(), table ? K : M, u, xi));
   return res_outer<S>(h, fkd::ResTerms<S>{r0, xi, slot, 0, 0.0, 0.0}, 2, h->dout.as<double>());

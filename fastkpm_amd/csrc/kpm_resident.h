@@ -16,8 +16,8 @@
 // the table sums of stoch_matrix (k_table_sums).
 //
 // A row's products and the axpby are the operations of the step kernels in
-// kpm_kernels.h in the same order, so the vectors are bitwise theirs; the dots
-// and D accumulate in FP64.
+// kpm_kernels.h, in FP32 in the same order, so that the vectors are bitwise
+// theirs (FP64 takes the diagonal block first); the dots and D accumulate in FP64.
 #pragma once
 #include "kpm_kernels.h"
 
@@ -49,6 +49,8 @@ struct ResGeo {
   }
 };
 constexpr int RES_VL_FWD = 2, RES_VL_XI = 2, RES_VL_BWD = 5;
+// Two more vectors with RES_OWN.
+constexpr int res_vl(int vl, int mode) { return mode == 2 ? vl + 2 : vl; }
 // FP64 with streamed blocks keeps the registers of one more vector free: 9^3 x 2
 // (two rows a thread) streamed two blocks of seven slower than three.
 template <typename S, bool ST>
@@ -93,8 +95,9 @@ __device__ __forceinline__ void stn(S* p, const S (&v)[N]) {
 
 // H as the resident kernels read it: block d of the row owned by thread slot
 // i (i < nt) as PK packets at (d * PK + k) * nt + i, and the LDS byte offset
-// of its column block; rows with fewer blocks, and slots past the last row,
-// are filled with zero blocks on the zero vector block nb.
+// of its column block (FP64: block 0 is the diagonal one); rows with fewer blocks,
+// and slots past the last row, are filled with zero blocks on the zero vector
+// block nb.
 template <typename S>
 struct ResH {
   const S* val;
@@ -117,8 +120,13 @@ __global__ __launch_bounds__(WG) void k_res_pack_H(const int* __restrict__ rp,
   const int n = nt * deg;
   for (int w = blockIdx.x * WG + threadIdx.x; w < n; w += gridDim.x * WG) {
     const int d = w / nt, i = w % nt;
-    const int p = i < nb ? rp[i] + d : 0;
+    int p = i < nb ? rp[i] + d : 0;
     const bool live = i < nb && p < rp[i + 1];
+    if (sizeof(S) == 8 && live) {  // FP64: the diagonal block first, then the others in order
+      int pd = rp[i];
+      while (ci[pd] != i) pd++;  // every row has one (set_H requires it)
+      if (p <= pd) p = d == 0 ? pd : p - 1;
+    }
     off[w] = (live ? ci[p] : nb) * GE::BYTES;
 #pragma unroll
     for (int k = 0; k < GE::PK; k++)
@@ -129,9 +137,18 @@ __global__ __launch_bounds__(WG) void k_res_pack_H(const int* __restrict__ rp,
   }
 }
 
+// What a kernel does with the blocks and vectors its registers do not have to
+// hold.  RES_ST: blocks past DREG are streamed.  RES_OWN (FP64, every block in
+// registers): the thread's own rows of the last two vectors stay in registers
+// too, so the diagonal block and the recursion's second term read no LDS: five
+// accesses of a vector element instead of seven on a 2-D lattice (M = 128: 16x16 x 2
+// moments 54.5 -> 50.5 us, autodiff_matrix 125 -> 119).
+enum ResMode { RES_REG = 0, RES_ST = 1, RES_OWN = 2 };
+
 // The registers a thread keeps of H.
-template <typename S, bool CX, int B, int RPT, int VL, bool ST>
+template <typename S, bool CX, int B, int RPT, int VL, int MODE>
 struct ResRegs {
+  static constexpr bool ST = MODE == RES_ST, OWN = MODE == RES_OWN;
   using GE = ResGeo<S, CX, B, RPT>;
   static constexpr int DREG = GE::template dreg<VL, ST>();
   static constexpr int DA = DREG > 0 ? DREG : 1;
@@ -178,7 +195,8 @@ struct ResRegs {
   }
 
   template <int D0>
-  __device__ __forceinline__ void group(int deg, const char* xb, S (&acc)[RPT][GE::NV]) const {
+  __device__ __forceinline__ void group(int deg, const char* xb, const S (*own)[GE::NV],
+                                        S (&acc)[RPT][GE::NV]) const {
     if constexpr (D0 < DREG) {
       constexpr int D1 = D0 + (D0 == 0 ? 5 : 2) < DREG ? D0 + (D0 == 0 ? 5 : 2) : DREG;
       if (D0 < deg) {
@@ -187,17 +205,27 @@ struct ResRegs {
           S x[D1 - D0][GE::NV];
 #pragma unroll
           for (int d = D0; d < D1; d++)
-            ldn<S, GE::NV>(reinterpret_cast<const S*>(xb + off[k][d]), x[d - D0]);
+            if (!OWN || d > 0)
+              ldn<S, GE::NV>(reinterpret_cast<const S*>(xb + off[k][d]), x[d - D0]);
 #pragma unroll
-          for (int d = D0; d < D1; d++) mac(acc[k], h[k][d], x[d - D0]);
+          for (int d = D0; d < D1; d++) {
+            if constexpr (OWN) {
+              if (d == 0) {
+                mac(acc[k], h[k][0], own[k]);
+                continue;
+              }
+            }
+            mac(acc[k], h[k][d], x[d - D0]);
+          }
         }
-        group<D1>(deg, xb, acc);
+        group<D1>(deg, xb, own, acc);
       }
     }
   }
 
-  // acc[k] = (Hs x) of the thread's rows, x in LDS at xb
-  __device__ __forceinline__ void mul(const ResH<S>& H, const char* xb,
+  // acc[k] = (Hs x) of the thread's rows, x in LDS at xb (its own rows, with OWN,
+  // in `own`)
+  __device__ __forceinline__ void mul(const ResH<S>& H, const char* xb, const S (*own)[GE::NV],
                                       S (&acc)[RPT][GE::NV]) const {
 #pragma unroll
     for (int k = 0; k < RPT; k++)
@@ -206,7 +234,7 @@ struct ResRegs {
     // whole groups without a branch, so that a group's LDS reads are in flight
     // together: five blocks (a 2-D lattice row), then pairs; blocks past the
     // row's end are zero on the zero vector block
-    group<0>(H.deg, xb, acc);
+    group<0>(H.deg, xb, own, acc);
     if constexpr (ST) {
       for (int d = DREG; d < H.deg; d++) {
 #pragma unroll
@@ -262,7 +290,7 @@ __device__ __forceinline__ void res_zero_block(char* lds, int nb, int bufb) {
 // remaining blocks otherwise.  A step of the launched kernels took 4.5 us of
 // launch and latency at these sizes; here 0.56 us at 16x16 x 2 FP64, 0.50 us
 // at 32x32 x 1, 1.3 us at 45x42 x 2 FP32 (5.2 us before).
-template <typename S, bool CX, int B, int RPT, bool ST>
+template <typename S, bool CX, int B, int RPT, int MODE>
 __global__ __launch_bounds__(RES_T) void k_res_forward(ResH<S> H, const S* __restrict__ R, int sp,
                                                        S* __restrict__ tab, size_t slot,
                                                        int nsteps) {
@@ -271,14 +299,22 @@ __global__ __launch_bounds__(RES_T) void k_res_forward(ResH<S> H, const S* __res
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int bufb = res_buf_bytes<GE::BYTES>(H.nb);
   const size_t col = (size_t)blockIdx.x * H.nb * NV;
-  ResRegs<S, CX, B, RPT, RES_VL_FWD, ST> G;
+  constexpr bool OWN = MODE == RES_OWN;
+  ResRegs<S, CX, B, RPT, res_vl(RES_VL_FWD, MODE), MODE> G;
   G.load(H);
+  S x1[OWN ? RPT : 1][NV], x0[OWN ? RPT : 1][NV];  // OWN: rows of alpha_m, alpha_{m-1}
   {
     S r[RPT][NV];
     res_load_R<S, CX, B, RPT>(R, sp, H.nb, blockIdx.x, r);
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
       const int i = k * blockDim.x + threadIdx.x;
+      if constexpr (OWN)
+#pragma unroll
+        for (int e = 0; e < NV; e++) {
+          x1[k][e] = r[k][e];
+          x0[k][e] = S(0);
+        }
       if (i < H.nb) {
         stn<S, NV>(reinterpret_cast<S*>(lds + i * GE::BYTES), r[k]);
         stn<S, NV>(tab + col + (size_t)i * NV, r[k]);
@@ -291,15 +327,22 @@ __global__ __launch_bounds__(RES_T) void k_res_forward(ResH<S> H, const S* __res
     const char* xb = lds + (m & 1) * bufb;
     char* yb = lds + ((m & 1) ^ 1) * bufb;  // holds alpha_{m-1}
     S acc[RPT][NV];
-    G.mul(H, xb, acc);
+    G.mul(H, xb, x1, acc);
     S* out = tab + (size_t)(m + 1) * slot + col;
     S y[RPT][NV];
-    res_own<S, RPT, NV>(yb, H.nb, y);
+    if constexpr (!OWN) res_own<S, RPT, NV>(yb, H.nb, y);
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
       const int i = k * blockDim.x + threadIdx.x;
 #pragma unroll
-      for (int e = 0; e < NV; e++) y[k][e] = m > 0 ? fma(S(2), acc[k][e], -y[k][e]) : acc[k][e];
+      for (int e = 0; e < NV; e++) {
+        if constexpr (OWN) y[k][e] = x0[k][e];
+        y[k][e] = m > 0 ? fma(S(2), acc[k][e], -y[k][e]) : acc[k][e];
+        if constexpr (OWN) {
+          x0[k][e] = x1[k][e];
+          x1[k][e] = y[k][e];
+        }
+      }
       if (i < H.nb) {
         stn<S, NV>(reinterpret_cast<S*>(yb + i * GE::BYTES), y[k]);
         stn<S, NV>(out + (size_t)i * NV, y[k]);
@@ -318,7 +361,7 @@ __global__ __launch_bounds__(RES_T) void k_res_forward(ResH<S> H, const S* __res
 // alpha_{m+1} stay in registers, or (LA) in two more LDS buffers, which leaves
 // the registers of three vectors to blocks of H (45x42 x 2 FP32: all of it, 2.7 ->
 // 2.4 us a step).
-template <typename S, bool CX, int B, int RPT, bool ST, bool LA>
+template <typename S, bool CX, int B, int RPT, int MODE, bool LA>
 __global__ __launch_bounds__(RES_T) void k_res_backward(ResH<S> H, const S* __restrict__ tab,
                                                         S* __restrict__ btab, size_t slot, int M2,
                                                         const double* __restrict__ c, double sb) {
@@ -327,8 +370,10 @@ __global__ __launch_bounds__(RES_T) void k_res_backward(ResH<S> H, const S* __re
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int bufb = res_buf_bytes<GE::BYTES>(H.nb);
   const size_t col = (size_t)blockIdx.x * H.nb * NV;
-  ResRegs<S, CX, B, RPT, LA ? RES_VL_BWD_LA<S, ST> : RES_VL_BWD, ST> G;
+  constexpr bool OWN = MODE == RES_OWN;
+  ResRegs<S, CX, B, RPT, LA ? RES_VL_BWD_LA<S, MODE == RES_ST> : res_vl(RES_VL_BWD, MODE), MODE> G;
   G.load(H);
+  S b1[OWN ? RPT : 1][NV], b2o[OWN ? RPT : 1][NV];  // OWN: rows of beta_{m+1}, beta_{m+2}
   S ai[LA ? 1 : RPT][NV], a1[LA ? 1 : RPT][NV];
 #pragma unroll
   for (int k = 0; k < RPT; k++) {
@@ -338,6 +383,12 @@ __global__ __launch_bounds__(RES_T) void k_res_backward(ResH<S> H, const S* __re
     ldn<S, NV>(tab + (size_t)M2 * slot + col + (size_t)i * NV, t1);
     // clamped rows: the same value
     stn<S, NV>(reinterpret_cast<S*>(lds + i * GE::BYTES), t);
+    if constexpr (OWN)
+#pragma unroll
+      for (int e = 0; e < NV; e++) {
+        b1[k][e] = t[e];
+        b2o[k][e] = S(0);
+      }
     if constexpr (LA) {
       stn<S, NV>(reinterpret_cast<S*>(lds + 2 * bufb + i * GE::BYTES), t);
       stn<S, NV>(reinterpret_cast<S*>(lds + 3 * bufb + i * GE::BYTES), t1);
@@ -362,10 +413,10 @@ __global__ __launch_bounds__(RES_T) void k_res_backward(ResH<S> H, const S* __re
     const char* ab = lds + (2 + q) * bufb;      // LA: alpha_m
     char* a1b = lds + (2 + (q ^ 1)) * bufb;     // LA: alpha_{m+1}, then alpha_{m-1}
     S acc[RPT][NV];
-    G.mul(H, xb, acc);
+    G.mul(H, xb, b1, acc);
     S* out = btab + (size_t)m * slot + col;
     S y[RPT][NV];
-    res_own<S, RPT, NV>(yb, H.nb, y);
+    if constexpr (!OWN) res_own<S, RPT, NV>(yb, H.nb, y);
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
       const int i = k * blockDim.x + threadIdx.x;
@@ -377,11 +428,16 @@ __global__ __launch_bounds__(RES_T) void k_res_backward(ResH<S> H, const S* __re
       }
 #pragma unroll
       for (int e = 0; e < NV; e++) {
+        if constexpr (OWN) y[k][e] = b2o[k][e];
         const S b2 = first || second ? asb2 * t1[e] : y[k][e];
         S v = fma(ab2, acc[k][e], -b2);
         v = fma(ac4, t[e], v);
         v = fma(ac2, t1[e], v);
         y[k][e] = fma(aw, an[k][e], v);
+        if constexpr (OWN) {
+          b2o[k][e] = b1[k][e];
+          b1[k][e] = y[k][e];
+        }
         if constexpr (!LA) {
           t1[e] = t[e];
           t[e] = an[k][e];
@@ -401,7 +457,7 @@ __global__ __launch_bounds__(RES_T) void k_res_backward(ResH<S> H, const S* __re
 // recurrence from R (u null; b_{M-1} = c_{M-1} R virtual), or as
 // v + 2 T_K(Hs) u from the table sums u, v (K = M steps).  `r0` is slot 0 of the
 // output layout (column by column), where R is also written when u is null.
-template <typename S, bool CX, int B, int RPT, bool ST>
+template <typename S, bool CX, int B, int RPT, int MODE>
 __global__ __launch_bounds__(RES_T) void k_res_xi(ResH<S> H, const S* __restrict__ R, int sp,
                                                   const S* __restrict__ u, const S* __restrict__ v,
                                                   const double* __restrict__ c, int M,
@@ -411,8 +467,10 @@ __global__ __launch_bounds__(RES_T) void k_res_xi(ResH<S> H, const S* __restrict
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int bufb = res_buf_bytes<GE::BYTES>(H.nb);
   const size_t col = (size_t)blockIdx.x * H.nb * NV;
-  ResRegs<S, CX, B, RPT, RES_VL_XI, ST> G;
+  constexpr bool OWN = MODE == RES_OWN;
+  ResRegs<S, CX, B, RPT, res_vl(RES_VL_XI, MODE), MODE> G;
   G.load(H);
+  S x1[OWN ? RPT : 1][NV], x0[OWN ? RPT : 1][NV];  // OWN: rows of the last two vectors
   const bool cl = u == nullptr;
   {
     S x[RPT][NV];
@@ -420,11 +478,17 @@ __global__ __launch_bounds__(RES_T) void k_res_xi(ResH<S> H, const S* __restrict
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
       const int i = k * blockDim.x + threadIdx.x;
+      if constexpr (OWN)
+#pragma unroll
+        for (int e = 0; e < NV; e++) x1[k][e] = x0[k][e] = S(0);
       if (i >= H.nb) continue;
       if (cl)
         stn<S, NV>(r0 + col + (size_t)i * NV, x[k]);
       else
         ldn<S, NV>(u + col + (size_t)i * NV, x[k]);
+      if constexpr (OWN)
+#pragma unroll
+        for (int e = 0; e < NV; e++) x1[k][e] = x[k][e];
       stn<S, NV>(reinterpret_cast<S*>(lds + i * GE::BYTES), x[k]);
     }
   }
@@ -450,14 +514,16 @@ __global__ __launch_bounds__(RES_T) void k_res_xi(ResH<S> H, const S* __restrict
     const char* xb = lds + (t & 1) * bufb;
     char* yb = lds + ((t & 1) ^ 1) * bufb;
     S acc[RPT][NV];
-    G.mul(H, xb, acc);
+    G.mul(H, xb, x1, acc);
     S y[RPT][NV];
-    res_own<S, RPT, NV>(yb, H.nb, y);
+    if constexpr (!OWN) res_own<S, RPT, NV>(yb, H.nb, y);
 #pragma unroll
     for (int k = 0; k < RPT; k++)
 #pragma unroll
-      for (int e = 0; e < NV; e++)
+      for (int e = 0; e < NV; e++) {
+        if constexpr (OWN) y[k][e] = x0[k][e];
         y[k][e] = t > 0 ? fma(acx, acc[k][e], acz * y[k][e]) : acx * acc[k][e];
+      }
     if (cr != 0.0) {
       S r[RPT][NV];  // written by this thread, or by an earlier kernel
 #pragma unroll
@@ -468,6 +534,14 @@ __global__ __launch_bounds__(RES_T) void k_res_xi(ResH<S> H, const S* __restrict
 #pragma unroll
         for (int e = 0; e < NV; e++) y[k][e] = fma(acr, r[k][e], y[k][e]);
     }
+    if constexpr (OWN)
+#pragma unroll
+      for (int k = 0; k < RPT; k++)
+#pragma unroll
+        for (int e = 0; e < NV; e++) {
+          x0[k][e] = x1[k][e];
+          x1[k][e] = y[k][e];
+        }
 #pragma unroll
     for (int k = 0; k < RPT; k++) {
       const int i = k * blockDim.x + threadIdx.x;
@@ -609,16 +683,16 @@ __global__ __launch_bounds__(WG) void k_res_coef(const double* __restrict__ src,
 #endif  // FKD_RES_SHARED
 
 // Entry points of one (storage type, real/complex, block size, rows per
-// thread); [1]: some blocks streamed, [0]: every block of a row in registers
-// (rows of at most dreg_* blocks).
+// thread); first index: ResMode; every block of a row in registers (rows of at
+// most dreg_* blocks) except with RES_ST.
 template <class S>
 struct ResSet {
   void (*pack)(const int*, const int*, const S*, int, int, int, S*, int*) = nullptr;
-  void (*fwd[2])(ResH<S>, const S*, int, S*, size_t, int) = {};
+  void (*fwd[3])(ResH<S>, const S*, int, S*, size_t, int) = {};
   // second index 1: own rows of alpha in LDS (four buffers instead of two)
-  void (*bwd[2][2])(ResH<S>, const S*, S*, size_t, int, const double*, double) = {};
-  void (*xi[2])(ResH<S>, const S*, int, const S*, const S*, const double*, int, S*, S*) = {};
-  int dreg_fwd[2] = {}, dreg_bwd[2][2] = {}, dreg_xi[2] = {};
+  void (*bwd[3][2])(ResH<S>, const S*, S*, size_t, int, const double*, double) = {};
+  void (*xi[3])(ResH<S>, const S*, int, const S*, const S*, const double*, int, S*, S*) = {};
+  int dreg_fwd[3] = {}, dreg_bwd[3][2] = {}, dreg_xi[3] = {};  // 0: no such kernel
   int elem_bytes = 0;   // one block row of one column
   int block_bytes = 0;  // one H block
 };
