@@ -294,15 +294,15 @@ class HipEngine:
         return out.view(np.complex128).reshape(M, M)
 
     def set_store_alpha(self, mode) -> None:
-        """Keep every forward vector for autodiff_matrix (FKPM_OPT_STORE_ALPHA):
-        True / 2 whenever the table fits, 1 (default) the same but for lattices
-        that run the whole-recursion kernels, False / 0 recompute alpha
-        backward."""
+        """Keep the forward vectors for autodiff_matrix (FKPM_OPT_STORE_ALPHA):
+        True / 2 as far as they fit the table (all, or the first ones from a third
+        of M on), 1 (default) the same but for lattices that run the
+        whole-recursion kernels, False / 0 recompute alpha backward."""
         call("fkpm_set_option", self._h, _capi.OPT_STORE_ALPHA,
              2 if mode is True else 0 if mode is False else int(mode))
 
     def alpha_table(self) -> bool:
-        """Whether the last moments(M) kept its forward vectors."""
+        """Whether the last moments(M) kept its forward vectors (all, or the first)."""
         v = C.c_int()
         call("fkpm_get_alpha_table", self._h, C.byref(v))
         return bool(v.value)

@@ -277,8 +277,8 @@ int fkpm_get_kernel_mfma(fkpm_handle* h, int kind, int* mfma);
  * segments of s workgroup passes.  The autotuner times 0, 1, 2 and 8. */
 int fkpm_get_kernel_sweep(fkpm_handle* h, int kind, int* sweep);
 
-/* *stored = 1 when the last fkpm_moments kept its forward vectors for the
- * next fkpm_autodiff_matrix (FKPM_OPT_STORE_ALPHA). */
+/* *stored = 1 when the last fkpm_moments kept its forward vectors, all or the
+ * first of them, for the next fkpm_autodiff_matrix (FKPM_OPT_STORE_ALPHA). */
 int fkpm_get_alpha_table(fkpm_handle* h, int* stored);
 
 /* Step loops replayed as a hipGraph and graphs captured so far (FKPM_OPT_GRAPH). */
