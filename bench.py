@@ -176,6 +176,14 @@ def run_gpu(H, groups, cfg, prec: str, steps: int, warmup: int, seed: int, tune:
     wall = time.perf_counter() - t_all
     eng.set_timing(False)
     stoch_method = eng.stoch_method()  # from the kept forward vectors, or Clenshaw
+    whole_recursion = eng.whole_recursion()
+    launches = sum(n for _, n in tot.values())
+    if whole_recursion:  # one launch a recursion: count its Chebyshev steps instead
+        table = stoch_method == "table"  # the pass over the table counted as one
+        for kind, n in (("moments", M // 2), ("autodiff", M // 2 - 1),
+                        ("stoch", (M + 1) // 2 + 1 if table else M - 1)):
+            if tot[kind][1] <= 2 * steps:
+                tot[kind][1] = n * steps
     energy = float(np.dot(cE, mu))
     # the device-to-host copy of one D (pageable host memory, as a caller's
     # SpMatBsr holds it): two of them are inside every timed step
@@ -193,7 +201,8 @@ def run_gpu(H, groups, cfg, prec: str, steps: int, warmup: int, seed: int, tune:
     return dict(eng=eng, es=es, N=N, S=S, M=M, mu=mu, energy=energy, wall=wall, times=times,
                 kernel_ms=tot, Dg=Dg.val.copy(), Ds=Ds.val.copy(), config=eng.config(),
                 kernel_config=kcfg, tune_s=t_tune, state=eng.state(), alpha_table=alpha_table,
-                stoch_method=stoch_method, d2h_ms=d2h_ms,
+                stoch_method=stoch_method, d2h_ms=d2h_ms, launches=launches,
+                whole_recursion=whole_recursion,
                 energy_scale_s=None if "es" in cfg else t_es)
 
 
@@ -423,17 +432,19 @@ def conductivity_leg(H, groups, cfg, es, seed: int, M2: int, reps: int = 2) -> d
 def small_solve_leg(name: str, seed: int, reps: int = 20) -> dict:
     """Wall time of one full solve (moments + autodiff_matrix + stoch_matrix,
     both D's to the host) of a workload too small to fill the GPU (C1: 1024
-    orbitals x 16 probe columns), where the per-step launches, not HBM, set
-    the time: compared with the sum of the step kernels' device time."""
+    orbitals x 16 probe columns), where launches and latency, not HBM, set
+    the time: compared with the sum of the recursions' device time."""
     H, groups, cfg = build_workload(name, seed)
     r = run_gpu(H, groups, cfg, "fp64", reps, 2, seed, tune=False)
     wall_ms = 1e3 * r["wall"] / reps
-    launches = sum(n for _, n in r["kernel_ms"].values()) // reps
+    launches = r["launches"] // reps
+    n_steps = sum(n for _, n in r["kernel_ms"].values()) // reps
     dev_ms = sum(ms for ms, _ in r["kernel_ms"].values()) / reps
     return {"workload": f"{name}: {WORKLOADS[name]}", "N": r["N"], "S": r["S"], "M": r["M"],
             "solve_ms": round(wall_ms, 3), "step_launches_per_solve": int(launches),
             "step_loops_device_ms": round(dev_ms, 3),
-            "us_per_step_launch": round(1e3 * dev_ms / max(launches, 1), 2),
+            "whole_recursion": r["whole_recursion"], "steps_per_solve": int(n_steps),
+            "us_per_step": round(1e3 * dev_ms / max(n_steps, 1), 2),
             "energy": r["energy"]}
 
 
@@ -568,7 +579,10 @@ def main(argv=None) -> int:
     if r["alpha_table"] and dom != "stoch":
         kind += "_table"
     kc = r["kernel_config"][kind]
-    if kc.get("mfma"):
+    if r["whole_recursion"]:
+        names = {"moments": "k_res_forward", "stoch": "k_res_xi", "autodiff": "k_res_backward"}
+        geo = f"b={H.b_len}, a workgroup per column"
+    elif kc.get("mfma"):
         rr = "_rr" if kc.get("mfma_variant") == 2 else ""
         names = {"moments": f"k_mfma_step{rr}", "stoch": f"k_mfma_step{rr} (Clenshaw)",
                  "autodiff": f"k_mfma_autodiff{rr}"}

@@ -52,6 +52,7 @@ SIGNATURES = {
     "fkpm_get_kernel_mfma": (_I, [_P, _I, _IP]),
     "fkpm_get_kernel_sweep": (_I, [_P, _I, _IP]),
     "fkpm_get_alpha_table": (_I, [_P, _IP]),
+    "fkpm_get_whole_recursion": (_I, [_P, _IP]),
     "fkpm_get_stoch_method": (_I, [_P, _IP]),
     "fkpm_get_state": (_I, [_P, _IP, _IP, _IP]),
     "fkpm_get_graph_stats": (_I, [_P, C.POINTER(C.c_longlong), C.POINTER(C.c_longlong)]),

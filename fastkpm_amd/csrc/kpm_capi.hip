@@ -1433,7 +1433,7 @@ int res_moments(fkpm_handle* h, int M, double* mu, bool* done) {
   CHK(timing_begin(h));
   CHK(launch_lds(rs.fwd[res_mode(h->max_deg, rs.dreg_fwd)], dim3(h->s), dim3(h->res.threads), res_lds<S>(h), h->stream,
                  res_H<S>(h), h->R.as<const S>(), h->sp, h->res.atab.as<S>(), slot, nsteps));
-  CHK(timing_end(h, &h->ms_mom, &h->n_mom, nsteps));
+  CHK(timing_end(h, &h->ms_mom, &h->n_mom, 1));
   CHK(launch(&fkd::k_res_dots<S>, dim3(nsteps, ny), dim3(fkd::WG), h->stream,
              h->res.atab.as<const S>(), slot, cnt, h->partial.as<double>()));
   double* ps = static_cast<double*>(h->res.pin.p);
@@ -1492,7 +1492,7 @@ int res_autodiff(fkpm_handle* h, int M, const double* c, double diag) {
   fkd::ResTerms<S> T{h->res.atab.as<const S>(), h->res.btab.as<const S>(), slot, M2, diag,
                      2 * c[M - 1]};
   CHK(res_outer<S>(h, T, M2 > 1 ? M2 + 1 : 1, h->dacc.as<double>()));
-  return timing_end(h, &h->ms_ad, &h->n_ad, M2 - 1);
+  return timing_end(h, &h->ms_ad, &h->n_ad, M2 > 1 ? 1 : 0);
 }
 
 // xi by the Clenshaw recurrence, or from the resident table, then D into dout.
@@ -1826,7 +1826,7 @@ int stoch_t(fkpm_handle* h, int M, const double* c) {
     h->stoch_used = table ? FKPM_STOCH_TABLE : FKPM_STOCH_CLENSHAW;
     CHK(timing_begin(h));
     CHK(res_stoch<S>(h, M, c, table));
-    CHK(timing_end(h, &h->ms_stoch, &h->n_stoch, table ? (M + 1) / 2 + 1 : M - 1));
+    CHK(timing_end(h, &h->ms_stoch, &h->n_stoch, table ? 2 : 1));
     h->alpha_M = 0;
     return 0;
   }
@@ -2865,6 +2865,12 @@ int fkpm_get_kernel_mfma(fkpm_handle* h, int kind, int* mfma) {
 int fkpm_get_alpha_table(fkpm_handle* h, int* stored) {
   if (!h || !stored) return fail(FKPM_E_ARG, "null argument");
   *stored = (h->a_slots > 0 && h->alpha_M > 0) ? 1 : 0;
+  return 0;
+}
+
+int fkpm_get_whole_recursion(fkpm_handle* h, int* on) {
+  if (!h || !on) return fail(FKPM_E_ARG, "null argument");
+  *on = h->res.state ? 1 : 0;
   return 0;
 }
 

@@ -302,9 +302,16 @@ class HipEngine:
              2 if mode is True else 0 if mode is False else int(mode))
 
     def alpha_table(self) -> bool:
-        """Whether the last moments(M) kept its forward vectors (all, or the first)."""
+        """Whether the last moments(M) kept its forward vectors (all, or the first)
+        for the step kernels (the whole-recursion kernels always keep theirs)."""
         v = C.c_int()
         call("fkpm_get_alpha_table", self._h, C.byref(v))
+        return bool(v.value)
+
+    def whole_recursion(self) -> bool:
+        """Whether the last moments(M) ran as one whole-recursion kernel."""
+        v = C.c_int()
+        call("fkpm_get_whole_recursion", self._h, C.byref(v))
         return bool(v.value)
 
     def set_sweep(self, sweep: int) -> None:

@@ -137,7 +137,8 @@ int fkpm_get_D(fkpm_handle* h, void* D_val);
 /* Per-call timing of the dominant recursion kernels, measured with HIP events
  * on the handle's stream when enabled: total milliseconds and launch counts of
  * the Chebyshev step kernels of the last fkpm_moments / fkpm_stoch_matrix /
- * fkpm_autodiff_matrix call. */
+ * fkpm_autodiff_matrix call: one launch per step (and one for the table sums of
+ * FKPM_STOCH_TABLE), or one per recursion where a whole-recursion kernel ran. */
 int fkpm_set_timing(fkpm_handle* h, int on);
 int fkpm_get_timing(fkpm_handle* h, double* ms_moments, int* n_moments, double* ms_stoch,
                     int* n_stoch, double* ms_autodiff, int* n_autodiff);
@@ -258,11 +259,14 @@ int fkpm_set_option(fkpm_handle* h, int option, int value);
 /* Autotune the geometry (lanes per block row, packets per lane, workgroup
  * count, nontemporal hints) of every kernel kind on the current H and R by
  * timing the candidates on the device; the result is kept for this handle and
- * for every later handle of the same problem shape in the process.  Discards
- * the moments state.  No counterpart in the reference. */
+ * for every later handle of the same problem shape in the process.  The
+ * whole-recursion kernels have no geometry to tune and stay in use where they
+ * run.  Discards the moments state.  No counterpart in the reference. */
 int fkpm_autotune(fkpm_handle* h);
 
-/* Geometry in use for one kernel kind. */
+/* Geometry in use for one kernel kind; where the whole-recursion kernels run
+ * (fkpm_get_whole_recursion) the step kernels' geometry, which the other calls
+ * (fkpm_moments2, FKPM_STOCH_FORWARD) use. */
 int fkpm_get_kernel_config(fkpm_handle* h, int kind, int* lanes, int* kq, int* n_wg, int* nt);
 
 /* *mfma = 0 if that kernel kind runs on the vector units, 1 on the matrix
@@ -278,8 +282,16 @@ int fkpm_get_kernel_mfma(fkpm_handle* h, int kind, int* mfma);
 int fkpm_get_kernel_sweep(fkpm_handle* h, int kind, int* sweep);
 
 /* *stored = 1 when the last fkpm_moments kept its forward vectors, all or the
- * first of them, for the next fkpm_autodiff_matrix (FKPM_OPT_STORE_ALPHA). */
+ * first of them, for the step kernels of the next fkpm_autodiff_matrix
+ * (FKPM_OPT_STORE_ALPHA); 0 where the whole-recursion kernels ran, which always
+ * keep theirs (fkpm_get_whole_recursion). */
 int fkpm_get_alpha_table(fkpm_handle* h, int* stored);
+
+/* *on = 1 when the last fkpm_moments ran as a whole-recursion kernel (small
+ * lattices with every switch that names a step kernel at its default), which keeps
+ * all its forward vectors in a table of its own for fkpm_autodiff_matrix and
+ * fkpm_stoch_matrix.  No counterpart in the reference. */
+int fkpm_get_whole_recursion(fkpm_handle* h, int* on);
 
 /* Step loops replayed as a hipGraph and graphs captured so far (FKPM_OPT_GRAPH). */
 int fkpm_get_graph_stats(fkpm_handle* h, long long* launches, long long* captures);
