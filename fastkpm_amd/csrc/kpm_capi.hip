@@ -1279,16 +1279,26 @@ void stoch_table3_weights(int M, const double* c, std::vector<double>& w) {
 // LDS of one workgroup.
 constexpr size_t kLdsBytes = 160 << 10;
 // Bytes of H beyond its registers that a workgroup of the backward recursion may
-// read from the L2 in every step.  A call of M = 128 (us, resident against the
-// step kernels; S columns):
-//                       KiB streamed   moments      autodiff_matrix
-//   32x32 x 2, S 32           267     127 / 386      271 / 640
-//   12^3 x 2, S 16            803     407 / 423      618 / 694
-//   8^3 x 4, S 32             910     481 / 580      670 / 1650
-//   64^2 x 1, S 16            320     227 / 400      633 / 521
-// so up to 1 MiB the two calls together gain; past it (14^3 x 2 and larger) a
-// column no longer fits the LDS twice in FP64.
+// read from the L2 in every step (most of H at a column that still fits the LDS twice).
 constexpr size_t kResStream = 1024 << 10;
+
+// 16-byte L2 loads of H (smaller blocks: one each) a thread may have in a forward
+// step, where it owns four rows or more, or two of 4x4 blocks; with fewer rows the
+// streamed loads of a step overlap.  Every row is padded to the longest one, so an
+// uneven pattern streams far more than it holds.  moments / moments + autodiff_matrix
+// of M = 128 (us), whole recursion against step kernels, by loads:
+//   b = 1  2000 rows of 19, FP64        44    518 / 556     1235 / 1351
+//          2000 rows of 27, FP32        48    541 / 629     1223 / 1703
+//          2000 rows, hub of 21         52    580 / 420     1271 / 1108
+//          4000 rows, hub of 11         64    460 / 357     1410 / 835
+//          4000 rows of 13              80    534 / 446     1655 / 1029
+//          3000 rows of 27, real       160   1379 / 589     3004 / 1509
+//   b = 2  1000 rows, hub of 17 (two)   96    495 / 576     1061 / 1429
+//          1500 rows of 9              112    452 / 379     1189 / 959
+//          1100 rows, hub of 15        208    684 / 432     1450 / 1114
+//   b = 4  900 rows of 9, FP32         112    536 / 829     1202 / 2437
+//          600 rows of 5               128    506 / 429     1212 / 1193
+constexpr int res_max_loads(int b) { return b == 1 ? 48 : b == 2 ? 104 : 120; }
 
 bool find_res(fkpm_handle* h, int rpt) {
   if (h->single)
@@ -1310,6 +1320,19 @@ int res_mode(int deg, const int (&dreg)[3]) {
   return deg <= dreg[fkd::RES_OWN] ? fkd::RES_OWN
          : deg <= dreg[fkd::RES_REG] ? fkd::RES_REG
                                      : fkd::RES_ST;
+}
+
+// Blocks of a row it streams.
+int res_streamed(int deg, const int (&dreg)[3]) {
+  return res_mode(deg, dreg) == fkd::RES_ST ? deg - dreg[fkd::RES_ST] : 0;
+}
+
+// The streamed 16-byte loads of a thread in a step, 0 where its rows are few enough
+// for them to overlap.
+template <class S>
+int res_loads(fkpm_handle* h, int rpt, const int (&dreg)[3]) {
+  if (rpt < (h->b == 4 ? 2 : 4)) return 0;
+  return res_streamed(h->max_deg, dreg) * rpt * std::max(1, h->rset<S>().block_bytes / 16);
 }
 
 // The backward recursion's kernel: the thread's rows of the forward vectors in
@@ -1335,7 +1358,7 @@ ResBwd res_bwd(fkpm_handle* h) {
 // Whether the whole-recursion kernels run for the current H and R: the
 // defaults of every switch that names a step kernel or the table (a forced
 // geometry, sweep, order, graph or table mode asks for the step kernels), and a
-// column that fits the LDS twice with little of H left to stream.
+// column that fits the LDS twice with little of H left to stream (res_max_loads).
 template <class S>
 bool res_wanted(fkpm_handle* h) {
   if (h->force_L > 0 || h->max_wg > 0 || h->sweep_force >= 0 || h->slice_force >= 0 ||
@@ -1349,6 +1372,7 @@ bool res_wanted(fkpm_handle* h) {
   if (!find_res(h, rpt)) return false;
   const fkd::ResSet<S>& rs = h->rset<S>();
   if (2 * ((size_t)(h->nb + 1) * rs.elem_bytes + 16) > kLdsBytes) return false;
+  if (res_loads<S>(h, rpt, rs.dreg_fwd) > res_max_loads(h->b)) return false;
   const int threads = ((h->nb + rpt - 1) / rpt + 63) / 64 * 64;
   const ResBwd rb = res_bwd<S>(h);
   if (rb.mode == fkd::RES_ST) {

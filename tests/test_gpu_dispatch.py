@@ -69,3 +69,56 @@ def test_timing_counts_the_launches_of_either_path(oracle, whole):
     eng.autodiff_matrix(c[:2], D)
     assert eng.timing()["moments_launches"] == 1 and eng.timing()["autodiff_launches"] == 0
     eng.close()
+
+
+def _pattern(nb, b, reach=0, hub=0, real=False, seed=5):
+    """Random Hermitian blocks on a periodic chain of nb sites: neighbours up to
+    `reach` away and, for site 0, `hub` more (the rows then have uneven lengths)."""
+    from fastkpm_amd import lattice
+    rng = np.random.default_rng(seed)
+    i = np.arange(nb)
+    pairs = [np.stack([i, (i + d) % nb]) for d in range(1, reach + 1)]
+    if hub:
+        pairs.append(np.stack([np.zeros(hub, dtype=int),
+                               np.sort(rng.choice(np.arange(reach + 1, nb - reach), hub, False))]))
+    r, c = np.concatenate(pairs, axis=1)
+    T = rng.standard_normal((len(r), b, b)) + (0 if real else 1j) * rng.standard_normal((len(r), b, b))
+    X = rng.standard_normal((nb, b, b)) + (0 if real else 1j) * rng.standard_normal((nb, b, b))
+    X = X + np.conj(X.transpose(0, 2, 1))
+    return lattice.coo_to_bsr(nb, b, np.concatenate([i, r, c]), np.concatenate([i, c, r]),
+                              np.concatenate([X, T, np.conj(T.transpose(0, 2, 1))]),
+                              np.float64 if real else np.complex128)
+
+
+def _check_all(oracle, eng, orc, H, M, bound, tol=FP64_TOL):
+    """moments, autodiff_matrix and stoch_matrix (from the kept vectors, and by the
+    recurrence) against the oracle."""
+    c = fermi_coeffs(oracle, M, -bound, bound, kT=0.05)
+    D = H.like(eng.np_dtype)
+    assert rel_err(eng.moments(M), orc.moments(M)) < tol
+    eng.autodiff_matrix(c, D)
+    assert rel_err(D.val, orc.autodiff_matrix(c, H)) < tol
+    s = orc.stoch_matrix(c, H)
+    eng.stoch_matrix(c, D)
+    assert rel_err(D.val, s) < tol
+    eng.set_stoch_method("clenshaw")
+    eng.stoch_matrix(c, D)
+    assert rel_err(D.val, s) < tol
+    eng.set_stoch_method("auto")
+
+
+# (rows, block size, reach, hub bonds, real, whole recursion): either side of the
+# loads a thread may stream, rows padded to a hub's length among them
+@pytest.mark.parametrize("nb,b,reach,hub,real,whole", [
+    (2000, 1, 9, 0, False, True), (2000, 1, 2, 16, False, False),
+    (3000, 1, 4, 0, False, True), (3000, 1, 6, 0, False, False), (3000, 1, 2, 10, False, False),
+    (3000, 1, 13, 0, True, False), (1000, 1, 2, 40, False, True),
+    (1500, 2, 3, 0, False, True), (1500, 2, 4, 0, False, False), (1000, 2, 2, 12, False, True),
+    (1100, 2, 2, 10, False, False), (500, 4, 3, 0, False, True), (600, 4, 2, 0, False, False)])
+def test_rows_too_long_for_the_whole_recursion(oracle, nb, b, reach, hub, real, whole):
+    H = _pattern(nb, b, reach, hub, real)
+    eng, orc, bound = _set_up(oracle, H, 3, real=real)
+    _check_all(oracle, eng, orc, H, 12, bound)
+    eng.moments(2)
+    assert eng.whole_recursion() is whole
+    eng.close()
