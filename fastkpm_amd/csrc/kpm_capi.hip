@@ -1355,6 +1355,28 @@ ResBwd res_bwd(fkpm_handle* h) {
                 la ? 2 * lds : lds};
 }
 
+// Streamed blocks of a workgroup and step from which autodiff_matrix leaves the
+// backward recursion to the step kernels, where the forward vectors do not fit the LDS
+// beside its own (FP64 complex) and a thread has all its rows: it then streams nearly
+// all of H.  autodiff_matrix of M = 128 (us), whole recursion / step kernels recomputing
+// alpha from the last two forward vectors:
+//   40x40 x 2       8000   478 / 494 (S = 4)   810 / 861 (S = 128)
+//   11^3 x 2        9317   590 / 609           917 / 968
+//   1500 x 2, 7     10500  612 / 536           673 / 601 (S = 32)
+//   57x57 x 1       12996  506 / 399           834 / 772
+//   64x64 x 1       16384  538 / 379          1722 / 1480 (S = 256)
+//   15^3 x 1        20250  693 / 472 (S = 16) 1074 / 930
+constexpr int kResBwdBlocks = 10240;
+
+template <class S>
+bool res_bwd_wanted(fkpm_handle* h) {
+  const ResBwd rb = res_bwd<S>(h);
+  if (rb.mode != fkd::RES_ST || rb.la || h->b == 4 || h->res.rpt < fkd::res_max_rpt(h->b))
+    return true;
+  const int d = h->max_deg - h->rset<S>().dreg_bwd[fkd::RES_ST][0];
+  return (long long)d * h->nb <= kResBwdBlocks;
+}
+
 // Whether the whole-recursion kernels run for the current H and R: the
 // defaults of every switch that names a step kernel or the table (a forced
 // geometry, sweep, order, graph or table mode asks for the step kernels), and a
@@ -1497,6 +1519,18 @@ int res_outer(fkpm_handle* h, const fkd::ResTerms<S>& T, int nterm, double* dst)
   if (h->b == 4) rc = h->cx ? go(&fkd::k_res_outer<S, true, 4>) : go(&fkd::k_res_outer<S, false, 4>);
   CHK(rc);
   return sum_parts(h, h->res.part.as<const double>(), (int)ny, cnt, dst, false);
+}
+
+// alpha_{M/2-1} and alpha_{M/2} of the resident table into the step kernels' ring.
+template <class S>
+int res_to_ring(fkpm_handle* h, int M) {
+  const dim3 grid((h->n + fkd::RES_TILE - 1) / fkd::RES_TILE,
+                  (h->sp + fkd::RES_TILE - 1) / fkd::RES_TILE);
+  for (int k = M / 2 - 1; k <= M / 2; k++)
+    CHK(launch(h->cx ? &fkd::k_res_to_rows<S, true> : &fkd::k_res_to_rows<S, false>, grid,
+               dim3(fkd::WG), h->stream, h->res.atab.as<const S>() + (size_t)k * res_slot(h), h->n,
+               h->s, h->sp, h->A[k % 3].as<S>()));
+  return 0;
 }
 
 // The backward recursion and D from the resident table, into dacc.
@@ -1950,8 +1984,11 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
   double diag = c[1];
   for (int m = 1; m < M / 2; m++) diag -= c[2 * m + 1];
   if (h->res.state) {
-    CHK(res_autodiff<S>(h, M, c, diag));
-    return finish_autodiff(h);
+    if (M == 2 || res_bwd_wanted<S>(h)) {
+      CHK(res_autodiff<S>(h, M, c, diag));
+      return finish_autodiff(h);
+    }
+    CHK(res_to_ring<S>(h, M));  // and on with the ring's steps
   }
   CHK(zero_doubles(h, dacc, dcount));
   // D = diag R R^+

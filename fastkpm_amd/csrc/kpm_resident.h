@@ -674,6 +674,33 @@ __global__ __launch_bounds__(WG) void k_res_outer(const int* __restrict__ drp,
   for (int e = 0; e < NH; e++) o[e] = acc[e];
 }
 
+// A slot of the table (column by column, n elements each, s of them) as a vector of
+// the step kernels: n rows of sp elements, zero from column s on.  32 x 32 tiles
+// through LDS, both sides in runs of 32 elements; two vectors a call.
+constexpr int RES_TILE = 32;
+template <typename S, bool CX>
+__global__ __launch_bounds__(WG) void k_res_to_rows(const S* __restrict__ src, int n, int s,
+                                                    int sp, S* __restrict__ dst) {
+  struct E {
+    S v[CX ? 2 : 1];
+  };
+  __shared__ E t[RES_TILE][RES_TILE + 1];
+  const int r0 = blockIdx.x * RES_TILE, c0 = blockIdx.y * RES_TILE;
+  const int x = threadIdx.x % RES_TILE, y = threadIdx.x / RES_TILE;
+#pragma unroll
+  for (int k = y; k < RES_TILE; k += WG / RES_TILE) {
+    E e{};
+    if (r0 + x < n && c0 + k < s)
+      e = reinterpret_cast<const E*>(src)[(size_t)(c0 + k) * n + r0 + x];
+    t[k][x] = e;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = y; k < RES_TILE; k += WG / RES_TILE)
+    if (r0 + k < n && c0 + x < sp)
+      reinterpret_cast<E*>(dst)[(size_t)(r0 + k) * sp + c0 + x] = t[x][k];
+}
+
 // n doubles from pinned host memory (the coefficients of a call).
 __global__ __launch_bounds__(WG) void k_res_coef(const double* __restrict__ src,
                                                  double* __restrict__ dst, int n) {

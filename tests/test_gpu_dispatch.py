@@ -122,3 +122,37 @@ def test_rows_too_long_for_the_whole_recursion(oracle, nb, b, reach, hub, real, 
     eng.moments(2)
     assert eng.whole_recursion() is whole
     eng.close()
+
+
+# (lattice, block size, columns, real, M, backward recursion as one launch): either
+# side of the streamed blocks at which autodiff_matrix goes to the step kernels
+@pytest.mark.parametrize("shape,b,S,real,M,whole", [
+    ((50, 50), 1, 3, False, 8, True), ((57, 57), 1, 3, False, 8, False),
+    ((64, 64), 1, 1, False, 4, False), ((64, 64), 1, 33, False, 10, False),
+    ((14, 14, 14), 1, 17, False, 6, False), ((64, 64), 1, 5, True, 8, True),
+    ((40, 40), 2, 3, False, 8, True), ((11, 11, 11), 2, 5, False, 6, True),
+    ((12, 12, 12), 2, 31, False, 6, False), ((12, 12, 12), 2, 2, False, 2, True)])
+@pytest.mark.parametrize("own_pattern", [True, False])
+def test_backward_recursion_of_streamed_lattices(oracle, shape, b, S, real, M, whole, own_pattern):
+    from fastkpm_amd import lattice
+    H = lattice.lattice(shape, b=b, seed=7, W=1.0, J=0.0 if b == 1 else 1.0,
+                        dtype=np.float64 if real else np.complex128)
+    eng, orc, bound = _set_up(oracle, H, S, real=real)
+    eng.set_timing(True)
+    nb = H.n_rows
+    Dp = H if own_pattern else lattice.coo_to_bsr(nb, b, range(nb), range(nb), np.zeros((nb, b, b)))
+    D = Dp.like(eng.np_dtype)
+    c = fermi_coeffs(oracle, M, -bound, bound, kT=0.05)
+    mu_o = orc.moments(M)
+    d_o = orc.autodiff_matrix(c, Dp)
+    for _ in range(3):  # the step loop is captured, then replayed
+        assert rel_err(eng.moments(M), mu_o) < FP64_TOL
+        assert eng.whole_recursion()
+        eng.autodiff_matrix(c, D)
+        assert eng.timing()["autodiff_launches"] == (0 if M == 2 else 1 if whole else M // 2 - 1)
+        assert rel_err(D.val, d_o) < FP64_TOL
+    # the resident table is still whole
+    eng.stoch_matrix(c, D)
+    assert eng.stoch_method() == "table"
+    assert rel_err(D.val, orc.stoch_matrix(c, Dp)) < FP64_TOL
+    eng.close()
