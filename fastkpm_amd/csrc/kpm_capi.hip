@@ -1408,6 +1408,26 @@ bool res_wanted(fkpm_handle* h) {
   return true;
 }
 
+// Whether stoch_matrix without a table runs as one launch: not where a step waits for
+// streamed blocks longer than the step kernels' launches and columns take.
+// stoch_matrix by the Clenshaw recurrence with set_H, M = 128 (us), whole recursion /
+// step kernels, by blocks streamed a row:
+//   64x64 x 1    2   619 / 621 (S = 4)   627 / 857 (S = 64)
+//   45x42 x 2    3   704 / 676 (16)      725 / 985 (128)
+//   13^3 x 1     4   838 / 664 (4)       844 / 731 (32)    865 / 1125 (128)
+//   12^3 x 2     5   890 / 807 (16)      895 / 904 (32)    896 / 1055 (64)
+//   3000 x 1, 9  6  1127 / 748 (4)      1145 / 857 (32)
+//   1500 x 1, 17 9   881 / 799 (4)       888 / 792 (32)
+//   FP32 x 2 and b = 4 gained at every size: 1900 rows of 9 636 / 968, 8^3 x 4 1004 / 1142
+// The step kernels' time grows with the vector from about 512 KiB a streamed block.
+template <class S>
+bool res_clenshaw_wanted(fkpm_handle* h) {
+  const int d = res_streamed(h->max_deg, h->rset<S>().dreg_xi);
+  const int loads = res_loads<S>(h, h->res.rpt, h->rset<S>().dreg_xi);
+  const bool waits = h->b == 1 ? loads >= 32 : h->b == 2 && !h->single && loads >= 80;
+  return !waits || h->vbytes() >= (size_t)d * (512 << 10);
+}
+
 // The tables of forward and backward vectors, within the budget of the step
 // kernels' table (moments_t).
 int res_tables(fkpm_handle* h, size_t abytes, size_t bbytes, bool* ok) {
@@ -1879,8 +1899,10 @@ int stoch_t(fkpm_handle* h, int M, const double* c) {
   const size_t dcount = (size_t)h->nnzbD * h->b * h->b * (h->cx ? 2 : 1);
   const KCfg& ko = h->kc[K_OUT];
   const auto& kso = h->ks<S>(K_OUT);
-  if (h->stoch_method != FKPM_STOCH_FORWARD && res_wanted<S>(h)) {
-    const bool table = h->stoch_method == FKPM_STOCH_AUTO && h->res.K >= (M + 1) / 2;
+  const bool res_table = h->stoch_method == FKPM_STOCH_AUTO && h->res.K >= (M + 1) / 2;
+  if (h->stoch_method != FKPM_STOCH_FORWARD && res_wanted<S>(h) &&
+      (res_table || res_clenshaw_wanted<S>(h))) {
+    const bool table = res_table;
     h->stoch_used = table ? FKPM_STOCH_TABLE : FKPM_STOCH_CLENSHAW;
     CHK(timing_begin(h));
     CHK(res_stoch<S>(h, M, c, table));

@@ -156,3 +156,37 @@ def test_backward_recursion_of_streamed_lattices(oracle, shape, b, S, real, M, w
     assert eng.stoch_method() == "table"
     assert rel_err(D.val, orc.stoch_matrix(c, Dp)) < FP64_TOL
     eng.close()
+
+
+# (lattice, block size, columns, precision, one launch): either side of the streamed
+# blocks and the vector size at which the Clenshaw recurrence goes to the step kernels
+@pytest.mark.parametrize("shape,b,S,prec,whole", [
+    ((64, 64), 1, 3, "fp64", True), ((13, 13, 13), 1, 3, "fp64", False),
+    ((13, 13, 13), 1, 64, "fp64", True), ((45, 42), 2, 5, "fp64", True),
+    ((12, 12, 12), 2, 5, "fp64", False), ((12, 12, 12), 2, 5, "fp32", True),
+    ((8, 8, 8), 4, 2, "fp64", True)])
+@pytest.mark.parametrize("dense", [True, False])
+def test_clenshaw_of_streamed_lattices(oracle, shape, b, S, prec, whole, dense):
+    from fastkpm_amd import lattice
+    H = lattice.lattice(shape, b=b, seed=9, W=1.0, J=1.0 if b == 2 else 0.0, orbital_blocks=b > 2)
+    eng, orc, bound = _set_up(oracle, H, S, prec=prec, dense=dense)
+    eng.set_timing(True)
+    M = 11
+    c = fermi_coeffs(oracle, M, -bound, bound, kT=0.05, kind=1)
+    D = H.like()
+    # FP32: M recursion steps of 16 roundings each
+    tol = FP64_TOL if prec == "fp64" else M * 16 * 2.0 ** -24
+    for m in (M, 2):
+        s = orc.stoch_matrix(c[:m], H)
+        for _ in range(3):
+            eng.stoch_matrix(c[:m], D)
+            assert eng.stoch_method() == "clenshaw"
+            assert eng.timing()["stoch_launches"] == (1 if whole else m - 1)
+            assert rel_err(D.val, s) < tol
+    assert eng.state()["r_compact"] is (not dense)
+    # a table of the same R and H is used by the whole-recursion kernels on either side
+    eng.moments(M + 1)
+    eng.stoch_matrix(c, D)
+    assert eng.stoch_method() == "table" and eng.timing()["stoch_launches"] == 2
+    assert rel_err(D.val, orc.stoch_matrix(c, H)) < tol
+    eng.close()
