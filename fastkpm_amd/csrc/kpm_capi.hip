@@ -1428,12 +1428,12 @@ bool res_clenshaw_wanted(fkpm_handle* h) {
   return !waits || h->vbytes() >= (size_t)d * (512 << 10);
 }
 
-// The tables of forward and backward vectors, within the budget of the step
-// kernels' table (moments_t).
+// Room for the tables of forward and (allocated by autodiff_matrix) backward vectors,
+// within the budget of the step kernels' table (moments_t).
 int res_tables(fkpm_handle* h, size_t abytes, size_t bbytes, bool* ok) {
   fkpm_handle::Resident& r = h->res;
   size_t budget = ~(size_t)0;
-  if (abytes > r.atab.bytes || bbytes > r.btab.bytes) {
+  if (abytes > r.atab.bytes) {
     size_t free_b = 0, total_b = 0;
     HIPCHK(hipMemGetInfo(&free_b, &total_b));
     budget = std::min(free_b / 2 + r.atab.bytes + r.btab.bytes, total_b / 4);
@@ -1441,8 +1441,7 @@ int res_tables(fkpm_handle* h, size_t abytes, size_t bbytes, bool* ok) {
   if (const char* e = getenv("FKPM_ALPHA_TABLE_BYTES")) budget = (size_t)strtoull(e, nullptr, 10);
   *ok = abytes + bbytes <= budget;
   if (!*ok) return 0;
-  CHK(r.atab.ensure(abytes));
-  return r.btab.ensure(bbytes);
+  return r.atab.ensure(abytes);
 }
 
 template <class S>
@@ -2006,7 +2005,9 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
   double diag = c[1];
   for (int m = 1; m < M / 2; m++) diag -= c[2 * m + 1];
   if (h->res.state) {
-    if (M == 2 || res_bwd_wanted<S>(h)) {
+    // without room for the backward vectors (taken since moments) too, the ring serves
+    const size_t bytes = (size_t)(M / 2) * res_slot(h) * sizeof(S);
+    if (M == 2 || (res_bwd_wanted<S>(h) && h->res.btab.ensure(bytes) == 0)) {
       CHK(res_autodiff<S>(h, M, c, diag));
       return finish_autodiff(h);
     }

@@ -190,3 +190,30 @@ def test_clenshaw_of_streamed_lattices(oracle, shape, b, S, prec, whole, dense):
     assert eng.stoch_method() == "table" and eng.timing()["stoch_launches"] == 2
     assert rel_err(D.val, orc.stoch_matrix(c, H)) < tol
     eng.close()
+
+
+def test_moments_alone_holds_one_table(oracle):
+    """The table of backward vectors is autodiff_matrix's: moments allocates only the
+    forward one (M/2 + 1 vectors), autodiff_matrix as much again."""
+    import ctypes
+    from fastkpm_amd import _capi, lattice
+
+    def free():  # of the runtime that the library itself is linked to
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert _capi.lib().hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    H = lattice.lattice((16, 16), b=2, seed=3, J=1.0)
+    S, M = 256, 512
+    eng, _, bound = _set_up(oracle, H, S)
+    table = (M // 2 + 1) * H.n_rows * 2 * S * 16  # 539 MB
+    eng.moments(2)
+    used = [free()]
+    eng.moments(M)
+    assert eng.whole_recursion()
+    used.append(free())
+    eng.autodiff_matrix(fermi_coeffs(oracle, M, -bound, bound), H.like())
+    used.append(free())
+    assert 0.9 * table < used[0] - used[1] < 1.5 * table
+    assert 0.9 * table < used[1] - used[2] < 1.5 * table
+    eng.close()
