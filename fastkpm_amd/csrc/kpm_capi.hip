@@ -1682,12 +1682,20 @@ int moments_t(fkpm_handle* h, int M, double* mu) {
 // A large copy to pageable memory runs at the rate of one core copying out of
 // pinned memory (17 GB/s), a third of the link's: from kBigCopy on, four threads
 // copy chunks out of a ring of pinned buffers while the next chunks arrive
-// (117 MB: 6.9 -> 2.7 ms).
+// (117 MB: 6.9 -> 2.7 ms).  Memory that the runtime knows (pinned, registered) takes
+// the link's full rate by itself (57 MB: 1.0 ms, through the ring 1.5).
 constexpr size_t kBigCopy = 16 << 20, kCopyChunk = 2 << 20;
 constexpr int kCopyThreads = 4;
 
+bool pageable(const void* p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+  (void)hipGetLastError();  // not an address of the runtime's: no error of ours
+  return true;
+}
+
 int copy_to_host(fkpm_handle* h, void* dst, const void* src, size_t bytes) {
-  if (bytes < kBigCopy) {
+  if (bytes < kBigCopy || !pageable(dst)) {
     HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
     return 0;

@@ -217,3 +217,40 @@ def test_moments_alone_holds_one_table(oracle):
     assert 0.9 * table < used[0] - used[1] < 1.5 * table
     assert 0.9 * table < used[1] - used[2] < 1.5 * table
     eng.close()
+
+
+def test_large_D_into_pinned_memory():
+    """A D of 57 MB into pinned and into pageable memory: the same bits, and the pinned
+    copy (one transfer at the link's rate, 0.65 of the time) not through the staging
+    ring of the pageable one (the same time)."""
+    import ctypes
+    import time
+    from fastkpm_amd import EnergyScale, _capi, lattice
+    H = lattice.lattice((20, 20, 20), b=8, seed=3, orbital_blocks=True)
+    eng = _engine()
+    eng.set_R(np.ones((H.n_rows * 8, 1), dtype=np.complex128))
+    eng.set_H(H, EnergyScale(-60.0, 60.0))
+    D = H.like()
+    eng.stoch_matrix([0.5, 0.25, 0.125], D)
+    want = D.val.copy()
+
+    def best():
+        t = []
+        for _ in range(20):
+            t0 = time.perf_counter()
+            eng.get_D(D)
+            t.append(time.perf_counter() - t0)
+        return min(t)
+
+    t_pageable = best()
+    p = ctypes.c_void_p()
+    assert _capi.lib().hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(want.nbytes), 0) == 0
+    D.val = np.frombuffer((ctypes.c_char * want.nbytes).from_address(p.value), dtype=np.complex128)
+    D.val[:] = 0
+    eng.get_D(D)
+    assert np.array_equal(D.val, want)
+    t_pinned = best()
+    D.val = None
+    eng.close()
+    _capi.lib().hipHostFree(p)
+    assert t_pinned < 0.85 * t_pageable, (t_pinned, t_pageable)
