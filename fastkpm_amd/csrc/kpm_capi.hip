@@ -352,6 +352,8 @@ struct fkpm_handle {
                           // in the ring A[3]
   int tab_K = 0;          // atab holds alpha_1 .. alpha_tab_K of the current H and R,
   int tab_M = 0;          // kept by moments(tab_M)
+  int unread = 0;         // moments in a row by the step kernels that no autodiff_matrix or
+                          // stoch_matrix followed
   DevBuf tabc;            // stoch_matrix weights of the table vectors
   std::vector<double> tabc_host;
   int store_alpha = 1;    // FKPM_OPT_STORE_ALPHA: 0 never, 1 auto, 2 whenever the table fits
@@ -754,6 +756,20 @@ KCfg default_cfg(fkpm_handle* h, int kind) {
 // and moments + autodiff_matrix + stoch_matrix 1827 / 1445; 140x120 x 1 1672 / 1667
 // and 2321 / 1921; 256^2 x 2 FP32 forward step 35 / 38, autodiff 107 / 91.
 bool table_wanted(const fkpm_handle* h) { return h->store_alpha != 0; }
+
+// By default not from the third moments on that nothing followed (a density of states,
+// a Monte Carlo walk on energies): the writes to fresh slots cost moments up to 15 %
+// (us, table / ring: 46x46 x 2, S = 8, M = 1024 3053 / 2658; 200x200 real, S = 16, M = 128
+// 465 / 399; 128^2 x 2 FP32, S = 32, M = 256 1089 / 940; the matrix-core steps lose nothing, 12^3 x 8
+// FP32 255 / 292).  Only where the forward step has one launch configuration either
+// way, so that the moments are bitwise the same.
+constexpr int kUnread = 2;
+
+bool table_idle(const fkpm_handle* h) {
+  const KCfg &a = h->kc[K_MOM], &b = h->kc[K_MOMT];
+  return h->store_alpha == 1 && h->unread >= kUnread && a.L == b.L && a.KQ == b.KQ &&
+         a.nwg == b.nwg && a.chunk == b.chunk && a.nt == b.nt && !a.mfma && !b.mfma;
+}
 
 // Process-wide cache of tuned geometries, keyed by the problem shape.
 std::mutex g_tune_mu;
@@ -1617,7 +1633,8 @@ int moments_t(fkpm_handle* h, int M, double* mu) {
   // half the free device memory (or the byte count in FKPM_ALPHA_TABLE_BYTES),
   // else as many as fit from a third of M on, the first ones (64^3 x 2 FP64, S = 128,
   // M = 160, 67 of 80 kept: moments + autodiff_matrix + stoch_matrix 305 -> 258 ms).
-  {
+  h->a_slots = 0;
+  if (table_wanted(h) && !table_idle(h)) {
     const size_t vb = h->vbytes(), need = (size_t)nsteps * vb;
     const int least = (M + 2) / 3;
     // default: half of what is free (the table already held counts as free),
@@ -1635,13 +1652,13 @@ int moments_t(fkpm_handle* h, int M, double* mu) {
     // a held table that serves is not grown for a few slots more
     if (slots < (size_t)nsteps && h->atab.bytes / vb >= (size_t)least)
       slots = std::min(slots, h->atab.bytes / vb);
-    h->a_slots = 0;
-    if (table_wanted(h) && slots >= (size_t)std::min(least, nsteps)) {
+    if (slots >= (size_t)std::min(least, nsteps)) {
       h->tab_K = 0;  // rewritten below (and lost if the table grows)
       CHK(h->atab.ensure(slots * vb));
       h->a_slots = (int)slots;
     }
   }
+  h->unread = std::min(h->unread + 1, kUnread);
   const dim3 block(fkd::WG);
   CHK(timing_begin(h));
   {
@@ -1899,6 +1916,7 @@ int stoch_table3(fkpm_handle* h, int M, const double* c, const S** xi_out) {
 template <class S>
 int stoch_t(fkpm_handle* h, int M, const double* c) {
   h->a_slots = 0;  // the forward method's alpha_k go to the ring
+  h->unread = 0;
   const dim3 block(fkd::WG);
   const int* rp = h->rp.as<const int>();
   const int* ci = h->ci.as<const int>();
@@ -2012,6 +2030,7 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
 
   double diag = c[1];
   for (int m = 1; m < M / 2; m++) diag -= c[2 * m + 1];
+  h->unread = 0;
   if (h->res.state) {
     // without room for the backward vectors (taken since moments) too, the ring serves
     const size_t bytes = (size_t)(M / 2) * res_slot(h) * sizeof(S);

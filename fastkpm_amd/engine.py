@@ -297,7 +297,8 @@ class HipEngine:
         """Keep the forward vectors for autodiff_matrix (FKPM_OPT_STORE_ALPHA):
         True / 2 as far as they fit the table (all, or the first ones from a third
         of M on), 1 (default) the same but for lattices that run the
-        whole-recursion kernels, False / 0 recompute alpha backward."""
+        whole-recursion kernels and for moments in a row that nothing reads,
+        False / 0 recompute alpha backward."""
         call("fkpm_set_option", self._h, _capi.OPT_STORE_ALPHA,
              2 if mode is True else 0 if mode is False else int(mode))
 

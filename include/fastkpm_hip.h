@@ -194,8 +194,14 @@ int fkpm_moments_noalloc(int device, int prec, int nb, int b, int nnzb, const in
                                    first ones and autodiff_matrix recomputes down to them;
                                    1 (default): the same, except that lattices small enough
                                    for the whole-recursion kernels (about 4096 orbital rows)
-                                   run those, with a table of their own; 0: the three-vector
-                                   ring and the recomputation */
+                                   run those, with a table of their own, and that from the
+                                   third fkpm_moments in a row on that no autodiff_matrix or
+                                   stoch_matrix followed the vector-unit kernels keep none
+                                   where the moments are the same bits without; 0: the three-vector ring and the
+                                   recomputation.  Kept vectors stay allocated: by default
+                                   up to a quarter of the device (FKPM_OPT_ALPHA_TABLE_MB),
+                                   M/2 vectors of nb b S elements; the whole-recursion
+                                   kernels hold M/2 + 1 and, after autodiff_matrix, M/2 more */
 #define FKPM_OPT_SWEEP 4        /* value 0: every kernel kind sweeps the rows per XCD; s in
                                    1..64: as one front in segments of s passes per XCD
                                    (fkpm_get_kernel_sweep); -1 (default): the configuration's
@@ -226,7 +232,9 @@ int fkpm_moments_noalloc(int device, int prec, int nb, int b, int nnzb, const in
                                    XCD's L2; results per row are the same as in row order, the
                                    moment sums add in another order; 0: row order; -1
                                    (default): the configuration's own (the tuner's choice,
-                                   else 0).  Patterns of another shape keep row order. */
+                                   else 1 where the vectors of a step exceed the last-level
+                                   cache and a block row holds 4 KiB or more).  Patterns of
+                                   another shape keep row order. */
 #define FKPM_OPT_ALPHA_TABLE_MB 7 /* value >= 0: the most MiB the table of forward vectors
                                    (FKPM_OPT_STORE_ALPHA) may hold on this handle; -1
                                    (default): a quarter of the device's memory and at most

@@ -254,3 +254,39 @@ def test_large_D_into_pinned_memory():
     eng.close()
     _capi.lib().hipHostFree(p)
     assert t_pinned < 0.85 * t_pageable, (t_pinned, t_pageable)
+
+
+@pytest.mark.parametrize("shape,b,prec", [((48, 45), 2, "fp64"), ((70, 61), 1, "fp32"),
+                                          ((6, 6, 6), 8, "fp64")])
+def test_moments_in_a_row_keep_no_table(oracle, shape, b, prec):
+    """From the third moments on that nothing followed the ring is used (not with the
+    matrix-core steps): the same bits, and autodiff_matrix and stoch_matrix as before;
+    either of them brings the table back."""
+    from fastkpm_amd import lattice
+    H = lattice.lattice(shape, b=b, seed=5, W=1.0, J=1.0 if b == 2 else 0.0, orbital_blocks=b > 2)
+    eng, orc, bound = _set_up(oracle, H, 5, prec=prec)
+    M = 20
+    tol = FP64_TOL if prec == "fp64" else M * 16 * 2.0 ** -24
+    c = fermi_coeffs(oracle, M, -bound, bound, kT=0.05)
+    D = H.like()
+    mu_o = orc.moments(M)
+    d_o, s_o = orc.autodiff_matrix(c, H), orc.stoch_matrix(c, H)
+    for follow in ("autodiff_matrix", "stoch_matrix"):
+        mu = [eng.moments(M)]
+        for kept in (True, False, False):
+            mu.append(eng.moments(M))
+            assert eng.alpha_table() is (kept or b == 8)
+            assert np.array_equal(mu[-1], mu[0])
+        assert rel_err(mu[0], mu_o) < tol
+        getattr(eng, follow)(c, D)
+        assert rel_err(D.val, d_o if follow == "autodiff_matrix" else s_o) < tol
+        for name, want in (("autodiff_matrix", d_o), ("stoch_matrix", s_o)):
+            assert np.array_equal(eng.moments(M), mu[0]) and eng.alpha_table()
+            getattr(eng, name)(c, D)
+            assert rel_err(D.val, want) < tol
+        assert eng.stoch_method() == "table"
+    eng.set_store_alpha(2)
+    for _ in range(4):
+        eng.moments(M)
+        assert eng.alpha_table()
+    eng.close()
