@@ -1382,10 +1382,14 @@ ResBwd res_bwd(fkpm_handle* h) {
 //   57x57 x 1       12996  506 / 399           834 / 772
 //   64x64 x 1       16384  538 / 379          1722 / 1480 (S = 256)
 //   15^3 x 1        20250  693 / 472 (S = 16) 1074 / 930
+// Below an order the two transposed vectors and the outer products at both ends cost
+// more than the steps gain (moments + autodiff_matrix, whole / step kernels: 57x57 x 1 M = 16
+// 168 / 172, M = 24 212 / 206; 12^3 x 2 M = 64 593 / 597).
 constexpr int kResBwdBlocks = 10240;
 
 template <class S>
-bool res_bwd_wanted(fkpm_handle* h) {
+bool res_bwd_wanted(fkpm_handle* h, int M) {
+  if (M < (h->b == 1 ? 24 : 96)) return true;
   const ResBwd rb = res_bwd<S>(h);
   if (rb.mode != fkd::RES_ST || rb.la || h->b == 4 || h->res.rpt < fkd::res_max_rpt(h->b))
     return true;
@@ -1435,9 +1439,12 @@ bool res_wanted(fkpm_handle* h) {
 //   3000 x 1, 9  6  1127 / 748 (4)      1145 / 857 (32)
 //   1500 x 1, 17 9   881 / 799 (4)       888 / 792 (32)
 //   FP32 x 2 and b = 4 gained at every size: 1900 rows of 9 636 / 968, 8^3 x 4 1004 / 1142
-// The step kernels' time grows with the vector from about 512 KiB a streamed block.
+// The step kernels' time grows with the vector from about 512 KiB a streamed block, and
+// below M = 16 their start costs more than the steps gain (2197 x 1, 7, M = 8 93 / 121,
+// M = 16 139 / 136; 12^3 x 2 171 / 171).
 template <class S>
-bool res_clenshaw_wanted(fkpm_handle* h) {
+bool res_clenshaw_wanted(fkpm_handle* h, int M) {
+  if (M < 16) return true;
   const int d = res_streamed(h->max_deg, h->rset<S>().dreg_xi);
   const int loads = res_loads<S>(h, h->res.rpt, h->rset<S>().dreg_xi);
   const bool waits = h->b == 1 ? loads >= 32 : h->b == 2 && !h->single && loads >= 80;
@@ -1926,7 +1933,7 @@ int stoch_t(fkpm_handle* h, int M, const double* c) {
   const auto& kso = h->ks<S>(K_OUT);
   const bool res_table = h->stoch_method == FKPM_STOCH_AUTO && h->res.K >= (M + 1) / 2;
   if (h->stoch_method != FKPM_STOCH_FORWARD && res_wanted<S>(h) &&
-      (res_table || res_clenshaw_wanted<S>(h))) {
+      (res_table || res_clenshaw_wanted<S>(h, M))) {
     const bool table = res_table;
     h->stoch_used = table ? FKPM_STOCH_TABLE : FKPM_STOCH_CLENSHAW;
     CHK(timing_begin(h));
@@ -2034,7 +2041,7 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
   if (h->res.state) {
     // without room for the backward vectors (taken since moments) too, the ring serves
     const size_t bytes = (size_t)(M / 2) * res_slot(h) * sizeof(S);
-    if (M == 2 || (res_bwd_wanted<S>(h) && h->res.btab.ensure(bytes) == 0)) {
+    if (M == 2 || (res_bwd_wanted<S>(h, M) && h->res.btab.ensure(bytes) == 0)) {
       CHK(res_autodiff<S>(h, M, c, diag));
       return finish_autodiff(h);
     }

@@ -125,13 +125,15 @@ def test_rows_too_long_for_the_whole_recursion(oracle, nb, b, reach, hub, real, 
 
 
 # (lattice, block size, columns, real, M, backward recursion as one launch): either
-# side of the streamed blocks at which autodiff_matrix goes to the step kernels
+# side of the streamed blocks and the order at which autodiff_matrix goes to the step
+# kernels
 @pytest.mark.parametrize("shape,b,S,real,M,whole", [
-    ((50, 50), 1, 3, False, 8, True), ((57, 57), 1, 3, False, 8, False),
-    ((64, 64), 1, 1, False, 4, False), ((64, 64), 1, 33, False, 10, False),
-    ((14, 14, 14), 1, 17, False, 6, False), ((64, 64), 1, 5, True, 8, True),
-    ((40, 40), 2, 3, False, 8, True), ((11, 11, 11), 2, 5, False, 6, True),
-    ((12, 12, 12), 2, 31, False, 6, False), ((12, 12, 12), 2, 2, False, 2, True)])
+    ((50, 50), 1, 3, False, 24, True), ((57, 57), 1, 3, False, 24, False),
+    ((57, 57), 1, 3, False, 22, True), ((64, 64), 1, 1, False, 24, False),
+    ((64, 64), 1, 33, False, 26, False), ((14, 14, 14), 1, 17, False, 30, False),
+    ((64, 64), 1, 5, True, 24, True), ((40, 40), 2, 3, False, 96, True),
+    ((11, 11, 11), 2, 5, False, 96, True), ((12, 12, 12), 2, 31, False, 96, False),
+    ((12, 12, 12), 2, 3, False, 94, True), ((12, 12, 12), 2, 2, False, 2, True)])
 @pytest.mark.parametrize("own_pattern", [True, False])
 def test_backward_recursion_of_streamed_lattices(oracle, shape, b, S, real, M, whole, own_pattern):
     from fastkpm_amd import lattice
@@ -159,7 +161,8 @@ def test_backward_recursion_of_streamed_lattices(oracle, shape, b, S, real, M, w
 
 
 # (lattice, block size, columns, precision, one launch): either side of the streamed
-# blocks and the vector size at which the Clenshaw recurrence goes to the step kernels
+# blocks, the vector size and the order at which the Clenshaw recurrence goes to the
+# step kernels
 @pytest.mark.parametrize("shape,b,S,prec,whole", [
     ((64, 64), 1, 3, "fp64", True), ((13, 13, 13), 1, 3, "fp64", False),
     ((13, 13, 13), 1, 64, "fp64", True), ((45, 42), 2, 5, "fp64", True),
@@ -171,17 +174,17 @@ def test_clenshaw_of_streamed_lattices(oracle, shape, b, S, prec, whole, dense):
     H = lattice.lattice(shape, b=b, seed=9, W=1.0, J=1.0 if b == 2 else 0.0, orbital_blocks=b > 2)
     eng, orc, bound = _set_up(oracle, H, S, prec=prec, dense=dense)
     eng.set_timing(True)
-    M = 11
+    M = 17
     c = fermi_coeffs(oracle, M, -bound, bound, kT=0.05, kind=1)
     D = H.like()
     # FP32: M recursion steps of 16 roundings each
     tol = FP64_TOL if prec == "fp64" else M * 16 * 2.0 ** -24
-    for m in (M, 2):
+    for m in (M, 15, 2):
         s = orc.stoch_matrix(c[:m], H)
         for _ in range(3):
             eng.stoch_matrix(c[:m], D)
             assert eng.stoch_method() == "clenshaw"
-            assert eng.timing()["stoch_launches"] == (1 if whole else m - 1)
+            assert eng.timing()["stoch_launches"] == (1 if whole or m < 16 else m - 1)
             assert rel_err(D.val, s) < tol
     assert eng.state()["r_compact"] is (not dense)
     # a table of the same R and H is used by the whole-recursion kernels on either side
