@@ -115,9 +115,9 @@ __global__ __launch_bounds__(WG) void k_batch_fwd(const SlotDev* __restrict__ sd
     mfma_step_dev<S>(wid, d.rp, d.ci, (const S*)d.hv, x, z, y, d.nb, d.qp, d.chunk, cx, cz, part,
                      0, nors);
   else
-    step_moments_dev<S, true, B, L, KQ>(wid, (d.nt & NT_ORDER) ? d.rord : d.rp, d.ci,
-                                        (const S*)d.hv, x, z, y, d.nb, d.qp, d.chunk, cx, cz, part,
-                                        d.nt, nors);
+    step_moments_dev<S, true, B, L, KQ, early_own<B, L, KQ>()>(
+        wid, (d.nt & NT_ORDER) ? d.rord : d.rp, d.ci, (const S*)d.hv, x, z, y, d.nb, d.qp, d.chunk,
+        cx, cz, part, d.nt, nors);
 }
 
 // Backward (autodiff) step of every slot of the class in its backward phase;

@@ -633,7 +633,8 @@ template <class S>
 auto mom_fn(const fkpm_handle* h, const fkd::KSet<S>& ks, const KCfg& c) {
   if (c.mfma == 2 && ks.mfma_mom_rr2 != nullptr && h->qp % 16 == 0)
     return c.dm == 7 ? ks.mfma_mom_rr2_7 : ks.mfma_mom_rr2;
-  return c.mfma == 2 ? (c.dm == 7 ? ks.mfma_mom_rr7 : ks.mfma_mom_rr) : c.mfma ? ks.mfma_mom : ks.mom;
+  if (c.mfma == 2) return c.dm == 7 ? ks.mfma_mom_rr7 : ks.mfma_mom_rr;
+  return c.mfma ? ks.mfma_mom : fkd::step_fn(ks, h->nb);
 }
 // The row-resident autodiff step in FP32 takes column tiles in pairs when the
 // padded width allows (16 packets, two 16-column tiles, divide it): C4 FP32
@@ -2306,8 +2307,8 @@ int moments2_t(fkpm_handle* h, int M, int col_chunk, size_t budget, double* mu) 
     // the row order and the row length belong to H's pattern
     KCfg rows = c;
     rows.nt &= ~fkd::NT_ORDER;
-    return launch(ks.mom, grid, block, h->stream, rp_, ci_, hv_, x, z, y, h->nb, qpc, c.chunk,
-                  cx, cz, (double*)nullptr, rp_ == rp ? nt_for(h, rows) : rows.nt,
+    return launch(fkd::step_fn(ks, h->nb), grid, block, h->stream, rp_, ci_, hv_, x, z, y,
+                  h->nb, qpc, c.chunk, cx, cz, (double*)nullptr, rp_ == rp ? nt_for(h, rows) : rows.nt,
                   no_rsource<S>());
   };
   const int* j1rp = h->j_rp[0].as<const int>();

@@ -16,6 +16,9 @@ template <class S>
 struct KSet {
   void (*mom)(const int*, const int*, const S*, const S*, const S*, S*, int, int, int, double,
               double, double*, int, RSource<S>) = nullptr;
+  // mom without the early load of the own rows (step_fn; 8-row blocks on a wave)
+  void (*mom_late)(const int*, const int*, const S*, const S*, const S*, S*, int, int, int,
+                   double, double, double*, int, RSource<S>) = nullptr;
   void (*xi)(const int*, const int*, const S*, const S*, const S*, S*, double*, int, int, int,
              double, double, double, double, int, int) = nullptr;
   void (*ad_fused)(const int*, const int*, const S*, const S*, const S*, const S*, const S*, S*,
@@ -84,6 +87,17 @@ struct KSet {
                      double) = nullptr;
   int B = 0, L = 0, KQ = 0;
 };
+
+// The forward step of a geometry on nb block rows.  With 8-row blocks on a wave a row,
+// the early load of the own rows costs one of four waves a SIMD: it pays while every
+// row's wave is resident either way, two on each of 1024 SIMDs.  Moments of M = 64 with
+// and without, real FP64 x 8 x 128 (us): 32x32 369 / 431, 10^3 584 / 629, 45x45 627 / 627;
+// 46x46 717 / 698, 16^3 1419 / 1099, 20^3 2303 / 2057.
+constexpr int kEarlyRows = 2048;
+template <class S>
+auto step_fn(const KSet<S>& ks, int nb) {
+  return nb > kEarlyRows && ks.mom_late != nullptr ? ks.mom_late : ks.mom;
+}
 
 // Entries of mfma_ads.
 enum MfmaAds { ADS_FUSED = 0, ADS_PLAIN = 1, ADS_RR = 2, ADS_RR7 = 3, ADS_RR2 = 4, ADS_RR2_7 = 5 };

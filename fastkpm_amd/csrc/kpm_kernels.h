@@ -596,6 +596,16 @@ __device__ __forceinline__ void add_rsource_rows(const RSource<S>& rs_, int i, s
   }
 }
 
+// The forward step's form EARLY: the own rows of z are loaded with the gather's first
+// loads, ahead of its adds, which holds KQ*B packets of registers through the gather.
+// More than two packets a lane go without, and so do 8-row blocks on less than a wave
+// (allocation-free moments of 10^3 x 8 x 32, M = 128: 1455 us with, 1392 without); 8-row
+// blocks on a wave have a kernel of each form (step_fn).
+template <int B, int L, int KQ>
+constexpr bool early_own() {
+  return KQ <= 2 && (B < 8 || L == WAVE);
+}
+
 // ---------------------------------------------------------------------------
 // Moments step: y = cx * (Hs x) + cz * z  (z may be null) [+ cr * R], and the
 // two moment dots sum |x_i|^2 and Re<y_i, x_i> over this workgroup's rows
@@ -604,7 +614,7 @@ __device__ __forceinline__ void add_rsource_rows(const RSource<S>& rs_, int i, s
 // (engine_cpu.cpp:63-84) fused with both cdot's; with the R term it is one
 // step b_k = c_k R + 2 Hs b_{k+1} - b_{k+2} of the Clenshaw recurrence.
 // ---------------------------------------------------------------------------
-template <typename S, bool CX, int B, int L, int KQ>
+template <typename S, bool CX, int B, int L, int KQ, bool EARLY>
 __device__ __forceinline__ void step_moments_dev(
     WgId wid,
     const int* __restrict__ rp, const int* __restrict__ ci, const S* __restrict__ hv,
@@ -636,8 +646,6 @@ __device__ __forceinline__ void step_moments_dev(
     const int p0 = cur.p0, p1 = cur.p1;
     for (int q0 = qs; q0 < qs + qw; q0 += L * KQ) {
       const size_t qo = (size_t)(q0 + l) * NS;
-      // own rows of z with the gather's first loads, where they take few registers
-      constexpr bool EARLY = KQ <= 2;
       A out[KQ][B][NS];
       if constexpr (EARLY)
         if (z != nullptr) load_rows_nt<S, A, B, L, KQ>(z, i, rs, qo, out, nt & NT_LOAD);
@@ -703,12 +711,13 @@ __device__ __forceinline__ void step_moments_dev(
   if (partial != nullptr) wg_sum2(dmm, dm1, partial + 2 * (size_t)wid.k);
 }
 
-template <typename S, bool CX, int B, int L, int KQ>
+template <typename S, bool CX, int B, int L, int KQ, bool EARLY>
 __global__ __launch_bounds__(WG) void k_step_moments(
     const int* __restrict__ rp, const int* __restrict__ ci, const S* __restrict__ hv,
     const S* __restrict__ x, const S* __restrict__ z, S* __restrict__ y, int nb, int qp,
     int chunk, double cx, double cz, double* __restrict__ partial, int nt, RSource<S> rsrc) {
-  step_moments_dev<S, CX, B, L, KQ>(wg_self(), rp, ci, hv, x, z, y, nb, qp, chunk, cx, cz, partial, nt, rsrc);
+  step_moments_dev<S, CX, B, L, KQ, EARLY>(wg_self(), rp, ci, hv, x, z, y, nb, qp, chunk, cx, cz,
+                                           partial, nt, rsrc);
 }
 
 // ---------------------------------------------------------------------------

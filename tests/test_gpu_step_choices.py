@@ -108,3 +108,18 @@ def test_cut_table_at_high_order_fp32(oracle, monkeypatch, b, S, M):
     assert eng.stoch_method() == "clenshaw"
     assert err < 4 * rel_err(D.val, want) + 2.0 ** -22
     eng.close()
+
+
+@pytest.mark.parametrize("prec,S", [("fp64", 127), ("fp32", 253)])
+@pytest.mark.parametrize("shape", [(64, 32), (33, 63)])
+def test_eight_row_blocks_on_a_wave(oracle, shape, prec, S):
+    """The forward step's two forms: 2048 block rows and 2079, a ragged column tile."""
+    from fastkpm_amd import lattice
+    H = lattice.lattice(shape, b=8, seed=5, orbital_blocks=True)
+    H.val = np.ascontiguousarray(H.val.real)
+    eng, orc, bound = _set_up(oracle, H, S, real=True, prec=prec, dense=False)
+    M = 8
+    _check_all(oracle, eng, orc, H, M, bound, _tol(prec, M))
+    c = eng.kernel_config(0)
+    assert (c["lanes"], c["kq"]) == (64, 1), c
+    eng.close()
