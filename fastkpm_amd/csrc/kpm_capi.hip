@@ -2023,6 +2023,21 @@ int finish_autodiff(fkpm_handle* h) {
   return 0;
 }
 
+// Whether the fused backward steps compute alpha_{m-1} anew although the table holds
+// it.  Real 8-row blocks on a wave a row: of the step that recomputes one wave fits a
+// SIMD, of the one that reads two, and while the rows are one wave for each of 1024
+// SIMDs the first is the shorter chain.  autodiff_matrix of M = 64, recomputed / read
+// (us): FP64 x 128 6^3 1852 / 2170, 10^3 2177 / 2484, 32x32 1640 / 1870, 11^3 (1331 rows)
+// 3925 / 3052; FP32 x 256 32x32 1542 / 1739, 36x36 2751 / 2142.  On D's own pattern
+// reading is the faster everywhere (10^3 FP64 1091 / 1013).
+constexpr int kOneWaveRows = 1024;
+
+bool ad_recomputes(const fkpm_handle* h) {
+  const KCfg& a = h->kc[K_AD];
+  return h->store_alpha == 1 && h->b == 8 && !h->cx && a.L == fkd::WAVE && h->d_fused &&
+         h->nb <= kOneWaveRows;
+}
+
 template <class S>
 int autodiff_t(fkpm_handle* h, int M, const double* c) {
   const dim3 block(fkd::WG);
@@ -2057,10 +2072,11 @@ int autodiff_t(fkpm_handle* h, int M, const double* c) {
   CHK(timing_begin(h));
   LoopRecorder rec(h);
   if (M > 2) {
+    const bool again = ad_recomputes(h);
     const double sb = 2 * c[M - 1];  // beta_{M/2} = 2 c_{M-1} alpha_{M/2-1}
     for (int m = M / 2 - 1; m >= 1; m--) {
       // alpha_{m-1}: from the table, or recomputed into the ring by the step
-      const bool stored = h->a_slots > 0 && m - 1 <= h->a_slots;
+      const bool stored = h->a_slots > 0 && m - 1 <= h->a_slots && !again;
       const S* am = (const S*)h->vec_a(m);
       const S* am1 = (const S*)h->vec_a(m + 1);
       S* aout = stored ? (S*)h->vec_a(m - 1) : (S*)h->A[(m - 1) % 3].p;

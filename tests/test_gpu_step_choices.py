@@ -123,3 +123,31 @@ def test_eight_row_blocks_on_a_wave(oracle, shape, prec, S):
     c = eng.kernel_config(0)
     assert (c["lanes"], c["kq"]) == (64, 1), c
     eng.close()
+
+
+@pytest.mark.parametrize("own_pattern", [True, False])
+@pytest.mark.parametrize("prec,S", [("fp64", 127), ("fp32", 253)])
+@pytest.mark.parametrize("shape", [(4, 4), (32, 32), (25, 41)])
+def test_backward_of_eight_row_blocks_on_a_wave(oracle, shape, prec, S, own_pattern):
+    """Vectors computed anew beside a kept table up to 1024 block rows, read from 1025
+    on; the table still serves a stoch_matrix that follows."""
+    from fastkpm_amd import lattice
+    H = lattice.lattice(shape, b=8, seed=5, orbital_blocks=True)
+    H.val = np.ascontiguousarray(H.val.real)
+    eng, orc, bound = _set_up(oracle, H, S, real=True, prec=prec, dense=False)
+    nb, M = H.n_rows, 10
+    Dp = H if own_pattern else lattice.coo_to_bsr(nb, 8, range(nb), range(nb),
+                                                  np.zeros((nb, 8, 8)))
+    c = fermi_coeffs(oracle, M, -bound, bound, kT=0.05)
+    mu = orc.moments(M)
+    want, xi = orc.autodiff_matrix(c, Dp), orc.stoch_matrix(c, Dp)
+    for store in (1, 2, 0):  # read at once where it is forced, no table at all
+        eng.set_store_alpha(store)
+        assert rel_err(eng.moments(M), mu) < _tol(prec, M)
+        D = Dp.like(eng.np_dtype)
+        eng.autodiff_matrix(c, D)
+        assert rel_err(D.val, want) < _tol(prec, M), store
+        assert eng.kernel_config(2)["lanes"] == 64
+        eng.stoch_matrix(c, D)
+        assert rel_err(D.val, xi) < _tol(prec, M), store
+    eng.close()
