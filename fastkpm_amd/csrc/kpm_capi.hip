@@ -628,6 +628,21 @@ int nt_for(const fkpm_handle* h, const KCfg& c) {
   return same ? c.nt | h->max_deg << fkd::NT_DEG : c.nt;
 }
 
+// Grid of the forward method's step.  Rows of complex 8x8 blocks are padded to tiles of
+// the matrix cores, which leaves this vector-unit step passes as narrow as one tile
+// (144 columns FP64: nine); one after another in the workgroup of the row they are one
+// long chain, and few rows leave the chip idle meanwhile.  So with blocks of 4 and 8 the
+// passes of a sweep of up to 128 workgroups run side by side.  stoch_matrix of M = 32
+// (us), in turn / side by side: 12x12 x 8 FP64, S = 129 3674 / 911, 10^3 5679 / 3052, 45x45
+// (127 workgroups) 4824 / 3875; 15^3 (211) S = 65 4594 / 4989, FP32 S = 129 4201 / 4484.
+// Smaller blocks have few passes of many rows (60x60 x 1 FP32, S = 150 256 / 271).
+constexpr int kXiPassWgs = 128;
+
+dim3 xi_grid(const fkpm_handle* h, const KCfg& c) {
+  const bool apart = h->b >= 4 && c.nwg <= kXiPassWgs;
+  return dim3(c.nwg, apart ? h->qp / (c.L * c.KQ) : 1);
+}
+
 // Kernel entry of a kind under its configuration.
 template <class S>
 auto mom_fn(const fkpm_handle* h, const fkd::KSet<S>& ks, const KCfg& c) {
@@ -1126,7 +1141,7 @@ int tune_t(fkpm_handle* h) {
                             cl ? rsource<S>(h, 0.25) : no_rsource<S>());
             }
             if (kind == K_XI)
-              return launch(ks.xi, dim3(k.nwg), dim3(fkd::WG), h->stream, rp_for(h, k), ci, hv, (const S*)x,
+              return launch(ks.xi, xi_grid(h, k), dim3(fkd::WG), h->stream, rp_for(h, k), ci, hv, (const S*)x,
                             (const S*)z, y, h->xi.as<double>(), h->nb, h->qp, k.chunk, 2.0, -1.0,
                             0.0, 0.5, t == 0 ? 1 : 0, nt_for(h, k));
             // backward step: reads alpha_m, alpha_{m+1}, beta_{m+1}, beta_{m+2};
@@ -1972,7 +1987,7 @@ int stoch_t(fkpm_handle* h, int M, const double* c) {
     CHK(h->xi.ensure(h->accbytes()));
     const KCfg& kx = h->kc[K_XI];
     const auto& ksx = h->ks<S>(K_XI);
-    const dim3 grid(kx.nwg);
+    const dim3 grid = xi_grid(h, kx);
     {
       LoopRecorder rec(h);
       // alpha_1 = Hs R, xi = c0 R + c1 alpha_1

@@ -742,8 +742,9 @@ __global__ __launch_bounds__(WG) void k_step_xi(
   const A acx = (A)cx, acz = (A)cz;
   const S* const X[1] = {x};
 
-  const int qw = (nt & NT_SLICE) ? L * KQ : qp;  // columns per sweep over the rows
-  for (int qs = 0; qs < qp; qs += qw) {
+  // columns per sweep over the rows; a second grid dimension takes the passes apart
+  const int qw = (nt & NT_SLICE) || gridDim.y > 1 ? L * KQ : qp;
+  for (int qs = blockIdx.y * qw; qs < qp; qs += gridDim.y * qw) {
   RowPtr nxt = row_ptr(rp, first_row<L>(rr.r0 + g), rr.r1, nt);
   for (int base = rr.r0; base < rr.r1; base += rr.stride) {
     int i = base + g;

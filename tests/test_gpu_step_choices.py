@@ -151,3 +151,29 @@ def test_backward_of_eight_row_blocks_on_a_wave(oracle, shape, prec, S, own_patt
         eng.stoch_matrix(c, D)
         assert rel_err(D.val, xi) < _tol(prec, M), store
     eng.close()
+
+
+# columns and passes of the forward method's step: the passes of a row side by side up to
+# 128 workgroups a sweep, one after another from there on
+@pytest.mark.parametrize("prec,S,passes", [("fp64", 33, 3), ("fp64", 129, 9), ("fp32", 129, 5)])
+@pytest.mark.parametrize("shape,apart", [((3, 3), True), ((45, 45), True), ((46, 45), False)])
+@pytest.mark.parametrize("sliced", [False, True])
+def test_forward_method_column_passes(oracle, shape, apart, prec, S, passes, sliced):
+    from fastkpm_amd import lattice
+    H = lattice.lattice(shape, b=8, seed=5, orbital_blocks=True)
+    eng, orc, bound = _set_up(oracle, H, S, prec=prec, dense=False)
+    eng.set_stoch_method("forward")
+    if sliced:
+        eng.set_slice(1)
+    M = 8
+    c = fermi_coeffs(oracle, M, -bound, bound, kT=0.05, kind=1)
+    D = H.like(eng.np_dtype)
+    want = orc.stoch_matrix(c, H)
+    for _ in range(3):  # the step loop is captured, then replayed
+        eng.stoch_matrix(c, D)
+        assert rel_err(D.val, want) < _tol(prec, M)
+    k = eng.kernel_config(1)
+    ne = 1 if prec == "fp64" else 2
+    assert eng.config()["s_padded"] == passes * k["lanes"] * k["kq"] * ne
+    assert (k["n_wg"] <= 128) is apart
+    eng.close()
