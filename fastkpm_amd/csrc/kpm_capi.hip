@@ -681,6 +681,19 @@ auto adsp_fn(const fkd::KSet<S>& ks, const KCfg& c) {
 // Last-level cache of the device (MI355X: 256 MB).
 constexpr size_t kLlcBytes = (size_t)256 << 20;
 
+// Whether a row much longer than the others sets the time of a step: its blocks are one
+// chain of gathers in a lane group, longer by a third with two packets a lane than with
+// one, while the other rows stream past.  moments of M = 40 (us), two packets a lane /
+// one, rows of 5 blocks and one of 65: 30000 x 2 FP64 (15 MB a vector) 554 / 462, x 4 FP32
+// (31 MB) 1462 / 1118; one of 25: 9000 x 2 FP32 (5 MB) 273 / 218, 30000 x 4 FP32 (31 MB) 686 / 568,
+// but 30000 x 2 FP64 (15 MB) 308 / 352, x 4 (61 MB) 960 / 1265.
+bool long_rows(int nb, int nnzb, int max_deg) { return (long long)max_deg * nb > 2ll * nnzb; }
+
+bool chain_bound(const fkpm_handle* h) {
+  return long_rows(h->nb, h->nnzb, h->max_deg) &&
+         h->vbytes() < (size_t)h->max_deg * h->b * ((h->single ? 320 : 192) << 10);
+}
+
 // Default geometry of a kernel kind when nothing is tuned: one pass of width
 // wmax.  From 64 packets on, whole waves per row (wave-uniform rows, scalar
 // offsets and H); below, two packets per lane, which keeps more loads in
@@ -702,7 +715,7 @@ KCfg default_cfg(fkpm_handle* h, int kind) {
   KCfg c;
   auto packets = [&](int kq) {
     const int L = h->wmax / kq;
-    if (c.L > 0 || h->wmax % kq != 0 || !compiled(h->b, L, kq) ||
+    if (c.L > 0 || h->wmax % kq != 0 || !compiled(h->b, L, kq) || chain_bound(h) ||
         h->nb < 256 * (fkd::WG / fkd::WAVE) * (fkd::WAVE / L))
       return;
     c.L = L;
@@ -2782,13 +2795,16 @@ int fkpm_set_H(fkpm_handle* h, int nb, int b, int nnzb, const int* row_ptr, cons
   // The kernel choice depends on the block size, the block-row and block
   // counts (grids, tuned-shape key) and on whether every row has at most
   // kRowResidentMax blocks (row-resident matrix-core kernels read only that many),
-  // or at most 7 (their instantiation without a padding slot): a change of any
-  // of them picks the kernels again at the next use.
+  // or at most 7 (their instantiation without a padding slot), and on a row much
+  // longer than the others: a change of any of them picks the kernels again at the
+  // next use.
   const int old_b = h->b, old_nb = h->nb, old_nnzb = h->nnzb, old_deg = h->max_deg;
   if (!same) CHK(upload_pattern(h, nb, b, nnzb, row_ptr, col_idx));
   const bool geo_change = b != old_b || nb != old_nb || nnzb != old_nnzb ||
                           (old_deg <= kRowResidentMax) != (h->max_deg <= kRowResidentMax) ||
-                          (old_deg <= 7) != (h->max_deg <= 7);
+                          (old_deg <= 7) != (h->max_deg <= 7) ||
+                          (old_deg != h->max_deg && (long_rows(nb, nnzb, old_deg) ||
+                                                     long_rows(nb, nnzb, h->max_deg)));
   h->avg = avg;
   h->mag = mag;
   const size_t eb = h->single ? 4 : 8;

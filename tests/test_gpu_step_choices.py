@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from helpers import fermi_coeffs, rel_err
-from test_gpu_dispatch import FP64_TOL, _check_all, _engine, _set_up
+from test_gpu_dispatch import FP64_TOL, _check_all, _engine, _pattern, _set_up
 
 pytestmark = pytest.mark.gpu
 
@@ -176,4 +176,41 @@ def test_forward_method_column_passes(oracle, shape, apart, prec, S, passes, sli
     ne = 1 if prec == "fp64" else 2
     assert eng.config()["s_padded"] == passes * k["lanes"] * k["kq"] * ne
     assert (k["n_wg"] <= 128) is apart
+    eng.close()
+
+
+def _bonds(nb, b, pairs, real=False):
+    """A chain of rows of five blocks and the bonds `pairs` besides."""
+    from fastkpm_amd import lattice
+    H = _pattern(nb, b, 2, 0, real)
+    r, c = np.array(pairs, dtype=int).reshape(-1, 2).T
+    T = np.random.default_rng(3).standard_normal((len(r), b, b))
+    blocks = np.concatenate([H.val.reshape(-1, b, b).transpose(0, 2, 1), T, T.transpose(0, 2, 1)])
+    return lattice.coo_to_bsr(nb, b, np.concatenate([H.row_idx, r, c]),
+                              np.concatenate([H.col_idx, c, r]), blocks, H.val.dtype)
+
+
+# (rows, block size, columns, precision, real, blocks more in one row, lanes x packets of
+# the forward step): one packet a lane where the long row's chain outlasts the others
+@pytest.mark.parametrize("nb,b,S,prec,real,hub,want", [
+    (9000, 2, 11, "fp64", False, 20, (16, 1)), (9000, 2, 11, "fp64", False, 0, (8, 2)),
+    (9000, 2, 11, "fp64", False, 5, (8, 2)), (25000, 2, 11, "fp64", False, 20, (8, 2)),
+    (9000, 1, 11, "fp64", False, 9, (16, 1)), (9000, 2, 24, "fp32", False, 8, (16, 1)),
+    (9000, 4, 24, "fp64", True, 20, (16, 1)), (9000, 4, 24, "fp32", False, 20, (16, 1))])
+def test_one_long_row(oracle, nb, b, S, prec, real, hub, want):
+    """... and the choice follows a pattern of as many rows and blocks."""
+    from fastkpm_amd import EnergyScale
+    long = [(0, 1000 + 7 * k) for k in range(hub)]
+    even = [(20 * k, 3000 + 20 * k) for k in range(hub)]
+    M = 8
+    H = _bonds(nb, b, long, real)
+    eng, orc, bound = _set_up(oracle, H, S, real=real, prec=prec, dense=False)
+    for pairs, geo in ((long, want), (even, (8, 2)), (long, want)):
+        H = _bonds(nb, b, pairs, real)
+        eng.set_H(H, EnergyScale(-bound, bound))
+        orc.set_H(H, -bound, bound)
+        _check_all(oracle, eng, orc, H, M, bound, _tol(prec, M))
+        for kind in (0, 4):
+            c = eng.kernel_config(kind)
+            assert (c["lanes"], c["kq"]) == geo, (pairs[:1], kind, c)
     eng.close()
