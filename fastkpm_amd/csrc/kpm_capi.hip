@@ -628,6 +628,19 @@ int nt_for(const fkpm_handle* h, const KCfg& c) {
   return same ? c.nt | h->max_deg << fkd::NT_DEG : c.nt;
 }
 
+// Whether a row much longer than the others sets the time of a step: its blocks are one
+// chain of gathers in a lane group, longer by a third with two packets a lane than with
+// one, while the other rows stream past.  moments of M = 40 (us), two packets a lane /
+// one, rows of 5 blocks and one of 65: 30000 x 2 FP64 (15 MB a vector) 554 / 462, x 4 FP32
+// (31 MB) 1462 / 1118; one of 25: 9000 x 2 FP32 (5 MB) 273 / 218, 30000 x 4 FP32 (31 MB) 686 / 568,
+// but 30000 x 2 FP64 (15 MB) 308 / 352, x 4 (61 MB) 960 / 1265.
+bool long_rows(int nb, int nnzb, int max_deg) { return (long long)max_deg * nb > 2ll * nnzb; }
+
+bool chain_bound(const fkpm_handle* h) {
+  return long_rows(h->nb, h->nnzb, h->max_deg) &&
+         h->vbytes() < (size_t)h->max_deg * h->b * ((h->single ? 320 : 192) << 10);
+}
+
 // Grid of the forward method's step.  Rows of complex 8x8 blocks are padded to tiles of
 // the matrix cores, which leaves this vector-unit step passes as narrow as one tile
 // (144 columns FP64: nine); one after another in the workgroup of the row they are one
@@ -649,7 +662,7 @@ auto mom_fn(const fkpm_handle* h, const fkd::KSet<S>& ks, const KCfg& c) {
   if (c.mfma == 2 && ks.mfma_mom_rr2 != nullptr && h->qp % 16 == 0)
     return c.dm == 7 ? ks.mfma_mom_rr2_7 : ks.mfma_mom_rr2;
   if (c.mfma == 2) return c.dm == 7 ? ks.mfma_mom_rr7 : ks.mfma_mom_rr;
-  return c.mfma ? ks.mfma_mom : fkd::step_fn(ks, h->nb);
+  return c.mfma ? ks.mfma_mom : fkd::step_fn(ks, h->nb, chain_bound(h));
 }
 // The row-resident autodiff step in FP32 takes column tiles in pairs when the
 // padded width allows (16 packets, two 16-column tiles, divide it): C4 FP32
@@ -680,19 +693,6 @@ auto adsp_fn(const fkd::KSet<S>& ks, const KCfg& c) {
 
 // Last-level cache of the device (MI355X: 256 MB).
 constexpr size_t kLlcBytes = (size_t)256 << 20;
-
-// Whether a row much longer than the others sets the time of a step: its blocks are one
-// chain of gathers in a lane group, longer by a third with two packets a lane than with
-// one, while the other rows stream past.  moments of M = 40 (us), two packets a lane /
-// one, rows of 5 blocks and one of 65: 30000 x 2 FP64 (15 MB a vector) 554 / 462, x 4 FP32
-// (31 MB) 1462 / 1118; one of 25: 9000 x 2 FP32 (5 MB) 273 / 218, 30000 x 4 FP32 (31 MB) 686 / 568,
-// but 30000 x 2 FP64 (15 MB) 308 / 352, x 4 (61 MB) 960 / 1265.
-bool long_rows(int nb, int nnzb, int max_deg) { return (long long)max_deg * nb > 2ll * nnzb; }
-
-bool chain_bound(const fkpm_handle* h) {
-  return long_rows(h->nb, h->nnzb, h->max_deg) &&
-         h->vbytes() < (size_t)h->max_deg * h->b * ((h->single ? 320 : 192) << 10);
-}
 
 // Default geometry of a kernel kind when nothing is tuned: one pass of width
 // wmax.  From 64 packets on, whole waves per row (wave-uniform rows, scalar
@@ -2351,7 +2351,7 @@ int moments2_t(fkpm_handle* h, int M, int col_chunk, size_t budget, double* mu) 
     // the row order and the row length belong to H's pattern
     KCfg rows = c;
     rows.nt &= ~fkd::NT_ORDER;
-    return launch(fkd::step_fn(ks, h->nb), grid, block, h->stream, rp_, ci_, hv_, x, z, y,
+    return launch(fkd::step_fn(ks, h->nb, chain_bound(h)), grid, block, h->stream, rp_, ci_, hv_, x, z, y,
                   h->nb, qpc, c.chunk, cx, cz, (double*)nullptr, rp_ == rp ? nt_for(h, rows) : rows.nt,
                   no_rsource<S>());
   };

@@ -19,6 +19,9 @@ struct KSet {
   // mom without the early load of the own rows (step_fn; 8-row blocks on a wave)
   void (*mom_late)(const int*, const int*, const S*, const S*, const S*, S*, int, int, int,
                    double, double, double*, int, RSource<S>) = nullptr;
+  // mom for patterns bound by one long row (step_fn; real FP64 4-row blocks)
+  void (*mom_long)(const int*, const int*, const S*, const S*, const S*, S*, int, int, int,
+                   double, double, double*, int, RSource<S>) = nullptr;
   void (*xi)(const int*, const int*, const S*, const S*, const S*, S*, double*, int, int, int,
              double, double, double, double, int, int) = nullptr;
   void (*ad_fused)(const int*, const int*, const S*, const S*, const S*, const S*, const S*, S*,
@@ -88,14 +91,19 @@ struct KSet {
   int B = 0, L = 0, KQ = 0;
 };
 
-// The forward step of a geometry on nb block rows.  With 8-row blocks on a wave a row,
-// the early load of the own rows costs one of four waves a SIMD: it pays while every
-// row's wave is resident either way, two on each of 1024 SIMDs.  Moments of M = 64 with
+// The forward step of a geometry on nb block rows; long_row: one long row sets its time.
+// Such a row takes two real 4x4 FP64 blocks a batch instead of one (moments of M = 40, us,
+// one / two, rows of 5 blocks and one of 65, S = 24: 2000 rows 630 / 534, 9000 716 / 592, 30000 889 /
+// 656; one of 25 287 / 265, 350 / 310; complex and smaller blocks lost up to 17 % by it at
+// 25).  With 8-row blocks on a wave a row, the early load
+// of the own rows costs one of four waves a SIMD: it pays while every row's wave is
+// resident either way, two on each of 1024 SIMDs.  Moments of M = 64 with
 // and without, real FP64 x 8 x 128 (us): 32x32 369 / 431, 10^3 584 / 629, 45x45 627 / 627;
 // 46x46 717 / 698, 16^3 1419 / 1099, 20^3 2303 / 2057.
 constexpr int kEarlyRows = 2048;
 template <class S>
-auto step_fn(const KSet<S>& ks, int nb) {
+auto step_fn(const KSet<S>& ks, int nb, bool long_row) {
+  if (long_row && ks.mom_long != nullptr) return ks.mom_long;
   return nb > kEarlyRows && ks.mom_late != nullptr ? ks.mom_late : ks.mom;
 }
 

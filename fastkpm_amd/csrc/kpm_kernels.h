@@ -326,6 +326,14 @@ struct Geo {
   }
 };
 
+// The forward steps' budget, and that of real 4x4 blocks where one long row's chain of
+// batches sets the time (step_fn).
+constexpr int LONG_ROW_BUDGET = 64;
+template <typename S, int L>
+constexpr int gather_budget() {
+  return sizeof(S) == 8 && L < WAVE ? 40 : 64;
+}
+
 // Rows of one workgroup.  Workgroups reach the 8 XCDs round-robin
 // (blockIdx % 8); XCD x owns one contiguous region of block rows, the union
 // of the chunks of its workgroups, and its workgroups sweep that region
@@ -500,14 +508,14 @@ __device__ __forceinline__ void gather_row_pre(const int* __restrict__ ci,
 }
 
 // The forward steps' gather (no prefetched values, the larger batch budget).
-template <typename S, typename A, bool CX, int B, int L, int KQ, int NX, class F>
+template <typename S, typename A, bool CX, int B, int L, int KQ, int NX, int BUD = gather_budget<S, L>(),
+          class F>
 __device__ __forceinline__ void gather_row(const int* __restrict__ ci, const S* __restrict__ hv,
                                            const S* const (&X)[NX], size_t rs, size_t qo, int p0,
                                            int p1, A (&acc)[NX][KQ][B][Vec16<S>::N], F&& blk) {
   const A none[KQ][B][Vec16<S>::N] = {};
   auto nopre = [](int) { return NoPre{}; };
   auto blk4 = [&](int p, int jb, auto& xv, NoPre) { blk(p, jb, xv); };
-  constexpr int BUD = sizeof(S) == 8 && L < WAVE ? 40 : 64;
   gather_row_pre<S, A, CX, B, L, KQ, NX, false, decltype(blk4)&, decltype(nopre)&, BUD>(
       ci, hv, X, rs, qo, p0, p1, acc, blk4, nopre, -1, none);
 }
@@ -614,7 +622,7 @@ constexpr bool early_own() {
 // (engine_cpu.cpp:63-84) fused with both cdot's; with the R term it is one
 // step b_k = c_k R + 2 Hs b_{k+1} - b_{k+2} of the Clenshaw recurrence.
 // ---------------------------------------------------------------------------
-template <typename S, bool CX, int B, int L, int KQ, bool EARLY>
+template <typename S, bool CX, int B, int L, int KQ, bool EARLY, int BUD = gather_budget<S, L>()>
 __device__ __forceinline__ void step_moments_dev(
     WgId wid,
     const int* __restrict__ rp, const int* __restrict__ ci, const S* __restrict__ hv,
@@ -662,7 +670,7 @@ __device__ __forceinline__ void step_moments_dev(
             acc[0][k][bi][e] = A(0);
             xd[k][bi][e] = A(0);
           }
-      gather_row<S, A, CX, B, L, KQ, 1>(ci, hv, X, rs, qo, p0, p1, acc,
+      gather_row<S, A, CX, B, L, KQ, 1, BUD>(ci, hv, X, rs, qo, p0, p1, acc,
                                          [&](int, int jb, auto& xv) {
                                            if (jb != i) return;
 #pragma unroll
@@ -711,13 +719,13 @@ __device__ __forceinline__ void step_moments_dev(
   if (partial != nullptr) wg_sum2(dmm, dm1, partial + 2 * (size_t)wid.k);
 }
 
-template <typename S, bool CX, int B, int L, int KQ, bool EARLY>
+template <typename S, bool CX, int B, int L, int KQ, bool EARLY, int BUD = gather_budget<S, L>()>
 __global__ __launch_bounds__(WG) void k_step_moments(
     const int* __restrict__ rp, const int* __restrict__ ci, const S* __restrict__ hv,
     const S* __restrict__ x, const S* __restrict__ z, S* __restrict__ y, int nb, int qp,
     int chunk, double cx, double cz, double* __restrict__ partial, int nt, RSource<S> rsrc) {
-  step_moments_dev<S, CX, B, L, KQ, EARLY>(wg_self(), rp, ci, hv, x, z, y, nb, qp, chunk, cx, cz,
-                                           partial, nt, rsrc);
+  step_moments_dev<S, CX, B, L, KQ, EARLY, BUD>(wg_self(), rp, ci, hv, x, z, y, nb, qp, chunk, cx,
+                                                cz, partial, nt, rsrc);
 }
 
 // ---------------------------------------------------------------------------

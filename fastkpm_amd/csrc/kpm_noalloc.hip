@@ -210,7 +210,7 @@ int run(int device, unsigned char* base, int nb, int b, int nnzb, const int* rp,
     const S* x = alpha(m);
     const S* z = m == 0 ? nullptr : alpha(m - 1);
     S* y = alpha(m + 1);
-    if (launch(fkd::step_fn(ks, nb), dim3(nwg), blk, st, (const int*)rp, (const int*)ci,
+    if (launch(fkd::step_fn(ks, nb, false), dim3(nwg), blk, st, (const int*)rp, (const int*)ci,
                (const S*)hv, x, z, y, nb, qp, chunk, m == 0 ? 1.0 : 2.0, m == 0 ? 0.0 : -1.0,
                part + (size_t)m * nwg * 2, 0, nors))
       return FKPM_E_HIP;
