@@ -641,7 +641,7 @@ bool chain_bound(const fkpm_handle* h) {
          h->vbytes() < (size_t)h->max_deg * h->b * ((h->single ? 320 : 192) << 10);
 }
 
-// Grid of the forward method's step.  Rows of complex 8x8 blocks are padded to tiles of
+// Column passes side by side in the forward method's step.  Rows of complex 8x8 blocks are padded to tiles of
 // the matrix cores, which leaves this vector-unit step passes as narrow as one tile
 // (144 columns FP64: nine); one after another in the workgroup of the row they are one
 // long chain, and few rows leave the chip idle meanwhile.  So with blocks of 4 and 8 the
@@ -651,9 +651,12 @@ bool chain_bound(const fkpm_handle* h) {
 // Smaller blocks have few passes of many rows (60x60 x 1 FP32, S = 150 256 / 271).
 constexpr int kXiPassWgs = 128;
 
-dim3 xi_grid(const fkpm_handle* h, const KCfg& c) {
-  const bool apart = h->b >= 4 && c.nwg <= kXiPassWgs;
-  return dim3(c.nwg, apart ? h->qp / (c.L * c.KQ) : 1);
+int xi_apart(const fkpm_handle* h, const KCfg& c) {
+  return h->b >= 4 && c.nwg <= kXiPassWgs ? h->qp / (c.L * c.KQ) : 1;
+}
+template <class S>
+auto xi_fn(const fkpm_handle* h, const fkd::KSet<S>& ks, const KCfg& c) {
+  return xi_apart(h, c) > 1 ? ks.xi_apart : ks.xi;
 }
 
 // Kernel entry of a kind under its configuration.
@@ -1154,7 +1157,7 @@ int tune_t(fkpm_handle* h) {
                             cl ? rsource<S>(h, 0.25) : no_rsource<S>());
             }
             if (kind == K_XI)
-              return launch(ks.xi, xi_grid(h, k), dim3(fkd::WG), h->stream, rp_for(h, k), ci, hv, (const S*)x,
+              return launch(xi_fn(h, ks, k), dim3(k.nwg, xi_apart(h, k)), dim3(fkd::WG), h->stream, rp_for(h, k), ci, hv, (const S*)x,
                             (const S*)z, y, h->xi.as<double>(), h->nb, h->qp, k.chunk, 2.0, -1.0,
                             0.0, 0.5, t == 0 ? 1 : 0, nt_for(h, k));
             // backward step: reads alpha_m, alpha_{m+1}, beta_{m+1}, beta_{m+2};
@@ -2000,16 +2003,16 @@ int stoch_t(fkpm_handle* h, int M, const double* c) {
     CHK(h->xi.ensure(h->accbytes()));
     const KCfg& kx = h->kc[K_XI];
     const auto& ksx = h->ks<S>(K_XI);
-    const dim3 grid = xi_grid(h, kx);
+    const dim3 grid(kx.nwg, xi_apart(h, kx));
     {
       LoopRecorder rec(h);
       // alpha_1 = Hs R, xi = c0 R + c1 alpha_1
-      CHK(launch(ksx.xi, grid, block, h->stream, rp_for(h, kx), ci, hv, (const S*)h->vec_a(0),
+      CHK(launch(xi_fn(h, ksx, kx), grid, block, h->stream, rp_for(h, kx), ci, hv, (const S*)h->vec_a(0),
                  (const S*)nullptr, (S*)h->vec_a(1), h->xi.as<double>(), h->nb, h->qp, kx.chunk,
                  1.0, 0.0, c[0], c[1], 1, nt_for(h, kx)));
       for (int m = 2; m < M; m++) {
         // alpha_m = 2 Hs alpha_{m-1} - alpha_{m-2}; xi += c_m alpha_m
-        CHK(launch(ksx.xi, grid, block, h->stream, rp_for(h, kx), ci, hv,
+        CHK(launch(xi_fn(h, ksx, kx), grid, block, h->stream, rp_for(h, kx), ci, hv,
                    (const S*)h->vec_a(m - 1),
                    (const S*)h->vec_a(m - 2), (S*)h->vec_a(m), h->xi.as<double>(), h->nb, h->qp,
                    kx.chunk, 2.0, -1.0, 0.0, c[m], 0, nt_for(h, kx)));

@@ -24,6 +24,9 @@ struct KSet {
                    double, double, double*, int, RSource<S>) = nullptr;
   void (*xi)(const int*, const int*, const S*, const S*, const S*, S*, double*, int, int, int,
              double, double, double, double, int, int) = nullptr;
+  // xi with its column passes side by side (blocks of 4 and 8)
+  void (*xi_apart)(const int*, const int*, const S*, const S*, const S*, S*, double*, int, int, int,
+                   double, double, double, double, int, int) = nullptr;
   void (*ad_fused)(const int*, const int*, const S*, const S*, const S*, const S*, const S*, S*,
                    S*, double*, int, int, int, double, double, double, double, double,
                    double, int) = nullptr;

@@ -731,9 +731,10 @@ __global__ __launch_bounds__(WG) void k_step_moments(
 // ---------------------------------------------------------------------------
 // Stochastic-matrix step: y = cx * (Hs x) + cz * z, and xi (FP64) updated as
 // xi = c0 * x_i + c1 * y  (first step, x = R) or xi += c1 * y.  This is the
-// loop body of Engine_CPU::stoch_matrix (engine_cpu.cpp:229-244).
+// loop body of Engine_CPU::stoch_matrix (engine_cpu.cpp:229-244).  APART: one
+// column pass a workgroup, the pass by the grid's second dimension.
 // ---------------------------------------------------------------------------
-template <typename S, bool CX, int B, int L, int KQ>
+template <typename S, bool CX, int B, int L, int KQ, bool APART>
 __global__ __launch_bounds__(WG) void k_step_xi(
     const int* __restrict__ rp, const int* __restrict__ ci, const S* __restrict__ hv,
     const S* __restrict__ x, const S* __restrict__ z, S* __restrict__ y,
@@ -750,9 +751,8 @@ __global__ __launch_bounds__(WG) void k_step_xi(
   const A acx = (A)cx, acz = (A)cz;
   const S* const X[1] = {x};
 
-  // columns per sweep over the rows; a second grid dimension takes the passes apart
-  const int qw = (nt & NT_SLICE) || gridDim.y > 1 ? L * KQ : qp;
-  for (int qs = blockIdx.y * qw; qs < qp; qs += gridDim.y * qw) {
+  const int qw = APART || (nt & NT_SLICE) ? L * KQ : qp;  // columns per sweep over the rows
+  for (int qs = APART ? blockIdx.y * qw : 0; qs < qp; qs += APART ? qp : qw) {
   RowPtr nxt = row_ptr(rp, first_row<L>(rr.r0 + g), rr.r1, nt);
   for (int base = rr.r0; base < rr.r1; base += rr.stride) {
     int i = base + g;
