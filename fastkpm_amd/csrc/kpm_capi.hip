@@ -641,14 +641,15 @@ bool chain_bound(const fkpm_handle* h) {
          h->vbytes() < (size_t)h->max_deg * h->b * ((h->single ? 320 : 192) << 10);
 }
 
-// Column passes side by side in the forward method's step.  Rows of complex 8x8 blocks are padded to tiles of
-// the matrix cores, which leaves this vector-unit step passes as narrow as one tile
-// (144 columns FP64: nine); one after another in the workgroup of the row they are one
-// long chain, and few rows leave the chip idle meanwhile.  So with blocks of 4 and 8 the
-// passes of a sweep of up to 128 workgroups run side by side.  stoch_matrix of M = 32
-// (us), in turn / side by side: 12x12 x 8 FP64, S = 129 3674 / 911, 10^3 5679 / 3052, 45x45
-// (127 workgroups) 4824 / 3875; 15^3 (211) S = 65 4594 / 4989, FP32 S = 129 4201 / 4484.
-// Smaller blocks have few passes of many rows (60x60 x 1 FP32, S = 150 256 / 271).
+// Column passes side by side in the forward method's step.  Rows of complex 8x8 blocks
+// are padded to tiles of the matrix cores, which leaves this vector-unit step passes as
+// narrow as one tile (144 columns FP64: nine); one after another in the workgroup of the
+// row they are one long chain, and few rows leave the chip idle meanwhile.  So with
+// blocks of 4 and 8 the passes of a sweep of up to 128 workgroups run side by side.
+// stoch_matrix of M = 32 (us), in turn / side by side: 12x12 x 8 FP64, S = 129 3674 / 911,
+// 10^3 5679 / 3052, 45x45 (127 workgroups) 4824 / 3875; 15^3 (211) S = 65 4594 / 4989, FP32
+// S = 129 4201 / 4484.  Smaller blocks have few passes of many rows (60x60 x 1 FP32, S = 150
+// 256 / 271).
 constexpr int kXiPassWgs = 128;
 
 int xi_apart(const fkpm_handle* h, const KCfg& c) {
@@ -1157,9 +1158,10 @@ int tune_t(fkpm_handle* h) {
                             cl ? rsource<S>(h, 0.25) : no_rsource<S>());
             }
             if (kind == K_XI)
-              return launch(xi_fn(h, ks, k), dim3(k.nwg, xi_apart(h, k)), dim3(fkd::WG), h->stream, rp_for(h, k), ci, hv, (const S*)x,
-                            (const S*)z, y, h->xi.as<double>(), h->nb, h->qp, k.chunk, 2.0, -1.0,
-                            0.0, 0.5, t == 0 ? 1 : 0, nt_for(h, k));
+              return launch(xi_fn(h, ks, k), dim3(k.nwg, xi_apart(h, k)), dim3(fkd::WG),
+                            h->stream, rp_for(h, k), ci, hv, (const S*)x, (const S*)z, y,
+                            h->xi.as<double>(), h->nb, h->qp, k.chunk, 2.0, -1.0, 0.0, 0.5,
+                            t == 0 ? 1 : 0, nt_for(h, k));
             // backward step: reads alpha_m, alpha_{m+1}, beta_{m+1}, beta_{m+2};
             // writes alpha_{m-1}, beta_m into the third buffers
             return launch(adf_fn(h, ks, k), dim3(k.nwg), dim3(fkd::WG), h->stream, rp_for(h, k), ci, hv,
@@ -2007,9 +2009,10 @@ int stoch_t(fkpm_handle* h, int M, const double* c) {
     {
       LoopRecorder rec(h);
       // alpha_1 = Hs R, xi = c0 R + c1 alpha_1
-      CHK(launch(xi_fn(h, ksx, kx), grid, block, h->stream, rp_for(h, kx), ci, hv, (const S*)h->vec_a(0),
-                 (const S*)nullptr, (S*)h->vec_a(1), h->xi.as<double>(), h->nb, h->qp, kx.chunk,
-                 1.0, 0.0, c[0], c[1], 1, nt_for(h, kx)));
+      CHK(launch(xi_fn(h, ksx, kx), grid, block, h->stream, rp_for(h, kx), ci, hv,
+                 (const S*)h->vec_a(0), (const S*)nullptr, (S*)h->vec_a(1),
+                 h->xi.as<double>(), h->nb, h->qp, kx.chunk, 1.0, 0.0, c[0], c[1], 1,
+                 nt_for(h, kx)));
       for (int m = 2; m < M; m++) {
         // alpha_m = 2 Hs alpha_{m-1} - alpha_{m-2}; xi += c_m alpha_m
         CHK(launch(xi_fn(h, ksx, kx), grid, block, h->stream, rp_for(h, kx), ci, hv,

@@ -96,13 +96,13 @@ struct KSet {
 
 // The forward step of a geometry on nb block rows; long_row: one long row sets its time.
 // Such a row takes two real 4x4 FP64 blocks a batch instead of one (moments of M = 40, us,
-// one / two, rows of 5 blocks and one of 65, S = 24: 2000 rows 630 / 534, 9000 716 / 592, 30000 889 /
-// 656; one of 25 287 / 265, 350 / 310; complex and smaller blocks lost up to 17 % by it at
-// 25).  With 8-row blocks on a wave a row, the early load
-// of the own rows costs one of four waves a SIMD: it pays while every row's wave is
-// resident either way, two on each of 1024 SIMDs.  Moments of M = 64 with
-// and without, real FP64 x 8 x 128 (us): 32x32 369 / 431, 10^3 584 / 629, 45x45 627 / 627;
-// 46x46 717 / 698, 16^3 1419 / 1099, 20^3 2303 / 2057.
+// one / two, rows of 5 blocks and one of 65, S = 24: 2000 rows 630 / 534, 9000 716 / 592,
+// 30000 889 / 656; one of 25: 287 / 265, 350 / 310; complex and smaller blocks lost up to
+// 17 % by it at 25).  With 8-row blocks on a wave a row, the early load of the own rows
+// costs one of four waves a SIMD: it pays while every row's wave is resident either way,
+// two on each of 1024 SIMDs.  Moments of M = 64 with and without, real FP64 x 8 x 128
+// (us): 32x32 369 / 431, 10^3 584 / 629, 45x45 627 / 627; 46x46 717 / 698, 16^3 1419 / 1099,
+// 20^3 2303 / 2057.
 constexpr int kEarlyRows = 2048;
 template <class S>
 auto step_fn(const KSet<S>& ks, int nb, bool long_row) {
